@@ -270,7 +270,10 @@ __device__ __forceinline__ void hold(T& v) {
 }
 
 // The chunks into the wave's LDS region in order: tile (t, j) then starts at word (2 t + j) * 4 K2. Only the wave
-// itself reads its region, and a wave's LDS accesses complete in order, so no barrier follows.
+// itself reads its region, and a wave's LDS accesses complete in order, so no barrier instruction follows. The compiler
+// must not see through that: a lane that stores no chunk (narrow widths) reads words other lanes stored, and without a
+// memory clobber its reads of the previous chunk were taken as still current (no store of its own in between), which
+// gave wrong sums at widths 2 and 3 in the small items' down product.
 template <int NKT>
 __device__ __forceinline__ void stage_store(uint32_t* st, int k2, int lane, const u4v (&v)[stage_loads<NKT>()]) {
     const int chunks = (k2 >= 2 && k2 <= STAGE_MAXK2) ? NKT * 2 * k2 : 0;
@@ -279,6 +282,7 @@ __device__ __forceinline__ void stage_store(uint32_t* st, int k2, int lane, cons
         const int c = 64 * i + lane;
         if (c < chunks) *reinterpret_cast<u4v*>(st + 4 * c) = v[i];
     }
+    issued();
 }
 
 // The same for a width known at compile time: the loads a wave issues are exactly ceil(NKT * K2 / 32), and the
@@ -305,6 +309,7 @@ __device__ __forceinline__ void stage_store_k(uint32_t* st, int lane, const u4v 
         const int c = 64 * i + lane;
         if ((NKT * 2 * K2) % 64 == 0 || c < NKT * 2 * K2) *reinterpret_cast<u4v*>(st + 4 * c) = v[i];
     }
+    issued();
 }
 template <int K2>
 __device__ __forceinline__ LaneQuad lane_quad_k(int lane) {

@@ -218,6 +218,22 @@ def test_prompt_experts_every_staged_width(ea, k2):
 
 
 @pytest.mark.parametrize("planes", [True, False])
+@pytest.mark.parametrize("k2,R,E", [(2, 20, 64), (3, 20, 64), (5, 20, 64), (3, 100, 24)])
+def test_prompt_experts_narrow_widths_resident_down(ea, k2, R, E, planes):
+    """Widths whose staged chunk does not fill a wave's 16-byte loads, at a D the resident-activation down kernel takes
+    (16 column blocks): lanes that store nothing read the words of lanes that do. Items of at most 6 pairs, and (24
+    experts, 100 rows) both lists."""
+    device, _, _, pe, synth = ea
+    D = 2048
+    host, ex, sc, x, pick, wts, dx, dp, dw = _prompt_case(ea, R, E, D, 256, k2, 950 + k2, zipf=False, planes=planes)
+    want = orc.prompt_experts(x, pick, wts, oracle_routed(host), R, 8, bf16=True)
+    out = device.zeros((R, D), torch.float32)
+    pe.run(device.stream(), dx.data_ptr(), D, dp.data_ptr(), dw.data_ptr(), ex, sc, out.data_ptr(), R, do_round=False)
+    assert_close_rms(device.download(out), want, 2e-3, f"narrow widths, K2 {k2}, planes={planes}")
+    assert device.device_status() == 0
+
+
+@pytest.mark.parametrize("planes", [True, False])
 def test_prompt_experts_f32_activations(ea, planes):
     """fp32 activations (x_dtype 2: the rotation launch reads them and rounds the rotated rows to fp16 as for 16-bit
     ones), with the pair plane and without it, against the oracle on the same fp32 rows."""
