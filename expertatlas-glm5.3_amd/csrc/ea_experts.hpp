@@ -12,7 +12,7 @@ int launch_group(hipStream_t s, const int* pick, int* uids, int* ucount, int* me
                  uint32_t experts, uint32_t maxm);
 int launch_rot_in(hipStream_t s, const void* x, int x_dtype, uint32_t x_stride, const int* pick, const uint16_t* suh0,
                   const uint16_t* suh1, uint16_t* out0, uint16_t* out1, uint32_t rows, uint32_t kdim, uint32_t slots,
-                  uint32_t experts, void* zero = nullptr, int zero_half = 0);
+                  uint32_t experts);
 int launch_grouped(hipStream_t s, const ea_grouped_args& a);
 // The prefill path's scratch inside a moe scratch of more than 16 rows (ea_prompt.hip): its bytes, and its carve
 // from `base` (the pair plane included; zeroed by ea_moe_scratch_init, which is all a prompt scratch needs).
@@ -27,7 +27,7 @@ int launch_gateup_epilogue(hipStream_t s, const float* z, const int* pick, const
                            int only = -1);
 int launch_down_combine(hipStream_t s, const float* z, const int* pick, const uint16_t* svh_d, float* y,
                         const float* wts, float* out, uint32_t rows, uint32_t p, uint32_t d, uint32_t sk,
-                        uint32_t slots, uint32_t experts, bool skip_invalid = false);
+                        uint32_t slots, uint32_t experts);
 
 // The most rows the decode layer's launches take; a moe scratch above it holds the prefill path's region instead.
 constexpr uint32_t DL_REGION_ROWS = 16;

@@ -3,11 +3,11 @@
 // (prompt_experts.cu / prompt_experts.zig of the reference give the interface and the item scheme).
 //
 // A pass over <= 4096 rows: route -> per-pair input rotation -> item GEMM gate|up -> gate/up epilogue -> item GEMM
-// down -> [down epilogue + slot-ordered combine] [-> bf16 rounding]. Every row's arithmetic is independent of which
-// item or M-tile it lands in (MFMA rows do not mix). With a pair plane (the reference's deterministic mode 2) the
-// down GEMM writes each pair's row and the combine adds the slots in order, so the output is the same on every run.
-// Without one (modes 0 and 1, the reference's default) the down GEMM's epilogue adds each pair into its row of out
-// with fp32 (or packed fp16) atomics in arrival order; the rotation launch clears out first.
+// down -> down epilogue + slot-ordered combine (+ bf16 rounding). Every row's arithmetic is independent of which
+// item or M-tile it lands in (MFMA rows do not mix), and the combine adds a row's slots in order, so the output is the
+// same on every run. The down products go to a pair plane, or, in a scratch without one (planes 0, the reference's
+// default), over the pairs' own rotated inputs: see PairPlane. (The reference adds each slot into out with atomics there;
+// that form was bound by the atomics' rate, 320 G/s: 737 against 632 us at 2048 rows and 8 slots of 6144.)
 #include <hip/hip_runtime.h>
 
 #include "ea_device.hpp"
@@ -157,99 +157,27 @@ __global__ void __launch_bounds__(ROUTE_THREADS) route_kernel(const int* __restr
     for (int i = ROUTE_HELD * ROUTE_THREADS + threadIdx.x; i < n; i += ROUTE_THREADS) place(i, pick[i]);
 }
 
-// ---- the down epilogue without a pair plane ---------------------------------------------------------------------
+// ---- the pair plane -----------------------------------------------------------------------------------------------
 
-constexpr int ES = 128 + 4;  // LDS row stride of a row tile's epilogue buffer, floats (rows 4 apart on other banks)
-
-// Where the atomic down epilogue adds: out [rows, D] fp32 (fp16 with half), the expert's svh_d row, the item's pairs
-// and routing weights (LDS), and a double buffer of one row tile x 128 columns in LDS.
-struct DnAtomic {
-    void* out;
-    const uint16_t* svh;  // svh_d + e * D
-    const int* pair_sh;   // the item's pairs, -1 past its count
-    const float* wts_sh;  // their routing weights
-    float* ebuf;          // [2][16][ES]
-    int D, slots, half;
+// Where the down products go: fp32 [pairs, D] rows of one plane, or (a scratch without a plane) each pair's row split in
+// two halves of D / 2 columns over the pair's own rotated inputs, which the pair's gate|up product has read by then: the
+// lower columns in its xg row, the upper in its xu row (D fp16 = D / 2 fp32 each). The item lists run side by side, but a
+// pair's rows belong to one list, whose gate|up precedes its down product on one stream. Column col of pair p is at
+// base(col)[p * stride + col].
+struct PairPlane {
+    float *lo, *hi;  // hi already moved back by half columns
+    int half, stride;
+    __host__ __device__ float* base(int col) const { return col < half ? lo : hi; }
 };
-
-// The down items' epilogue without a pair plane (prompt_experts.cu:719-797, modes 0 and 1): for each occupied row
-// tile, the block's four waves hand their 16 rows x 32 columns (two column tiles each, MFMA accumulator layout) to LDS,
-// then thread (row r, lane l16) takes the row's columns g + 16 j (g = h8_group(l16)) of the 128-column block cb: the
-// FWHT over the block (fwht128_x8: column bits 4, 5, 6 inside the thread, bits 0..3 across the row's 16 lanes), the
-// output scale svh_d * HAD_SCALE (sv, loaded by the caller) and the pair's routing weight, then an atomic add into
-// its row of out: fp32, 16 lanes a row covering 64 contiguous bytes an instruction; or, with half, packed fp16 pairs
-// once the lanes of a column pair have traded values. The slots of a row meet in out in arrival order, so the sums' bits may differ run to run.
-// The buffer halves alternate (eb), so one barrier a row tile suffices: a half is written again only after the
-// barrier that follows every thread's reads of it.
-template <int MT>
-__device__ __forceinline__ void dn_atomic(const f4v (&acc)[MT][2], int mts, int wave, int lane, int cb,
-                                          const uint32_t (&sv)[4], const DnAtomic& a, int& eb) {
-    const int r = (int)threadIdx.x >> 4, l16 = lane & 15, g = h8_group(lane);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        if (mt >= mts) break;  // uniform
-        float* E = a.ebuf + eb * 16 * ES;
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) E[(4 * (lane >> 4) + i) * ES + 32 * wave + 16 * j + l16] = acc[mt][j][i];
-        __syncthreads();
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = E[r * ES + 16 * j + g];
-        eb ^= 1;
-        const float sg = fwht128_x8(v, lane);  // the values' sign, folded into the scale (exact)
-        const int idx = mt * 16 + r, p = a.pair_sh[idx];
-        const float w = p >= 0 ? a.wts_sh[idx] : 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = v[j] * (sg * (h2f((uint16_t)(sv[j >> 1] >> (16 * (j & 1)))) * HAD_SCALE)) * w;
-        const size_t ro = (size_t)(p >= 0 ? p / a.slots : 0) * a.D + (size_t)cb * 128;
-        if (!a.half) {
-            if (p >= 0) {
-                float* o = static_cast<float*>(a.out) + ro + g;
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    __builtin_amdgcn_global_atomic_fadd_f32((__attribute__((address_space(1))) float*)(o + 16 * j),
-                                                            v[j]);
-            }
-        } else {
-            // lane pair (l16, l16 ^ 1) holds columns (16 j + even, 16 j + odd) (its groups differ in bit 0 only): the
-            // even column's lane adds j = 0..3, the odd one's j = 4..7, each as one packed pair at the even column
-            // (static indices only: both lanes' pairs are formed and one is chosen)
-            const bool odd = g & 1;
-            uint16_t* base = static_cast<uint16_t*>(a.out) + ro + (g & ~1);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float oe = lane_xor<1>(v[q]), oo = lane_xor<1>(v[q + 4]);  // the partner's values
-                const float lo = odd ? oo : v[q], hi = odd ? v[q + 4] : oe;
-                const h2v hv = __builtin_bit_cast(h2v, (uint32_t)f2h(lo) | ((uint32_t)f2h(hi) << 16));
-                if (p >= 0)
-                    __builtin_amdgcn_global_atomic_fadd_v2f16(
-                        (__attribute__((address_space(1))) h2v*)(base + 16 * (odd ? q + 4 : q)), hv);
-            }
-        }
-    }
-}
-
-// svh_d of thread (r, l16)'s eight columns g + 16 j (g = h8_group(l16)) of column block cb, two fp16 a word (j even
-// low).
-__device__ __forceinline__ void dn_atomic_scales(const uint16_t* svh, int cb, int lane, uint32_t (&sv)[4]) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-        sv[q] = (uint32_t)svh[cb * 128 + 32 * q + h8_group(lane)] |
-                ((uint32_t)svh[cb * 128 + 32 * q + 16 + h8_group(lane)] << 16);
-}
 
 // Block (item, n block of NW * NTW tiles, matrix): wave w covers NTW n tiles over the whole K range for all of the
 // item's rows (IPM_WIDE_TILES groups of 16), so each trellis tile is decoded once per item. Z[mat][pair][n] fp32.
-template <int CB, int LO, int HI, int NTW, int NW, bool ATOM>
+template <int CB, int LO, int HI, int NTW, int NW>
 __global__ void __launch_bounds__(NW * 64) item_gemm_kernel(
     const uint16_t* __restrict__ X0, const uint16_t* __restrict__ X1, const int64_t* __restrict__ TP0,
     const int64_t* __restrict__ TP1, const int* __restrict__ K2_0, const int* __restrict__ K2_1,
     const int* __restrict__ sorted, const int* __restrict__ items, const int* __restrict__ item_count,
-    float* __restrict__ Z, int K, int N, int P, int big, int max_items, int* __restrict__ status,
-    const float* __restrict__ wts, const uint16_t* __restrict__ svh_d, void* __restrict__ out, int slots, int half) {
-    static_assert(!ATOM || NTW * NW == 8, "the atomic epilogue takes 128-column blocks of four waves");
+    PairPlane plane, size_t mat_stride, int K, int N, int P, int big, int max_items, int* __restrict__ status) {
     int e, first, cnt;
     if (!item_at(items, item_count, big, max_items, blockIdx.x, e, first, cnt)) return;
     const int mat = blockIdx.z;
@@ -258,16 +186,10 @@ __global__ void __launch_bounds__(NW * 64) item_gemm_kernel(
     const int k2 = mat ? K2_1[e] : K2_0[e];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     __shared__ int pair_sh[IPM_WIDE];
-    constexpr int EWORDS = ATOM ? 2 * 16 * ES : 1;
-    constexpr int WWORDS = ATOM ? IPM_WIDE : 1;
-    __shared__ float ebuf[EWORDS];
-    __shared__ float wts_sh[WWORDS];
     if (threadIdx.x < IPM_WIDE) pair_sh[threadIdx.x] = (int)threadIdx.x < cnt ? sorted[first + threadIdx.x] : -1;
-    if constexpr (ATOM)
-        if (threadIdx.x < IPM_WIDE) wts_sh[threadIdx.x] = (int)threadIdx.x < cnt ? wts[sorted[first + threadIdx.x]] : 0.f;
     __syncthreads();
     const int nt0 = (blockIdx.y * NW + wave) * NTW;
-    if (!ATOM && nt0 * 16 >= N) return;  // ATOM: N % 128 == 0 (host-checked), every wave in range
+    if (nt0 * 16 >= N) return;
     const uint16_t* xrow[IPM_WIDE_TILES];
 #pragma unroll
     for (int m = 0; m < IPM_WIDE_TILES; ++m) {
@@ -291,15 +213,7 @@ __global__ void __launch_bounds__(NW * 64) item_gemm_kernel(
 #pragma unroll
             for (int j = 0; j < NTW; ++j) acc[m][j] = nan4();
     }
-    if constexpr (ATOM) {
-        uint32_t sv[4];
-        dn_atomic_scales(svh_d + (size_t)e * N, (int)blockIdx.y, lane, sv);
-        int eb = 0;
-        const DnAtomic at{out, svh_d + (size_t)e * N, pair_sh, wts_sh, ebuf, N, slots, half};
-        dn_atomic<IPM_WIDE_TILES>(acc, (cnt + 15) >> 4, wave, lane, (int)blockIdx.y, sv, at, eb);
-        return;
-    }
-    float* Zm = Z + (size_t)mat * P * N;
+    float* Zm = plane.base(nt0 * 16) + (size_t)mat * mat_stride;  // a wave's columns lie in one half (half % 128 == 0)
 #pragma unroll
     for (int m = 0; m < IPM_WIDE_TILES; ++m)
 #pragma unroll
@@ -308,7 +222,7 @@ __global__ void __launch_bounds__(NW * 64) item_gemm_kernel(
             const int p = pair_sh[row];
             if (p < 0) continue;
 #pragma unroll
-            for (int j = 0; j < NTW; ++j) Zm[(size_t)p * N + (nt0 + j) * 16 + (lane & 15)] = acc[m][j][i];
+            for (int j = 0; j < NTW; ++j) Zm[(size_t)p * plane.stride + (nt0 + j) * 16 + (lane & 15)] = acc[m][j][i];
         }
 }
 
@@ -710,18 +624,15 @@ item_ring_kernel(const uint16_t* __restrict__ X0, const uint16_t* __restrict__ X
 
 // The column blocks of a down block for one width: step s is column block s / nch, chunk s % nch; the trellis two
 // steps ahead; each column block's rows are stored when its last chunk is done.
-template <int CB, int K2, int MT, int NG, bool ATOM>
+template <int CB, int K2, int MT, int NG>
 __device__ __forceinline__ void dn_loop(const TileSpan& sp, const uint16_t* xa, uint32_t* st, int lane, int wave,
-                                        int mts, int nch, int nb0, const int* pair_sh, float* __restrict__ Z, int N,
-                                        const DnAtomic& at) {
+                                        int mts, int nch, int nb0, const int* pair_sh, const PairPlane& plane) {
     constexpr int NL = stage_loads_k<PK, K2>();
     constexpr int TWB = 16 * K2;
     const LaneQuad lq = lane_quad_k<K2>(lane);
     const int steps = NG * nch;  // even (NG even, or nch = 2: the caller's choice): two steps an iteration
     u4v ta[NL], tb[NL];
     f4v acc[MT][2];
-    uint32_t sv[4];  // ATOM: svh_d of this thread's epilogue columns, loaded at a column block's first chunk
-    int eb = 0;
     auto issue_t = [&](int s2, u4v (&tv)[NL]) __attribute__((always_inline)) {
         s2 = s2 < steps ? s2 : steps - 1;
         TileSpan sc = sp;
@@ -733,15 +644,13 @@ __device__ __forceinline__ void dn_loop(const TileSpan& sp, const uint16_t* xa, 
         if (c == 0) {
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = f4v{0.f, 0.f, 0.f, 0.f};
-            if constexpr (ATOM) dn_atomic_scales(at.svh, nb0 + s2 / nch, lane, sv);
         }
         stage_store_k<PK, K2>(st, lane, tv);  // only this wave reads its region, in order
         issue_t(s2 + 2, tv);
         item_chunk<CB, K2, MT>(st, lq, xa + c * PK * 16, mts, lane, acc, DXS);
-        if (c == nch - 1 && ATOM) {
-            if constexpr (ATOM) dn_atomic<MT>(acc, mts, wave, lane, nb0 + s2 / nch, sv, at, eb);
-        } else if (c == nch - 1) {
+        if (c == nch - 1) {
             const int nt0 = (nb0 + s2 / nch) * 8 + 2 * wave;
+            float* Z = plane.base(nt0 * 16);
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -749,7 +658,8 @@ __device__ __forceinline__ void dn_loop(const TileSpan& sp, const uint16_t* xa, 
                     const int p = pair_sh[mt * 16 + 4 * (lane >> 4) + i];
                     if (p < 0) continue;
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) Z[(size_t)p * N + (nt0 + j) * 16 + (lane & 15)] = acc[mt][j][i];
+                    for (int j = 0; j < 2; ++j)
+                        Z[(size_t)p * plane.stride + (nt0 + j) * 16 + (lane & 15)] = acc[mt][j][i];
                 }
         }
     };
@@ -763,15 +673,13 @@ __device__ __forceinline__ void dn_loop(const TileSpan& sp, const uint16_t* xa, 
 
 // The down matrix (K = I of 128 or 256: one or two chunks): a block (item of list MT > 2, NG column blocks of 128)
 // loads the item's activations for all of K into LDS once, then its waves run the column blocks independently. WB = 8
-// (the larger items with a pair plane): two groups of four waves, each over NG / 2 of the column blocks, share one copy
+// (the larger items): two groups of four waves, each over NG / 2 of the column blocks, share one copy
 // of the activations, so two blocks fit a CU's LDS at four waves a SIMD (four-wave blocks: three at three).
-template <int CB, int MT, int NG, bool ATOM, int WB = PW>
+template <int CB, int MT, int NG, int WB = PW>
 __global__ void __launch_bounds__(WB * 64) __attribute__((amdgpu_waves_per_eu(MT > 2 && WB == PW ? 2 : 4)))
 item_dn_kernel(const uint16_t* __restrict__ X, const int64_t* __restrict__ TP, const int* __restrict__ K2T,
                const int* __restrict__ sorted, const int* __restrict__ items, const int* __restrict__ item_count,
-               float* __restrict__ Z, int K, int N, int P, int max_items, int* __restrict__ status,
-               const float* __restrict__ wts, const uint16_t* __restrict__ svh_d, void* __restrict__ out, int slots,
-               int half) {
+               PairPlane plane, int K, int N, int P, int max_items, int* __restrict__ status) {
     int e, first, cnt;
     // the larger items' blocks in XCD order (a column group's slice of an expert on the same XCDs for all of the
     // expert's items); the small items' (one item an expert) item by item
@@ -787,20 +695,12 @@ item_dn_kernel(const uint16_t* __restrict__ X, const int64_t* __restrict__ TP, c
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ int pair_sh[MT * 16];
     __shared__ __attribute__((aligned(16))) uint16_t xa[MT * 16 * DXS];
-    static_assert(WB == PW || (WB == 2 * PW && !ATOM && NG % 2 == 0), "two wave groups: pair-plane blocks");
+    static_assert(WB == PW || (WB == 2 * PW && NG % 2 == 0), "two wave groups: half the column blocks each");
     __shared__ __attribute__((aligned(16))) uint32_t st[WB][PSTAGE];
-    constexpr int EWORDS = ATOM ? 2 * 16 * ES : 1;
-    constexpr int WWORDS = ATOM ? MT * 16 : 1;
-    __shared__ float ebuf[EWORDS];
-    __shared__ float wts_sh[WWORDS];
     if (tid < MT * 16) pair_sh[tid] = tid < cnt ? sorted[first + tid] : -1;
-    if constexpr (ATOM)
-        if (tid < MT * 16) wts_sh[tid] = tid < cnt ? wts[sorted[first + tid]] : 0.f;
     __syncthreads();
     const int mts = (cnt + 15) >> 4;
     const int nch = K / (PK * 16);  // 1 or 2
-    DnAtomic at{};
-    if constexpr (ATOM) at = DnAtomic{out, svh_d + (size_t)e * N, pair_sh, wts_sh, ebuf, N, slots, half};
     {
         // 256 threads cover a chunk of a row tile; with eight waves each half of the block loads one chunk
         constexpr int CPT = WB == PW ? 2 : 1;  // chunks a thread loads
@@ -835,40 +735,43 @@ item_dn_kernel(const uint16_t* __restrict__ X, const int64_t* __restrict__ TP, c
     sp.kstride = ns * TWB;
     __syncthreads();  // the activations are in LDS
     const bool ok = EA_K2_SWITCH(
-        k2, 2, 10, (dn_loop<CB, K2V, MT, NGW, ATOM>(sp, xa, st[wave], lane, w4, mts, nch, nb0, pair_sh, Z, N, at)));
+        k2, 2, 10, (dn_loop<CB, K2V, MT, NGW>(sp, xa, st[wave], lane, w4, mts, nch, nb0, pair_sh, plane)));
     if (!ok) {  // no product ran: the item's outputs of the block's column blocks are NaN
         if (lane == 0) record_error(status, DEV_UNSUPPORTED_WIDTH);
         for (int g = 0; g < NGW; ++g)
             for (int i = 0; i < MT * 16; ++i) {
                 const int p = pair_sh[i];
                 if (p < 0) continue;
-                const size_t o = (size_t)(nb0 + g) * 128 + w4 * 32 + (lane & 31);
-                if (!ATOM) Z[(size_t)p * N + o] = __builtin_nanf("");
-                else if (!half) static_cast<float*>(out)[(size_t)(p / slots) * N + o] = __builtin_nanf("");
-                else static_cast<uint16_t*>(out)[(size_t)(p / slots) * N + o] = 0x7E00;
+                const int o = (nb0 + g) * 128 + w4 * 32 + (lane & 31);
+                plane.base(o)[(size_t)p * plane.stride + o] = __builtin_nanf("");
             }
     }
 }
 
+// How a pass's sums leave the combine: fp32, fp32 rounded through bf16 (prompt_experts.zig:246), or fp16 (half sums).
+enum OutMode : int { OUT_F32 = 0, OUT_BF16R = 1, OUT_F16 = 2 };
+
 // The down epilogue and slot combine of a prompt pass. Block (row r, 2048 columns): a thread holds 8 consecutive
 // columns of one 128-block (16 lanes a block, lane l the columns 8 h8_group(l) .. + 7); for each slot in order
-// y = FWHT(plane[pair]) * HAD_SCALE * svh_d[e], then out = fma(w, y, out) from zero, a slot without an expert adding
-// w * 0. These are the operations and the order of down_combine_kernel with one split (the butterflies over
+// y = FWHT(plane[pair]) * HAD_SCALE * svh_d[e], then out = fma(w, y, out) from zero; a slot without an expert adds w * 0,
+// or nothing with skip. These are the operations and the order of down_combine_kernel with one split (the butterflies over
 // value-index bits 0..6, three inside a lane and four across lanes: fwht128_x8), so the same bits (a zero y's sign
-// does not reach out, which starts at +0); the rotated plane is not written back (nothing reads it after the combine).
+// does not reach out, which starts at +0). Bound by the plane's bytes: the rounding happens here and not in a launch of
+// its own, which read and wrote out again (2048 rows: 24 us).
 // (prompt_experts.cu's deterministic combine; exl3_experts.cu:186-214 for the epilogue.)
-__global__ void __launch_bounds__(256) prompt_combine_kernel(const float* __restrict__ Z, const int* __restrict__ pick,
+__global__ void __launch_bounds__(256) prompt_combine_kernel(PairPlane plane, const int* __restrict__ pick,
                                                              const uint16_t* __restrict__ svh_d,
-                                                             const float* __restrict__ wts, float* __restrict__ out,
-                                                             int D, int E, int slots) {
+                                                             const float* __restrict__ wts, void* __restrict__ out,
+                                                             int D, int E, int slots, int mode, int skip) {
     const int r = blockIdx.x, lane = threadIdx.x & 63;
     const int k = blockIdx.y * 2048 + 128 * ((int)threadIdx.x >> 4) + 8 * h8_group(lane);
     if (k >= D) return;  // whole 16-lane groups (D % 128 == 0)
+    const float* __restrict__ Z = plane.base(k);  // 8 columns never straddle the halves (half % 64 == 0)
     float a[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) a[j] = 0.f;
     // four slots at a time: their picks and weights, then all their plane and svh loads in flight before the first
-    // slot's rotation (a slot without an expert loads pair 0's row and expert 0's scales, and adds w * 0)
+    // slot's rotation (a slot without an expert loads pair 0's row and expert 0's scales)
     constexpr int QB = 4;
     for (int q0 = 0; q0 < slots; q0 += QB) {
         int ev[QB];
@@ -880,7 +783,7 @@ __global__ void __launch_bounds__(256) prompt_combine_kernel(const float* __rest
             const int p = r * slots + (q0 + j < slots ? q0 + j : q0), e = pick[p];
             wv[j] = wts[p];
             ev[j] = e >= 0 && e < E ? p : -1;
-            const size_t zo = (size_t)(ev[j] >= 0 ? p : r * slots) * D + k;
+            const size_t zo = (size_t)(ev[j] >= 0 ? p : r * slots) * plane.stride + k;
             z0[j] = *reinterpret_cast<const f4v*>(Z + zo);
             z1[j] = *reinterpret_cast<const f4v*>(Z + zo + 4);
             sv[j] = *reinterpret_cast<const u4v*>(svh_d + (size_t)(ev[j] >= 0 ? e : 0) * D + k);
@@ -901,6 +804,7 @@ __global__ void __launch_bounds__(256) prompt_combine_kernel(const float* __rest
 #pragma unroll
                 for (int i = 0; i < 8; ++i) o[i] = v[i] * sc * h2f((uint16_t)(sv[j][i >> 1] >> (16 * (i & 1))));
             } else {
+                if (skip) continue;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) o[i] = 0.f;
             }
@@ -908,14 +812,28 @@ __global__ void __launch_bounds__(256) prompt_combine_kernel(const float* __rest
             for (int i = 0; i < 8; ++i) a[i] = __builtin_fmaf(wv[j], o[i], a[i]);
         }
     }
-    *reinterpret_cast<f4v*>(out + (size_t)r * D + k) = f4v{a[0], a[1], a[2], a[3]};
-    *reinterpret_cast<f4v*>(out + (size_t)r * D + k + 4) = f4v{a[4], a[5], a[6], a[7]};
-}
-
-// out fp32 -> bf16 -> fp32 in place (prompt_experts.zig:246).
-__global__ void round_kernel(float* __restrict__ out, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        out[i] = bf16r(out[i]);
+    if (mode == OUT_BF16R)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] = bf16r(a[j]);
+    // 16-byte stores where out allows them (D % 128 == 0 keeps every row as aligned as the first), else 4-byte ones
+    const bool al = (reinterpret_cast<uintptr_t>(out) & 15) == 0;  // uniform
+    if (mode == OUT_F16) {
+        uint32_t* o = reinterpret_cast<uint32_t*>(static_cast<uint16_t*>(out) + (size_t)r * D + k);
+        const u4v h = {f2h2(a[0], a[1]), f2h2(a[2], a[3]), f2h2(a[4], a[5]), f2h2(a[6], a[7])};
+        if (al) *reinterpret_cast<u4v*>(o) = h;
+        else
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = h[j];
+        return;
+    }
+    float* o = static_cast<float*>(out) + (size_t)r * D + k;
+    if (al) {
+        *reinterpret_cast<f4v*>(o) = f4v{a[0], a[1], a[2], a[3]};
+        *reinterpret_cast<f4v*>(o + 4) = f4v{a[4], a[5], a[6], a[7]};
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = a[j];
+    }
 }
 
 static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -926,13 +844,13 @@ struct PromptLayout {
     bool has_plane;
 };
 
-// Whether a pass without a pair plane covers the layer's shape: the atomic epilogue of the staged down GEMM takes
-// K = I of at most 256 and whole pairs of 128-column blocks (D % 256 == 0). Other shapes keep the plane.
-static bool atomic_down_fits(const ea_routed* ex) { return ex->width <= 2 * PK * 16 && ex->dims % 256 == 0; }
+// Whether a pass without a pair plane covers the layer's shape: halves of whole 128-column blocks (D % 256 == 0) over the
+// pairs' rotated inputs, and the down kernel that takes K = I of at most 256. Other shapes keep the plane.
+static bool split_plane_fits(const ea_routed* ex) { return ex->width <= 2 * PK * 16 && ex->dims % 256 == 0; }
 
 static PromptLayout prompt_layout(const ea_routed* ex, uint32_t rows, uint32_t slots, int planes) {
     PromptLayout l{};
-    l.has_plane = planes || !atomic_down_fits(ex);
+    l.has_plane = planes || !split_plane_fits(ex);
     const uint32_t r = rows < CHUNK_ROWS ? rows : CHUNK_ROWS;
     const size_t n = (size_t)r * slots, D = ex->dims, I = ex->width;
     l.rows = r;
@@ -957,30 +875,16 @@ static PromptLayout prompt_layout(const ea_routed* ex, uint32_t rows, uint32_t s
     return l;
 }
 
-// The atomic epilogue's arguments for a down launch (out null: the pair plane Z instead).
-struct DownOut {
-    const float* wts = nullptr;
-    const uint16_t* svh_d = nullptr;
-    void* out = nullptr;
-    int slots = 0, half = 0;
-};
-
 template <int CB, int LO, int HI>
 static void item_gemm(hipStream_t s, const uint16_t* X0, const uint16_t* X1, const int64_t* TP0, const int64_t* TP1,
-                      const int* B0, const int* B1, const int* sorted, const int* items, const int* count, float* Z,
-                      int K, int N, int P, int mats, uint32_t max_items, int* status, const DownOut& d = DownOut{}) {
+                      const int* B0, const int* B1, const int* sorted, const int* items, const int* count,
+                      const PairPlane& z, size_t mat_stride, int K, int N, int P, int mats, uint32_t max_items,
+                      int* status) {
     constexpr int NTW = 2, NW = 4;
     dim3 grid(max_items, (N / 16 + NTW * NW - 1) / (NTW * NW), mats);
-    for (int big = 1; big >= 0; --big) {
-        if (d.out)
-            item_gemm_kernel<CB, LO, HI, NTW, NW, true><<<grid, NW * 64, 0, s>>>(
-                X0, X1, TP0, TP1, B0, B1, sorted, items, count, Z, K, N, P, big, (int)max_items, status, d.wts,
-                d.svh_d, d.out, d.slots, d.half);
-        else
-            item_gemm_kernel<CB, LO, HI, NTW, NW, false><<<grid, NW * 64, 0, s>>>(
-                X0, X1, TP0, TP1, B0, B1, sorted, items, count, Z, K, N, P, big, (int)max_items, status, nullptr,
-                nullptr, nullptr, 0, 0);
-    }
+    for (int big = 1; big >= 0; --big)
+        item_gemm_kernel<CB, LO, HI, NTW, NW><<<grid, NW * 64, 0, s>>>(X0, X1, TP0, TP1, B0, B1, sorted, items, count, z,
+                                                                      mat_stride, K, N, P, big, (int)max_items, status);
 }
 
 // What one item list's pass reads and writes: the rotated activations, the three matrices' trellis tables and
@@ -992,11 +896,11 @@ struct ListPass {
     const int* k2[3];
     const int *sorted, *items, *count, *pclass, *pick;
     const uint16_t *svh_g, *svh_u, *suh_d;
-    float *z, *zp, *plane;
+    float *z, *zp;
+    PairPlane plane;
     uint16_t* xd;
     int D, I, P, rows, slots, E, mi;
     int* status;
-    DownOut down;  // out set: no pair plane, the down items add into out (fp32, or fp16 with half)
 };
 
 // One item list from its gate|up product to its down product, in order on q: big = 1 takes the larger items (the
@@ -1022,51 +926,29 @@ static int list_pass(hipStream_t q, const ListPass& a, int big) {
                                (uint32_t)a.I, 1, (uint32_t)a.slots, (uint32_t)a.E, __builtin_inff(), 1, a.pclass, a.zp,
                                (uint32_t)ns, big);
     if (r) return r;
-    if (a.down.out) {  // no pair plane: the atomic epilogue (atomic_down_fits holds)
-        const DownOut& d = a.down;
-        const int nb = a.D / 128;
+    const int nb = a.D / 128;
+    if (a.I <= 2 * PK * 16 && nb % 2 == 0) {
+#define EA_DN(MT_, NG_, WB_, grid)                                                                                    \
+    item_dn_kernel<CB, MT_, NG_, WB_><<<grid, (WB_) * 64, 0, q>>>(a.xd, a.tp[2], a.k2[2], a.sorted, a.items, a.count,  \
+                                                                  a.plane, a.I, a.D, a.P, a.mi, a.status)
         if (big && a.rows > LONG_ROWS && nb % DNG_BIG_LONG == 0)
-            item_dn_kernel<CB, IPM_TILES, DNG_BIG_LONG, true><<<xcd_blocks(a.mi, 1, nb / DNG_BIG_LONG), PW * 64, 0, q>>>(
-                a.xd, a.tp[2], a.k2[2], a.sorted, a.items, a.count, nullptr, a.I, a.D, a.P, a.mi, a.status, d.wts,
-                d.svh_d, d.out, d.slots, d.half);
-        else if (big)
-            item_dn_kernel<CB, IPM_TILES, DNG_BIG, true><<<xcd_blocks(a.mi, 1, nb / DNG_BIG), PW * 64, 0, q>>>(
-                a.xd, a.tp[2], a.k2[2], a.sorted, a.items, a.count, nullptr, a.I, a.D, a.P, a.mi, a.status, d.wts,
-                d.svh_d, d.out, d.slots, d.half);
-        else if (nb % DNG == 0)
-            item_dn_kernel<CB, SMALL_ROWS / 16, DNG, true><<<dim3(a.mi, nb / DNG, 1), PW * 64, 0, q>>>(
-                a.xd, a.tp[2], a.k2[2], a.sorted, a.items, a.count, nullptr, a.I, a.D, a.P, a.mi, a.status, d.wts,
-                d.svh_d, d.out, d.slots, d.half);
-        else
-            item_dn_kernel<CB, SMALL_ROWS / 16, 2, true><<<dim3(a.mi, nb / 2, 1), PW * 64, 0, q>>>(
-                a.xd, a.tp[2], a.k2[2], a.sorted, a.items, a.count, nullptr, a.I, a.D, a.P, a.mi, a.status, d.wts,
-                d.svh_d, d.out, d.slots, d.half);
-    } else if (a.I <= 2 * PK * 16 && (a.D / 128) % DNG == 0) {
-        if (big && a.rows > LONG_ROWS && (a.D / 128) % DNG_BIG_LONG == 0)
-            item_dn_kernel<CB, IPM_TILES, DNG_BIG_LONG, false, 2 * PW>
-                <<<xcd_blocks(a.mi, 1, a.D / 128 / DNG_BIG_LONG), 2 * PW * 64, 0, q>>>(
-                a.xd, a.tp[2], a.k2[2], a.sorted, a.items, a.count, a.plane, a.I, a.D, a.P, a.mi, a.status, nullptr,
-                nullptr, nullptr, 0, 0);
+            EA_DN(IPM_TILES, DNG_BIG_LONG, 2 * PW, xcd_blocks(a.mi, 1, nb / DNG_BIG_LONG));
         else if (big && a.I == 2 * PK * 16)  // two chunks of K: a wave group's one column block is an even step count
-            item_dn_kernel<CB, IPM_TILES, DNG_BIG, false, 2 * PW>
-                <<<xcd_blocks(a.mi, 1, a.D / 128 / DNG_BIG), 2 * PW * 64, 0, q>>>(
-                a.xd, a.tp[2], a.k2[2], a.sorted, a.items, a.count, a.plane, a.I, a.D, a.P, a.mi, a.status, nullptr,
-                nullptr, nullptr, 0, 0);
+            EA_DN(IPM_TILES, DNG_BIG, 2 * PW, xcd_blocks(a.mi, 1, nb / DNG_BIG));
         else if (big)
-            item_dn_kernel<CB, IPM_TILES, DNG_BIG, false><<<xcd_blocks(a.mi, 1, a.D / 128 / DNG_BIG), PW * 64, 0, q>>>(
-                a.xd, a.tp[2], a.k2[2], a.sorted, a.items, a.count, a.plane, a.I, a.D, a.P, a.mi, a.status, nullptr,
-                nullptr, nullptr, 0, 0);
+            EA_DN(IPM_TILES, DNG_BIG, PW, xcd_blocks(a.mi, 1, nb / DNG_BIG));
+        else if (nb % DNG == 0)
+            EA_DN(SMALL_ROWS / 16, DNG, PW, dim3(a.mi, nb / DNG, 1));
         else
-            item_dn_kernel<CB, SMALL_ROWS / 16, DNG, false><<<dim3(a.mi, a.D / 128 / DNG, 1), PW * 64, 0, q>>>(
-                a.xd, a.tp[2], a.k2[2], a.sorted, a.items, a.count, a.plane, a.I, a.D, a.P, a.mi, a.status, nullptr,
-                nullptr, nullptr, 0, 0);
+            EA_DN(SMALL_ROWS / 16, 2, PW, dim3(a.mi, nb / 2, 1));
+#undef EA_DN
     } else if (big) {
         item_gu_kernel<CB><<<xcd_blocks(a.mi, a.D / (16 * 2 * PW), 1), PW * 64, 0, q>>>(
-            a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane, nullptr, a.I, a.D,
+            a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, nullptr, a.I, a.D,
             a.P, 1, 1, a.mi, a.status);
     } else {
         item_ring_kernel<CB, 4><<<dim3(a.mi, a.D / 128, 1), 4 * 64, 0, q>>>(
-            a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane, a.I, a.D, a.P, 1,
+            a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, a.I, a.D, a.P, 1,
             a.mi, a.status);
     }
     return launched();
@@ -1096,14 +978,14 @@ static int list_passes(hipStream_t s, uint32_t cb, const ListPass& a) {
 // Widths above 10 (three trellis words a lane): the register-streaming GEMM, both lists in turn on s.
 static void wide_gemm(hipStream_t s, uint32_t cb, const uint16_t* X0, const uint16_t* X1, const int64_t* TP0,
                       const int64_t* TP1, const int* B0, const int* B1, const int* sorted, const int* items,
-                      const int* count, float* Z, int K, int N, int P, int mats, uint32_t max_items, int* status,
-                      const DownOut& d = DownOut{}) {
+                      const int* count, const PairPlane& z, size_t ms, int K, int N, int P, int mats,
+                      uint32_t max_items, int* status) {
     if (cb == 1) {
-        item_gemm<1, 2, 16>(s, X0, X1, TP0, TP1, B0, B1, sorted, items, count, Z, K, N, P, mats, max_items, status, d);
+        item_gemm<1, 2, 16>(s, X0, X1, TP0, TP1, B0, B1, sorted, items, count, z, ms, K, N, P, mats, max_items, status);
     } else if (cb == 2) {
-        item_gemm<2, 2, 16>(s, X0, X1, TP0, TP1, B0, B1, sorted, items, count, Z, K, N, P, mats, max_items, status, d);
+        item_gemm<2, 2, 16>(s, X0, X1, TP0, TP1, B0, B1, sorted, items, count, z, ms, K, N, P, mats, max_items, status);
     } else {
-        item_gemm<0, 2, 16>(s, X0, X1, TP0, TP1, B0, B1, sorted, items, count, Z, K, N, P, mats, max_items, status, d);
+        item_gemm<0, 2, 16>(s, X0, X1, TP0, TP1, B0, B1, sorted, items, count, z, ms, K, N, P, mats, max_items, status);
     }
 }
 
@@ -1195,10 +1077,10 @@ int ea_prompt_experts_run(ea_stream_t stream, const void* x, int x_dtype, uint32
     if (!x || !pick || !wts || !ex || !sc || !out) return EA_BAD_ARGUMENT;
     if (x_dtype < 0 || x_dtype > 2 || sc->slots == 0) return EA_BAD_ARGUMENT;
     if (ex->width % 128 || ex->dims % 128) return EA_BAD_WIDTH;
-    // no pair plane: the down items add each slot into out with atomics (packed fp16 pairs with half_sums), which a
-    // scratch made for this layer's shape allows (atomic_down_fits) and which needs out 4-byte aligned
-    const bool atom = sc->plane == 0;
-    if (atom && (!atomic_down_fits(ex) || (reinterpret_cast<uintptr_t>(out) & 3))) return EA_BAD_ARGUMENT;
+    // no pair plane: the pairs' down outputs take the place of their rotated inputs, which a scratch made for this
+    // layer's shape allows (split_plane_fits); out 4-byte aligned (half sums are stored in pairs)
+    const bool split = sc->plane == 0;
+    if (split && (!split_plane_fits(ex) || (reinterpret_cast<uintptr_t>(out) & 3))) return EA_BAD_ARGUMENT;
     hipStream_t s = as_stream(stream);
     const uint32_t D = ex->dims, I = ex->width, E = ex->count, S = sc->slots;
     const size_t xb = x_dtype == 2 ? 4 : 2;
@@ -1218,20 +1100,12 @@ int ea_prompt_experts_run(ea_stream_t stream, const void* x, int x_dtype, uint32
                                                                   dptr<int>(sc->pclass), (int)max_items, ipm);
         int r = launched();
         if (r) return r;
-        // without a plane the pass's rows of out are cleared by the rotation launch, before any down item adds
-        char* opass = static_cast<char*>(out) + (size_t)r0 * D * ob;
         r = launch_rot_in(s, xs, x_dtype, xstride, pk, dptr<const uint16_t>(ex->suh_g), dptr<const uint16_t>(ex->suh_u),
-                          dptr<uint16_t>(sc->xg), dptr<uint16_t>(sc->xu), n, D, S, E, atom ? opass : nullptr,
-                          half_sums);
+                          dptr<uint16_t>(sc->xg), dptr<uint16_t>(sc->xu), n, D, S, E);
         if (r) return r;
-        DownOut down;
-        if (atom) {
-            down.wts = wt;
-            down.svh_d = dptr<const uint16_t>(ex->svh_d);
-            down.out = opass;
-            down.slots = (int)S;
-            down.half = half_sums;
-        }
+        const int dh = (int)(D / 2);
+        const PairPlane plane = split ? PairPlane{dptr<float>(sc->xg), dptr<float>(sc->xu) - dh, dh, dh}
+                                      : PairPlane{dptr<float>(sc->plane), dptr<float>(sc->plane), dh, (int)D};
         if (!wide) {
             ListPass a{};
             a.xg = dptr<const uint16_t>(sc->xg);
@@ -1250,7 +1124,7 @@ int ea_prompt_experts_run(ea_stream_t stream, const void* x, int x_dtype, uint32
             a.suh_d = dptr<const uint16_t>(ex->suh_d);
             a.z = dptr<float>(sc->z);
             a.zp = dptr<float>(sc->zp);
-            a.plane = dptr<float>(sc->plane);
+            a.plane = plane;
             a.xd = dptr<uint16_t>(sc->xd);
             a.D = (int)D;
             a.I = (int)I;
@@ -1260,14 +1134,14 @@ int ea_prompt_experts_run(ea_stream_t stream, const void* x, int x_dtype, uint32
             a.E = (int)E;
             a.mi = (int)max_items;
             a.status = c->status;
-            a.down = down;
             r = list_passes(s, ex->cb, a);
         } else {
             wide_gemm(s, ex->cb, dptr<const uint16_t>(sc->xg), dptr<const uint16_t>(sc->xu),
                       dptr<const int64_t>(ex->ptr[0]), dptr<const int64_t>(ex->ptr[1]), dptr<const int>(ex->k2[0]),
                       dptr<const int>(ex->k2[1]), dptr<const int>(sc->sorted), dptr<const int>(sc->items),
-                      dptr<const int>(sc->count), dptr<float>(sc->z), (int)D, (int)I, (int)pairs, 2, max_items,
-                      c->status);
+                      dptr<const int>(sc->count),
+                      PairPlane{dptr<float>(sc->z), dptr<float>(sc->z), (int)I, (int)I}, (size_t)pairs * I, (int)D, (int)I,
+                      (int)pairs, 2, max_items, c->status);
             r = launched();
             if (r) return r;
             r = launch_gateup_epilogue(s, dptr<const float>(sc->z), pk, dptr<const uint16_t>(ex->svh_g),
@@ -1277,36 +1151,15 @@ int ea_prompt_experts_run(ea_stream_t stream, const void* x, int x_dtype, uint32
             wide_gemm(s, ex->cb, dptr<const uint16_t>(sc->xd), dptr<const uint16_t>(sc->xd),
                       dptr<const int64_t>(ex->ptr[2]), dptr<const int64_t>(ex->ptr[2]), dptr<const int>(ex->k2[2]),
                       dptr<const int>(ex->k2[2]), dptr<const int>(sc->sorted), dptr<const int>(sc->items),
-                      dptr<const int>(sc->count), dptr<float>(sc->plane), (int)I, (int)D, (int)pairs, 1, max_items,
-                      c->status, down);
+                      dptr<const int>(sc->count), plane, 0, (int)I, (int)D, (int)pairs, 1, max_items, c->status);
             r = launched();
         }
         if (r) return r;
-        if (atom) {  // every slot is in out already
-            if (do_round) {
-                round_kernel<<<1024, 256, 0, s>>>(reinterpret_cast<float*>(opass), (size_t)n * D);
-                r = launched();
-                if (r) return r;
-            }
-            continue;
-        }
-        // the pair plane summed in slot order (fp32 rows only: half sums were refused above); slots without an
-        // expert add nothing (the reference's route skips them)
-        float* o32 = reinterpret_cast<float*>(opass);
-        if ((reinterpret_cast<uintptr_t>(o32) & 15) == 0) {  // 16-byte stores
-            prompt_combine_kernel<<<dim3(n, (D + 2047) / 2048), 256, 0, s>>>(dptr<const float>(sc->plane), pk,
-                                                                             dptr<const uint16_t>(ex->svh_d), wt, o32,
-                                                                             (int)D, (int)E, (int)S);
-            r = launched();
-        } else {
-            r = launch_down_combine(s, dptr<const float>(sc->plane), pk, dptr<const uint16_t>(ex->svh_d),
-                                    dptr<float>(sc->plane), wt, o32, n, pairs, D, 1, S, E, true);
-        }
-        if (r) return r;
-        if (do_round) {
-            round_kernel<<<1024, 256, 0, s>>>(o32, (size_t)n * D);
-            r = launched();
-        }
+        // the pair plane summed in slot order; slots without an expert add nothing (the reference's route skips them)
+        prompt_combine_kernel<<<dim3(n, (D + 2047) / 2048), 256, 0, s>>>(
+            plane, pk, dptr<const uint16_t>(ex->svh_d), wt, static_cast<char*>(out) + (size_t)r0 * D * ob, (int)D, (int)E,
+            (int)S, half_sums ? OUT_F16 : do_round ? OUT_BF16R : OUT_F32, split);
+        r = launched();
         if (r) return r;
     }
     return EA_OK;
