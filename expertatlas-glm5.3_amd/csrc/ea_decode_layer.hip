@@ -460,9 +460,7 @@ __device__ __forceinline__ void mfma_tiles(const uint32_t* st, const LaneQuad& l
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int t0 = (2 * t + j) * TW, t1 = (2 * (t + 1) + j) * TW;
-            const u2v b0 = decode_quad<K2, CB>(wa[t0], wb[t0], lq.sh);
-            const u2v b1 = decode_quad<K2, CB>(wa[t1], wb[t1], lq.sh);
-            const h8v bb = __builtin_bit_cast(h8v, (u4v{b0.x, b0.y, b1.x, b1.y}));
+            const h8v bb = __builtin_bit_cast(h8v, decode_quads<K2, CB>(wa[t0], wb[t0], wa[t1], wb[t1], lq.sh));
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bb, acc[j], 0, 0, 0);
         }
     }
@@ -1351,9 +1349,7 @@ __device__ __forceinline__ void l1_mfma(const uint32_t* st, const LaneQuad& lq, 
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int t0 = (2 * t + j) * TW, t1 = (2 * (t + 1) + j) * TW;
-            const u2v b0 = decode_quad<K2, CB>(wa[t0], wb[t0], lq.sh);
-            const u2v b1 = decode_quad<K2, CB>(wa[t1], wb[t1], lq.sh);
-            const h8v bb = __builtin_bit_cast(h8v, (u4v{b0.x, b0.y, b1.x, b1.y}));
+            const h8v bb = __builtin_bit_cast(h8v, decode_quads<K2, CB>(wa[t0], wb[t0], wa[t1], wb[t1], lq.sh));
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bb, acc[j], 0, 0, 0);
         }
     }
@@ -1415,9 +1411,7 @@ __device__ __forceinline__ bool l1_down_product(const DLArgs& a, L1Sh& sh, int u
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int t0 = (4 * tp + j) * TW, t1 = (4 * tp + 2 + j) * TW;
-            const u2v b0 = decode_quad<K2, CB>(wa[t0], wb[t0], lq.sh);
-            const u2v b1 = decode_quad<K2, CB>(wa[t1], wb[t1], lq.sh);
-            pb[tp][j] = u4v{b0.x, b0.y, b1.x, b1.y};
+            pb[tp][j] = decode_quads<K2, CB>(wa[t0], wb[t0], wa[t1], wb[t1], lq.sh);
         }
 #pragma unroll
     for (int tp = 0; tp < PRE; ++tp)
@@ -1443,9 +1437,7 @@ __device__ __forceinline__ bool l1_down_product(const DLArgs& a, L1Sh& sh, int u
                 bq = pb[tp < PRE ? tp : 0][j];
             } else {
                 const int t0 = (4 * tp + j) * TW, t1 = (4 * tp + 2 + j) * TW;
-                const u2v b0 = decode_quad<K2, CB>(wa[t0], wb[t0], lq.sh);
-                const u2v b1 = decode_quad<K2, CB>(wa[t1], wb[t1], lq.sh);
-                bq = u4v{b0.x, b0.y, b1.x, b1.y};
+                bq = decode_quads<K2, CB>(wa[t0], wb[t0], wa[t1], wb[t1], lq.sh);
             }
             acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(h8v, bq), acc[j], 0, 0, 0);
         }

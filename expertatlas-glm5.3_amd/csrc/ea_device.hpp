@@ -158,6 +158,34 @@ __device__ __forceinline__ uint32_t cb_pair(uint32_t s0, uint32_t s1) {
     }
 }
 
+// Eight codebook values (two quads' clean 16-bit states) as four packed pairs: cb_pair's instructions with the four
+// pairs' fp16 adds interleaved, every first half before any second one. The three adds between a register's two
+// half-writes are the wait states that cb_pair spends on s_nop; only the readers of the last results still need theirs.
+// Four pairs on their own spend eight s_nop, this form one, which tells where few waves share a SIMD (decode windows of
+// 37 / 128 rows 268 -> 262 / 301 -> 294 us, one-row decode layers 16.1 -> 15.9 us).
+template <int CB>
+__device__ __forceinline__ u4v cb_quads(const uint32_t (&s)[8]) {
+    if constexpr (CB == CB_MUL1) {
+        return u4v{cb_pair<CB>(s[0], s[1]), cb_pair<CB>(s[2], s[3]), cb_pair<CB>(s[4], s[5]), cb_pair<CB>(s[6], s[7])};
+    } else {
+        uint32_t y[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const uint32_t x = (CB == CB_MCG) ? s[i] * 0xCBAC1FEDu : s[i] * 89226354u + 64248484u;
+            y[i] = __builtin_amdgcn_bitop3_b32(x, 0x8FFF8FFFu, 0x3B603B60u, 0x6A);
+        }
+#define EA_ADD_LO(r) "v_add_f16_sdwa " r ", " r ", " r " dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+#define EA_ADD_HI(r, b) "v_add_f16_sdwa " r ", " b ", " b " dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
+        asm(EA_ADD_LO("%0") EA_ADD_LO("%1") EA_ADD_LO("%2") EA_ADD_LO("%3") EA_ADD_HI("%0", "%4") EA_ADD_HI("%1", "%5")
+                EA_ADD_HI("%2", "%6") EA_ADD_HI("%3", "%7") "s_nop 1"
+            : "+v"(y[0]), "+v"(y[2]), "+v"(y[4]), "+v"(y[6])
+            : "v"(y[1]), "v"(y[3]), "v"(y[5]), "v"(y[7]));
+#undef EA_ADD_LO
+#undef EA_ADD_HI
+        return u4v{y[0], y[2], y[4], y[6]};
+    }
+}
+
 // A lane's view of four consecutive stream values p0 .. p0 + 3 (p0 even) of a tile, for K2 <= 10: their four
 // windows lie inside the 32 stream bits that start at the first window, so one funnel shift of two words gives
 // all four. Lane constants: the two word indices and the shift.
@@ -173,17 +201,16 @@ __host__ __device__ constexpr Quad quad_of(int p0) {
     return Quad{a % TW, (a + 1) % TW, 32 - (b0 - 32 * a)};
 }
 
-// The four values from the lane's two words: one funnel shift, then a bit-field extract a state.
-template <int K2, int CB>
-__device__ __forceinline__ u2v decode_quad(uint32_t wa, uint32_t wb, int sh) {
+// The four states from the lane's two words: one funnel shift, then a bit-field extract a state.
+template <int K2>
+__device__ __forceinline__ void quad_states(uint32_t wa, uint32_t wb, int sh, uint32_t* s) {
     static_assert(K2 >= 2 && K2 <= 10, "the four windows must fit in 32 stream bits");
     const uint32_t seg = __builtin_amdgcn_alignbit(wa, wb, (uint32_t)sh);
     constexpr int e0 = stream_end<K2>(0);
-    const uint32_t s0 = seg >> 16;
-    const uint32_t s1 = __builtin_amdgcn_ubfe(seg, 16 - (stream_end<K2>(1) - e0), 16);
-    const uint32_t s2 = __builtin_amdgcn_ubfe(seg, 16 - (stream_end<K2>(2) - e0), 16);
-    const uint32_t s3 = __builtin_amdgcn_ubfe(seg, 16 - (stream_end<K2>(3) - e0), 16);
-    return u2v{cb_pair<CB>(s0, s1), cb_pair<CB>(s2, s3)};
+    s[0] = seg >> 16;
+    s[1] = __builtin_amdgcn_ubfe(seg, 16 - (stream_end<K2>(1) - e0), 16);
+    s[2] = __builtin_amdgcn_ubfe(seg, 16 - (stream_end<K2>(2) - e0), 16);
+    s[3] = __builtin_amdgcn_ubfe(seg, 16 - (stream_end<K2>(3) - e0), 16);
 }
 
 // Wider widths (K2 11..16): the four windows span up to 40 stream bits, so the lane reads three words and makes a
@@ -200,20 +227,18 @@ __host__ __device__ constexpr Quad3 quad3_of(int p0) {
     return Quad3{a % TW, (a + 1) % TW, (a + 2) % TW, 32 - (b0 - 32 * a)};
 }
 
-template <int K2, int CB>
-__device__ __forceinline__ u2v decode_quad3(uint32_t w0, uint32_t w1, uint32_t w2, int sh) {
+template <int K2>
+__device__ __forceinline__ void quad3_states(uint32_t w0, uint32_t w1, uint32_t w2, int sh, uint32_t* s) {
     static_assert(K2 >= 11 && K2 <= 16, "three-word form");
     const uint32_t hi = __builtin_amdgcn_alignbit(w0, w1, (uint32_t)sh);
     const uint32_t lo = __builtin_amdgcn_alignbit(w1, w2, (uint32_t)sh);
     constexpr int e0 = stream_end<K2>(0);
-    uint32_t s[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int d = (i == 0) ? 0 : (i == 1 ? stream_end<K2>(1) - e0 : (i == 2 ? stream_end<K2>(2) - e0 : stream_end<K2>(3) - e0));
         s[i] = d <= 16 ? __builtin_amdgcn_ubfe(hi, 16 - d, 16)
                        : (__builtin_amdgcn_alignbit(hi, lo, (uint32_t)(48 - d)) & 0xffffu);
     }
-    return u2v{cb_pair<CB>(s[0], s[1]), cb_pair<CB>(s[2], s[3])};
 }
 
 // MFMA 16x16x16 f16 B-operand layout for one tile: lane l holds B[k'][n] for n = l & 15 and k' = 4 (l >> 4) + i.

@@ -8,6 +8,15 @@ namespace ea {
 
 typedef const __attribute__((address_space(1))) uint32_t* gptr_u32;
 
+// Two tiles' quads of staged words as the B operand of a two-tile k step (widths 2..10).
+template <int K2, int CB>
+__device__ __forceinline__ u4v decode_quads(uint32_t wa0, uint32_t wb0, uint32_t wa1, uint32_t wb1, int sh) {
+    uint32_t s[8];
+    quad_states<K2>(wa0, wb0, sh, s);
+    quad_states<K2>(wa1, wb1, sh, s + 4);
+    return cb_quads<CB>(s);
+}
+
 // A global-memory load the compiler can see is global (not flat): trellis tables hold plain 64-bit addresses.
 __device__ __forceinline__ uint32_t gload(const uint32_t* p) { return *(gptr_u32)(p); }
 
@@ -44,10 +53,22 @@ struct TileLane {
         w[1] = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * w1, soff, 0);
         if constexpr (NW == 3) w[2] = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * w2, soff, 0);
     }
+    __device__ __forceinline__ void states(const uint32_t (&w)[NW], uint32_t* s) const {
+        if constexpr (K2 <= 10) quad_states<K2>(w[0], w[1], sh, s);
+        else quad3_states<K2>(w[0], w[1], w[2], sh, s);
+    }
     // The four values as two packed words (values 0, 1 in .x; 2, 3 in .y).
     __device__ __forceinline__ u2v decode(const uint32_t (&w)[NW]) const {
-        if constexpr (K2 <= 10) return decode_quad<K2, CB>(w[0], w[1], sh);
-        else return decode_quad3<K2, CB>(w[0], w[1], w[2], sh);
+        uint32_t s[4];
+        states(w, s);
+        return u2v{cb_pair<CB>(s[0], s[1]), cb_pair<CB>(s[2], s[3])};
+    }
+    // Two tiles' quads as the B operand of a two-tile k step (16x16x32).
+    __device__ __forceinline__ u4v decode2(const uint32_t (&wa)[NW], const uint32_t (&wb)[NW]) const {
+        uint32_t s[8];
+        states(wa, s);
+        states(wb, s + 4);
+        return cb_quads<CB>(s);
     }
     // This lane's four B values of the tile starting at `tile`.
     __device__ __forceinline__ u2v decode_at(const uint32_t* __restrict__ tile) const {
@@ -103,9 +124,7 @@ __device__ __forceinline__ void wave_tiles(const uint32_t* __restrict__ base, si
     auto compute = [&](uint32_t (&w)[NTW][2][NWD], const h8v (&a)[MG]) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < NTW; ++j) {
-            const u2v b0 = tl.decode(w[j][0]);
-            const u2v b1 = tl.decode(w[j][1]);
-            const h8v b = __builtin_bit_cast(h8v, (u4v{b0.x, b0.y, b1.x, b1.y}));
+            const h8v b = __builtin_bit_cast(h8v, tl.decode2(w[j][0], w[j][1]));
 #pragma unroll
             for (int m = 0; m < MG; ++m) acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[m], b, acc[m][j], 0, 0, 0);
         }

@@ -381,9 +381,7 @@ __global__ void __launch_bounds__(1024) lin_small_kernel(ea_jobs jobs, ea_rot_jo
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int t0 = (2 * t + j) * TW, t1 = (2 * (t + 1) + j) * TW;
-                const u2v b0 = decode_quad<K2, CB>(wa[t0], wb[t0], lq.sh);
-                const u2v b1 = decode_quad<K2, CB>(wa[t1], wb[t1], lq.sh);
-                bq[t >> 1][j] = u4v{b0.x, b0.y, b1.x, b1.y};
+                bq[t >> 1][j] = decode_quads<K2, CB>(wa[t0], wb[t0], wa[t1], wb[t1], lq.sh);
             }
     }
 #pragma unroll

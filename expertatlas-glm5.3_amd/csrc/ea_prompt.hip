@@ -266,9 +266,11 @@ __device__ __forceinline__ void item_chunk(const uint32_t* st, const LaneQuad& l
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int t0 = (2 * t + j) * TW, t1 = (2 * (t + 1) + j) * TW;
-            const u2v b0 = decode_quad<K2, CB>(wa[t0], wb[t0], lq.sh);
-            const u2v b1 = decode_quad<K2, CB>(wa[t1], wb[t1], lq.sh);
-            bb[j] = __builtin_bit_cast(h8v, (u4v{b0.x, b0.y, b1.x, b1.y}));
+            uint32_t s[8];  // pair by pair: with the accumulators of several row tiles, eight states at once cost registers
+            quad_states<K2>(wa[t0], wb[t0], lq.sh, s);
+            quad_states<K2>(wa[t1], wb[t1], lq.sh, s + 4);
+            bb[j] = __builtin_bit_cast(h8v, (u4v{cb_pair<CB>(s[0], s[1]), cb_pair<CB>(s[2], s[3]),
+                                                 cb_pair<CB>(s[4], s[5]), cb_pair<CB>(s[6], s[7])}));
         }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
@@ -311,9 +313,8 @@ __device__ __forceinline__ void item_chunk1(const uint32_t* st, const LaneQuad& 
         h8v bb[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const u2v b0 = decode_quad<K2, CB>(w[b][2 * j][0], w[b][2 * j][1], lq.sh);
-            const u2v b1 = decode_quad<K2, CB>(w[b][2 * j + 1][0], w[b][2 * j + 1][1], lq.sh);
-            bb[j] = __builtin_bit_cast(h8v, (u4v{b0.x, b0.y, b1.x, b1.y}));
+            bb[j] = __builtin_bit_cast(h8v, decode_quads<K2, CB>(w[b][2 * j][0], w[b][2 * j][1], w[b][2 * j + 1][0],
+                                                                 w[b][2 * j + 1][1], lq.sh));
         }
         acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b], bb[0], acc[0][0], 0, 0, 0);
         acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b], bb[1], acc[0][1], 0, 0, 0);
