@@ -1,12 +1,12 @@
-// EXL3 linear for 1 to 128 rows (the shared expert and any strips-layout linear): input rotation for 1..3 jobs
-// of one input, and one launch over 1..3 jobs with per-job K splits finished by the last-arriving block
-// (exl3_linear.cu:69-484, exl3.zig, linear.zig). Rows are independent; sums run in a fixed order: waves of a
-// block in order, then splits in order.
+// EXL3 linear: input rotation for 1..3 jobs of one input, the one-launch kernel for few rows, and the entry points
+// (exl3_linear.cu:69-484, exl3.zig, linear.zig). More rows, and jobs of one K split, take ea_linear_rows.hip. Rows are
+// independent; sums run in a fixed order: waves of a block in order, then splits in order.
 #include <hip/hip_runtime.h>
 
 #include "ea_device.hpp"
 #include "ea_gemm.hpp"
 #include "ea_host.hpp"
+#include "ea_linear.hpp"
 #include "ea_stamps.hpp"
 
 namespace ea {
@@ -24,147 +24,6 @@ __global__ void __launch_bounds__(256) lin_rot_in_kernel(const void* __restrict_
     fwht128_w64(v0, v1, lane);
     *reinterpret_cast<uint32_t*>(xh + (size_t)row * K + k) =
         (uint32_t)f2h(v0 * HAD_SCALE) | ((uint32_t)f2h(v1 * HAD_SCALE) << 16);
-}
-
-// One row's 128 outputs of a column block from their fp32 sums (two a lane): FWHT, * HAD_SCALE * svh (+ bias),
-// stored as y_dtype (exl3_linear.cu:69-81).
-__device__ __forceinline__ void finish_store(float v0, float v1, int lane, const uint16_t* svh, const uint16_t* bias,
-                                             void* y, int y_dtype, size_t at, int col) {
-    fwht128_w64(v0, v1, lane);
-    v0 = v0 * HAD_SCALE * h2f(svh[col]);
-    v1 = v1 * HAD_SCALE * h2f(svh[col + 1]);
-    if (bias) {
-        v0 += h2f(bias[col]);
-        v1 += h2f(bias[col + 1]);
-    }
-    store_act(y, y_dtype, at, v0);
-    store_act(y, y_dtype, at + 1, v1);
-}
-
-// The same with svh and bias already loaded: sw, bw hold this lane's two columns (two fp16 each; bias optional).
-__device__ __forceinline__ void finish_store_pre(float v0, float v1, int lane, uint32_t sw, bool has_bias, uint32_t bw,
-                                                 void* y, int y_dtype, size_t at) {
-    fwht128_w64(v0, v1, lane);
-    v0 = v0 * HAD_SCALE * h2f((uint16_t)(sw & 0xffffu));
-    v1 = v1 * HAD_SCALE * h2f((uint16_t)(sw >> 16));
-    if (has_bias) {
-        v0 += h2f((uint16_t)(bw & 0xffffu));
-        v1 += h2f((uint16_t)(bw >> 16));
-    }
-    store_act(y, y_dtype, at, v0);
-    store_act(y, y_dtype, at + 1, v1);
-}
-
-__device__ __forceinline__ float load_coherent(const float* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Block (job, column block nb of 128, split; pass of 16 rows = blockIdx.y): WK waves each take per_warp consecutive k
-// tiles of the split for the pass's rows. Every pass is its own block (the passes decode the same tiles side by side,
-// not one after another: 128 rows of a 6144 x 256 linear are 256 blocks, not 32 blocks of eight passes). SK == 1: the
-// block finishes its columns. SK > 1: partial sums to Z[split], and the block that arrives last on the (pass, nb)
-// counter sums the splits in order, finishes, and resets the counter to zero.
-template <int CB, int K2, int WK>
-__global__ void __launch_bounds__(WK * 64) linear_kernel(ea_jobs jobs, int M, int K) {
-    int ji = 0;
-#pragma unroll
-    for (int q = 1; q < EA_MAX_JOBS; ++q)
-        if (q < jobs.n && (int)blockIdx.x >= jobs.j[q].start) ji = q;
-    const ea_job& J = jobs.j[ji];
-    const uint16_t* __restrict__ xh = dptr<const uint16_t>(J.xh);
-    const uint32_t* __restrict__ T = dptr<const uint32_t>(J.T);
-    const uint16_t* svh = dptr<const uint16_t>(J.svh);
-    const uint16_t* bias = dptr<const uint16_t>(J.bias);
-    void* y = dptr<void>(J.y);
-    float* Z = dptr<float>(J.Z);
-    int* counters = dptr<int>(J.counters);
-    const int N = J.N, SK = J.SK, NB = N >> 7;
-    const int local = (int)blockIdx.x - J.start, nb = local % NB, split = local / NB;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int per_warp = (K >> 4) / SK / WK;
-    const int kt0 = split * (per_warp * WK) + wave * per_warp;
-    const uint32_t* base = T + nb * J.stride_nb + (int64_t)kt0 * J.stride_k;
-    const int col0 = nb * 128;
-
-    __shared__ float red[WK][16][128];
-    __shared__ int last;
-    {
-        const int pass = (int)blockIdx.y, m0 = 16 * pass;
-        const int R = min(16, M - m0);
-        const int r = m0 + (lane & 15);
-        const uint16_t* const xrow[1] = {r < M ? xh + (size_t)r * K : nullptr};
-        f4v acc[1][8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[0][j] = f4v{0.f, 0.f, 0.f, 0.f};
-        wave_tiles<CB, K2, 8, 1>(base, (size_t)J.stride_k, per_warp, kt0 * 16, xrow, lane, acc);
-        __syncthreads();  // red is free (the previous pass has read it)
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) red[wave][4 * (lane >> 4) + i][j * 16 + (lane & 15)] = acc[0][j][i];
-        __syncthreads();
-        if (SK == 1) {
-            for (int rr = wave; rr < R; rr += WK) {
-                float v0 = red[0][rr][2 * lane], v1 = red[0][rr][2 * lane + 1];
-#pragma unroll
-                for (int w = 1; w < WK; ++w) {
-                    v0 += red[w][rr][2 * lane];
-                    v1 += red[w][rr][2 * lane + 1];
-                }
-                finish_store(v0, v1, lane, svh, bias, y, J.y_dtype, (size_t)(m0 + rr) * N + col0 + 2 * lane,
-                             col0 + 2 * lane);
-            }
-        } else {
-            for (int idx = threadIdx.x; idx < R * 128; idx += WK * 64) {
-                const int rr = idx >> 7, c = idx & 127;
-                float s = red[0][rr][c];
-#pragma unroll
-                for (int w = 1; w < WK; ++w) s += red[w][rr][c];
-                Z[((size_t)split * M + m0 + rr) * N + col0 + c] = s;
-            }
-            __threadfence();
-            __syncthreads();
-            if (threadIdx.x == 0) last = atomicAdd(counters + pass * NB + nb, 1) == SK - 1;
-            __syncthreads();
-            if (last) {
-                __threadfence();
-                // the wave's rows wave, wave + WK, ..: QB splits of all of them loaded at once (64 values a lane),
-                // then added in split order (one round trip a batch of splits instead of one a split and row)
-                constexpr int RW = 16 / WK, QB = 32 / RW;
-                float v[RW][2];
-                for (int q0 = 0; q0 < SK; q0 += QB) {
-                    float z[QB][RW][2];
-#pragma unroll
-                    for (int q = 0; q < QB; ++q)
-#pragma unroll
-                        for (int i = 0; i < RW; ++i) {
-                            const int rr = wave + WK * i < R ? wave + WK * i : wave;  // rows past R re-read a row
-                            const size_t at = (size_t)(q0 + q < SK ? q0 + q : q0) * M * N +
-                                              ((size_t)m0 + rr) * N + col0 + 2 * lane;
-                            z[q][i][0] = load_coherent(Z + at);
-                            z[q][i][1] = load_coherent(Z + at + 1);
-                        }
-#pragma unroll
-                    for (int q = 0; q < QB; ++q)
-                        if (q0 + q < SK) {  // uniform
-#pragma unroll
-                            for (int i = 0; i < RW; ++i) {
-                                v[i][0] = q0 + q == 0 ? z[q][i][0] : v[i][0] + z[q][i][0];
-                                v[i][1] = q0 + q == 0 ? z[q][i][1] : v[i][1] + z[q][i][1];
-                            }
-                        }
-                }
-#pragma unroll
-                for (int i = 0; i < RW; ++i) {
-                    const int rr = wave + WK * i;
-                    if (rr >= R) break;  // uniform
-                    const size_t at = ((size_t)m0 + rr) * N + col0 + 2 * lane;
-                    finish_store(v[i][0], v[i][1], lane, svh, bias, y, J.y_dtype, at, col0 + 2 * lane);
-                }
-                if (threadIdx.x == 0) counters[pass * NB + nb] = 0;  // every split of the column block arrived
-            }
-        }
-    }
 }
 
 // ---- the small-row linear: up to 16 rows, K split, every CU busy ----------------------------------------------------
@@ -598,10 +457,10 @@ static int small_grid(ea_jobs& sj) {
     return nb;
 }
 
-// The small-row kernel when it applies (m <= 16, every job split (SK > 1) with the same even per-wave tile count up to
+// The small-row kernel when it applies (few rows, see below; every job split (SK > 1) with the same even per-wave tile count up to
 // 16, a width the staged decode takes, 16-bit activations when rotating); false otherwise, and nothing is launched.
 static bool launch_small(const ea_jobs& jobs, const ea_rot_jobs* rj, hipStream_t s, int M, int K, uint32_t k2,
-                         uint32_t cb, int wk, const void* x, int x_dtype, int* status) {
+                         uint32_t cb, int wk, const void* x, int x_dtype, int* status, int cus) {
     if (M > 128 || k2 > (uint32_t)STAGE_MAXK2) return false;
     if (rj && x_dtype != F16 && x_dtype != BF16) return false;
     const uintptr_t align = rj ? reinterpret_cast<uintptr_t>(x) | (uintptr_t)K * 2 : (uintptr_t)K * 2;
@@ -624,6 +483,15 @@ static bool launch_small(const ea_jobs& jobs, const ea_rot_jobs* rj, hipStream_t
     for (int i = 0; i < tj.n; ++i) tj.j[i].SK /= 2;
     ea_jobs sj = jobs;
     const int tb = small_grid(tj), nb = small_grid(sj);
+    // Where this kernel stops and the one for more rows (launch_linear_rows, two launches, each tile decoded once) is the
+    // better one. At 6144 x 2048: 4 rows 8.8 against 10.3 us, 8 rows 11.2 against 10.3, 16 rows 19.6 against 10.4. With
+    // more blocks a pass than CUs it is earlier (2048 x 6144: 4 rows 11.2 against 10.8). With few blocks the passes run at
+    // once and it is later, the later if no split is handed over (1024 x 640: 8.3 against 8.5 us up to 48 rows).
+    bool one = tag;
+    for (int i = 0; i < jobs.n; ++i) one = one && jobs.j[i].SK == 2;
+    const int passes = (M + LS_PASS - 1) / LS_PASS;
+    const bool few = tag && (one ? tb * passes <= cus : tb * passes < cus / 2);
+    if (M >= (tag && tb > cus ? 4 : 8) && !few) return false;
     // the tagged form on sixteen waves a block (four a SIMD) when its waves' k tiles halve evenly once more: the
     // same decode over twice the waves (config 1: 8.64 -> 8.55 us)
     int tw = 2 * wk, tn = nkt;
@@ -652,26 +520,6 @@ static bool launch_small(const ea_jobs& jobs, const ea_rot_jobs* rj, hipStream_t
 }
 
 // the (K2, codebook) pairs this build instantiates: the reference's four (exl3.zig:40) and 3 / 4 bits mcg
-template <int CB, int K2>
-static void launch_wk(const ea_jobs& jobs, int blocks, hipStream_t s, int M, int K, int wk) {
-    const dim3 grid((unsigned)blocks, (unsigned)((M + 15) / 16));  // passes of 16 rows side by side
-    if (wk == 2) linear_kernel<CB, K2, 2><<<grid, 2 * 64, 0, s>>>(jobs, M, K);
-    else if (wk == 4) linear_kernel<CB, K2, 4><<<grid, 4 * 64, 0, s>>>(jobs, M, K);
-    else linear_kernel<CB, K2, 8><<<grid, 8 * 64, 0, s>>>(jobs, M, K);
-}
-
-static bool launch_variant(const ea_jobs& jobs, int blocks, hipStream_t s, int M, int K, uint32_t k2, uint32_t cb,
-                           int wk) {
-#define EA_LV(K2_, CB_)                                            \
-    if (k2 == K2_ && cb == CB_) {                                  \
-        launch_wk<CB_, K2_>(jobs, blocks, s, M, K, wk);            \
-        return true;                                               \
-    }
-    EA_LV(10, 2) EA_LV(12, 2) EA_LV(8, 1) EA_LV(8, 2) EA_LV(6, 1) EA_LV(4, 1)
-#undef EA_LV
-    return false;
-}
-
 static bool variant_built(uint32_t k2, uint32_t cb, uint32_t wk) {
     if (wk != 2 && wk != 4 && wk != 8) return false;
     return (cb == 2 && (k2 == 10 || k2 == 12 || k2 == 8)) || (cb == 1 && (k2 == 8 || k2 == 6 || k2 == 4));
@@ -710,13 +558,9 @@ int launch_linear(hipStream_t s, const ea_jobs* jobs_in, uint32_t m, uint32_t kd
     if (!variant_built(k2, cb, wk)) return EA_UNPORTED_LINEAR_VARIANT;
     if (m == 0 || blocks == 0) return EA_OK;
     if (m > 128) return EA_NOT_GROUPABLE;
-    if (launch_small(jobs, rot, s, (int)m, (int)kdim, k2, cb, (int)wk, x, x_dtype, c->status)) return launched();
-    if (rot) {
-        const int r = launch_lin_rot_in(s, x, x_dtype, rot, (uint32_t)jobs.n, m, kdim);
-        if (r) return r;
-    }
-    launch_variant(jobs, blocks, s, (int)m, (int)kdim, k2, cb, (int)wk);
-    return launched();
+    if (launch_small(jobs, rot, s, (int)m, (int)kdim, k2, cb, (int)wk, x, x_dtype, c->status, c->cus))
+        return launched();
+    return launch_linear_rows(s, jobs, rot, (int)m, (int)kdim, k2, cb, x, x_dtype);
 }
 
 }  // namespace ea

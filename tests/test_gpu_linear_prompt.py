@@ -126,6 +126,46 @@ def test_linear_three_jobs_one_launch(ea):
         assert int(device.download(l.counters).sum()) == 0
 
 
+@pytest.mark.parametrize("M,K,Ns,k2,cb", [
+    (4, 2048, (6144,), 8, 1),       # more blocks than CUs on the one-row kernel: from four rows on here
+    (8, 6144, (2048,), 8, 1), (9, 1152, (384,), 6, 1), (15, 6144, (256, 256), 10, 2), (16, 384, (128,), 4, 1),
+    (17, 640, (8192,), 8, 2),       # one split, the finish in the block, a ragged chunk (five Hadamard blocks)
+    (31, 256, (6144,), 12, 2), (33, 2048, (1024, 128), 8, 1), (64, 6144, (256, 256), 10, 2), (65, 1536, (640,), 12, 2),
+    (97, 6144, (2048,), 6, 1), (127, 2048, (6144,), 8, 1),
+])
+@pytest.mark.parametrize("x_dtype", [1, 2])
+def test_linear_many_rows(ea, M, K, Ns, k2, cb, x_dtype):
+    """The launches that decode each tile once for all rows: the edges of row tiles, chunks and splits, several jobs,
+    rotated inside the products (16-bit x, few blocks) or before them (fp32 x). Against the oracle: fp32 sums of K
+    products of fp16 in another order, 1e-4 * RMS as for the other forms."""
+    device, linear, _, _, synth = ea
+    x = synth.activations(170 + M, M, K, "bf16" if x_dtype == 1 else "f32")
+    lins, wants, outs = [], [], []
+    for i, N in enumerate(Ns):
+        T = synth.trellis(171 + i, 0, 0, 0, K, N, k2)
+        suh, svh = synth.scales(172 + i, K, 1.0), synth.scales(173 + i, N, 0.02)
+        lin = linear.Linear(T, suh, svh, K, N, k2, cb)
+        xh = orc.exl3_rot_in(x, suh, M, K, bf16=x_dtype == 1)
+        tw = 4 * k2
+        lins.append(lin)
+        wants.append((xh, orc.exl3_linear(xh, linear.strips(T, K, N, k2), 8 * tw, (K // 16) * 8 * tw, svh, M, K, N, k2,
+                                          cb, lin.sk, lin.wk)))
+        outs.append(device.zeros((M, N), torch.float32))
+    sc = linear.Scratch(M, K, max(l.sk * M * l.n for l in lins))
+    dx = device.upload(x)
+    for rep in range(2):
+        linear.call(device.stream(), sc, lins, dx.data_ptr(), x_dtype, M, [o.data_ptr() for o in outs], [2] * len(lins))
+        for i, (o, (xh, w), l) in enumerate(zip(outs, wants, lins)):
+            np.testing.assert_array_equal(device.download(sc.xh[i][: M * K].view(torch.int16)).reshape(M, K), xh)
+            assert_close_rms(device.download(o), w, 1e-4, f"M={M} job {i} rep={rep}")
+            assert int(device.download(l.counters).sum()) == 0
+    first = [device.download(o) for o in outs]
+    linear.call_rotated(device.stream(), sc, lins, M, [o.data_ptr() for o in outs], [2] * len(lins))
+    for o, w in zip(outs, wants):
+        assert_close_rms(device.download(o), w[1], 1e-4, f"M={M} rotated")
+    assert device.device_status() == 0 and all(np.isfinite(f).all() for f in first)
+
+
 def test_linear_errors(ea):
     device, linear, _, _, synth = ea
     from ea_exl3._lib import EaError
