@@ -233,6 +233,10 @@ constexpr int PXS = PK * 16 + 8;                  // LDS row stride of a staged 
 constexpr int PW = 4;                             // waves a block: 8 column tiles, 128 columns
 constexpr int PSTAGE = PK * 2 * 4 * STAGE_MAXK2;  // a wave's staged trellis words a chunk
 constexpr int DNG = 16;  // down matrix: column blocks of 128 a block, small items (8, 24 and 48 measured slower at 512 rows)
+// the same in a decode window, whose items are too few to fill the GPU with blocks that long (37 rows, 112 experts: 336
+// blocks of 16 column blocks took 71 us, 1,344 of 4 take 39)
+constexpr int DNG_WINDOW = 4;
+constexpr int WINDOW_ROWS_MAX = 128;  // the widest decode window (forward.zig:21)
 constexpr int DNG_BIG = 2;  // the same for the larger items: more blocks for fewer items (4: 1 % slower at 512 rows)
 constexpr int DNG_BIG_LONG = 4;   // passes of more than LONG_ROWS rows: 1.5 % faster at 2048 rows
 constexpr int LONG_ROWS = 1024;
@@ -465,10 +469,11 @@ item_gu_kernel(const uint16_t* __restrict__ X0, const uint16_t* __restrict__ X1,
 // (filled >= NW (c / RING_S + 1)), computes it, and counts itself done. The slowest wave can always go on (every
 // chunk it waits for was stored at a step no later than its own, and every slot it stores into was freed before),
 // so every wait ends. Each wave's trellis goes through its own LDS region as in gu_loop; the activation piece of a
-// chunk (1/NW of it) and the trellis are loaded two chunks ahead. The nch chunks are summed as nsum splits
-// ([s nch / nsum, (s + 1) nch / nsum)), each accumulated from zero and added in order into tot (from zero): the bits
-// of a K-split item's sum of its split planes (item_gu_kernel, summed by the epilogue), so a pair's sums do not
-// depend on which list its item is in.
+// chunk (1/NW of it) and the trellis are loaded two chunks ahead. K is split as the larger items' is, over the same
+// chunk ranges and into the same planes, so a pair's sums do not depend on which list its item is in. (Decode windows
+// are bound by the waves there are, not by their work: 37 rows touch about 112 experts, and one block an (item, 128
+// columns, matrix) over all of K left 1.75 blocks a CU: 118 us, against 67 with the
+// two splits. Prompts of 512 and 2048 rows measured the same either way.)
 constexpr int RING_S = 6;  // activation chunk slots
 constexpr int RING_L = 2;  // a wave stores its piece of chunk c + RING_L at its step c
 
@@ -496,8 +501,8 @@ __device__ __forceinline__ bool lds_wait_geq(const int* p, int target) {
 
 template <int CB, int K2, int NW>
 __device__ __forceinline__ void ring_loop(__amdgpu_buffer_rsrc_t xrs, uint32_t aoff, int lofs, const TileSpan& sp,
-                                          uint16_t* ring, int* filled, int* done, uint32_t* st, int lane, int nch,
-                                          int nsum, f4v (&acc)[1][2], f4v (&tot)[1][2], bool& synced) {
+                                          uint16_t* ring, int* filled, int* done, uint32_t* st, int lane, int c0,
+                                          int nch, f4v (&acc)[1][2], bool& synced) {
     constexpr int NL = stage_loads_k<PK, K2>();
     constexpr int W = RingPiece<NW>::WORDS;  // 2 or 4
     constexpr int SLOT = 16 * PXS;
@@ -505,16 +510,15 @@ __device__ __forceinline__ void ring_loop(__amdgpu_buffer_rsrc_t xrs, uint32_t a
     const LaneQuad lq = lane_quad_k<K2>(lane);
     pv pa, pb;
     u4v ta[NL], tb[NL];
-    int sn = 1;  // the next split's index
     auto issue_p = [&](int c, pv& v) __attribute__((always_inline)) {
-        c = c < nch ? c : nch - 1;
+        c = c0 + (c < nch ? c : nch - 1);
         if constexpr (W == 4)
             v = __builtin_bit_cast(pv, __builtin_amdgcn_raw_buffer_load_b128(xrs, aoff, c * PK * 32, 0));
         else
             v = __builtin_bit_cast(pv, __builtin_amdgcn_raw_buffer_load_b64(xrs, aoff, c * PK * 32, 0));
     };
     auto issue_t = [&](int c, u4v (&tv)[NL]) __attribute__((always_inline)) {
-        c = c < nch ? c : nch - 1;
+        c = c0 + (c < nch ? c : nch - 1);
         TileSpan sc = sp;
         sc.off = sp.off + c * PK * sp.kstride;
         stage_issue_k<PK, K2>(sc, lane, tv);
@@ -541,14 +545,6 @@ __device__ __forceinline__ void ring_loop(__amdgpu_buffer_rsrc_t xrs, uint32_t a
         synced = synced && lds_wait_geq(&filled[sl], NW * (c / RING_S + 1));
         item_chunk1<CB, K2>(st, lq, ring + sl * SLOT, lane, acc, PXS);
         lds_add_release(&done[sl], 1, lane);  // after the chunk's reads of the slot have returned
-        if (c + 1 == sn * nch / nsum) {  // the end of a split (uniform)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                tot[0][j] += acc[0][j];
-                acc[0][j] = f4v{0.f, 0.f, 0.f, 0.f};
-            }
-            ++sn;
-        }
     };
     // chunks 0 .. RING_L - 1 go in before the loop; pa / pb then carry chunks RING_L and RING_L + 1
     for (int p = 0; p < RING_L && p < nch; ++p) {
@@ -573,10 +569,11 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4)
 item_ring_kernel(const uint16_t* __restrict__ X0, const uint16_t* __restrict__ X1, const int64_t* __restrict__ TP0,
                  const int64_t* __restrict__ TP1, const int* __restrict__ K2_0, const int* __restrict__ K2_1,
                  const int* __restrict__ sorted, const int* __restrict__ items, const int* __restrict__ item_count,
-                 float* __restrict__ Z, int K, int N, int P, int nsum, int max_items, int* __restrict__ status) {
+                 float* __restrict__ Z, float* __restrict__ Zp, int K, int N, int P, int nsplit, int max_items,
+                 int* __restrict__ status) {
     int e, first, cnt;
     if (!item_at(items, item_count, 0, max_items, blockIdx.x, e, first, cnt)) return;
-    const int mat = blockIdx.z;
+    const int mat = blockIdx.z / nsplit, split = blockIdx.z % nsplit;
     const uint16_t* X = mat ? X1 : X0;
     const uint32_t* T = reinterpret_cast<const uint32_t*>(mat ? TP1[e] : TP0[e]);
     const int k2 = mat ? K2_1[e] : K2_0[e];
@@ -602,24 +599,25 @@ item_ring_kernel(const uint16_t* __restrict__ X0, const uint16_t* __restrict__ X
     sp.r = buffer_rsrc(T, (uint32_t)((K >> 4) * ns * TWB));
     sp.off = nt0 * TWB;
     sp.kstride = ns * TWB;
-    f4v acc[1][2], tot[1][2];
-    acc[0][0] = acc[0][1] = tot[0][0] = tot[0][1] = f4v{0.f, 0.f, 0.f, 0.f};
+    f4v acc[1][2];
+    acc[0][0] = acc[0][1] = f4v{0.f, 0.f, 0.f, 0.f};
     const int nch = K / (PK * 16);
+    const int c0 = split * nch / nsplit, nc = (split + 1) * nch / nsplit - c0;  // nsplit <= nch: nc >= 1
     bool synced = true;
     const bool ok = EA_K2_SWITCH(k2, 2, 10,
-                                 (ring_loop<CB, K2V, NW>(xrs, aoff, lofs, sp, ring, filled, done, st[wave], lane, nch,
-                                                         nsum, acc, tot, synced)));
+                                 (ring_loop<CB, K2V, NW>(xrs, aoff, lofs, sp, ring, filled, done, st[wave], lane, c0,
+                                                         nc, acc, synced)));
     if (!ok || !synced) {
         if (lane == 0) record_error(status, ok ? DEV_SYNC_TIMEOUT : DEV_UNSUPPORTED_WIDTH);
-        tot[0][0] = tot[0][1] = nan4();
+        acc[0][0] = acc[0][1] = nan4();
     }
-    float* Zm = Z + (size_t)mat * P * N;
+    float* Zm = (split ? Zp + (size_t)(split - 1) * 2 * P * N : Z) + (size_t)mat * P * N;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int pp = pair_sh[4 * (lane >> 4) + i];
         if (pp < 0) continue;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) Zm[(size_t)pp * N + (nt0 + j) * 16 + (lane & 15)] = tot[0][j][i];
+        for (int j = 0; j < 2; ++j) Zm[(size_t)pp * N + (nt0 + j) * 16 + (lane & 15)] = 0.f + acc[0][j][i];
     }
 }
 
@@ -918,14 +916,14 @@ static int list_pass(hipStream_t q, const ListPass& a, int big) {
             a.xg, a.xu, a.tp[0], a.tp[1], a.k2[0], a.k2[1], a.sorted, a.items, a.count, a.z, a.zp, a.D, a.I, a.P, ns,
             2, a.mi, a.status);
     else  // blocks of 4 waves over 128 columns (8 waves over 256 measured 1 % slower at 512 rows, the same at 2048)
-        item_ring_kernel<CB, 4><<<dim3(a.mi, a.I / 128, 2), 4 * 64, 0, q>>>(
-            a.xg, a.xu, a.tp[0], a.tp[1], a.k2[0], a.k2[1], a.sorted, a.items, a.count, a.z, a.D, a.I, a.P, ns, a.mi,
-            a.status);
+        item_ring_kernel<CB, 4><<<dim3(a.mi, a.I / 128, 2 * ns), 4 * 64, 0, q>>>(
+            a.xg, a.xu, a.tp[0], a.tp[1], a.k2[0], a.k2[1], a.sorted, a.items, a.count, a.z, a.zp, a.D, a.I, a.P, ns,
+            a.mi, a.status);
     int r = launched();
     if (r) return r;
     r = launch_gateup_epilogue(q, a.z, a.pick, a.svh_g, a.svh_u, a.suh_d, a.xd, (uint32_t)a.rows, (uint32_t)a.P,
-                               (uint32_t)a.I, 1, (uint32_t)a.slots, (uint32_t)a.E, __builtin_inff(), 1, a.pclass, a.zp,
-                               (uint32_t)ns, big);
+                               (uint32_t)a.I, (uint32_t)ns, (uint32_t)a.slots, (uint32_t)a.E, __builtin_inff(), 1, a.zp, a.pclass,
+                               big);
     if (r) return r;
     const int nb = a.D / 128;
     if (a.I <= 2 * PK * 16 && nb % 2 == 0) {
@@ -938,6 +936,8 @@ static int list_pass(hipStream_t q, const ListPass& a, int big) {
             EA_DN(IPM_TILES, DNG_BIG, 2 * PW, xcd_blocks(a.mi, 1, nb / DNG_BIG));
         else if (big)
             EA_DN(IPM_TILES, DNG_BIG, PW, xcd_blocks(a.mi, 1, nb / DNG_BIG));
+        else if (a.rows <= WINDOW_ROWS_MAX && nb % DNG_WINDOW == 0)
+            EA_DN(SMALL_ROWS / 16, DNG_WINDOW, PW, dim3(a.mi, nb / DNG_WINDOW, 1));
         else if (nb % DNG == 0)
             EA_DN(SMALL_ROWS / 16, DNG, PW, dim3(a.mi, nb / DNG, 1));
         else
@@ -949,8 +949,8 @@ static int list_pass(hipStream_t q, const ListPass& a, int big) {
             a.P, 1, 1, a.mi, a.status);
     } else {
         item_ring_kernel<CB, 4><<<dim3(a.mi, a.D / 128, 1), 4 * 64, 0, q>>>(
-            a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, a.I, a.D, a.P, 1,
-            a.mi, a.status);
+            a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, nullptr, a.I, a.D, a.P,
+            1, a.mi, a.status);
     }
     return launched();
 }
