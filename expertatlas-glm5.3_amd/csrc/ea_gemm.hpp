@@ -53,6 +53,12 @@ struct TileLane {
         w[1] = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * w1, soff, 0);
         if constexpr (NW == 3) w[2] = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * w2, soff, 0);
     }
+    // The same from LDS.
+    __device__ __forceinline__ void staged(const uint32_t* tile, uint32_t (&w)[NW]) const {
+        w[0] = tile[w0];
+        w[1] = tile[w1];
+        if constexpr (NW == 3) w[2] = tile[w2];
+    }
     __device__ __forceinline__ void states(const uint32_t (&w)[NW], uint32_t* s) const {
         if constexpr (K2 <= 10) quad_states<K2>(w[0], w[1], sh, s);
         else quad3_states<K2>(w[0], w[1], w[2], sh, s);

@@ -1,0 +1,637 @@
+// The item lists of a prompt pass (ea_prompt.hip): the gate|up and down products of items of one expert's routed pairs,
+// and one list's launches. Included by the sources that instantiate it for widths up to 10 and up to 16.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "ea_device.hpp"
+#include "ea_experts.hpp"
+#include "ea_gemm.hpp"
+#include "ea_host.hpp"
+
+namespace ea {
+
+// Routed pairs an item at most: five row tiles. The reference's items hold up to 112 (prompt_experts.cu:55-58,
+// TF_PE_GPM). 80 against 48: the same at 512 rows and 3-4 % faster at 2048 (a heavy expert decoded in fewer items);
+// against 112 (seven row tiles, more accumulators) faster at both; 64 and 96 measured between. A pair's sums do not
+// depend on its item.
+constexpr int IPM = 80;
+constexpr int IPM_TILES = IPM / 16;
+
+constexpr int SMALL_ROWS = 16;     // items of at most this many pairs: the kernels holding one row tile
+
+// Item i of list `big` (0: items of at most SMALL_ROWS pairs, from the front of items[]; 1: the others, from its
+// back), or false past the list's count.
+__device__ __forceinline__ bool item_at(const int* __restrict__ items, const int* __restrict__ count, int big,
+                                        int max_items, int i, int& e, int& first, int& cnt) {
+    if (i >= count[big]) return false;
+    const int at = big ? max_items - 1 - i : i;
+    e = items[3 * at];
+    first = items[3 * at + 1];
+    cnt = items[3 * at + 2];
+    return true;
+}
+
+// ---- the pair plane -----------------------------------------------------------------------------------------------
+
+// Where the down products go: fp32 [pairs, D] rows of one plane, or (a scratch without a plane) each pair's row split in
+// two halves of D / 2 columns over the pair's own rotated inputs, which the pair's gate|up product has read by then: the
+// lower columns in its xg row, the upper in its xu row (D fp16 = D / 2 fp32 each). The item lists run side by side, but a
+// pair's rows belong to one list, whose gate|up precedes its down product on one stream. Column col of pair p is at
+// base(col)[p * stride + col].
+struct PairPlane {
+    float *lo, *hi;  // hi already moved back by half columns
+    int half, stride;
+    __host__ __device__ float* base(int col) const { return col < half ? lo : hi; }
+};
+
+// ---- the staged item GEMM --------------------------------------------------------------------------------------
+// Every kernel is built for widths up to MK: 10 (two trellis words a lane a tile), or 16 (three words above 10, larger
+// staging regions) for layers that hold a wider expert.
+
+constexpr int PK = 8;                             // k tiles a chunk: 128 k
+constexpr int PXS = PK * 16 + 8;                  // LDS row stride of a staged activation chunk, halves (272 bytes)
+constexpr int PW = 4;                             // waves a block: 8 column tiles, 128 columns
+constexpr int pstage(int mk) { return PK * 2 * 4 * mk; }  // a wave's staged trellis words a chunk
+constexpr int DNG = 16;  // down matrix: column blocks of 128 a block, small items (8, 24 and 48 measured slower at 512 rows)
+// the same in a decode window, whose items are too few to fill the GPU with blocks that long (37 rows, 112 experts: 336
+// blocks of 16 column blocks took 71 us, 1,344 of 4 take 39)
+constexpr int DNG_WINDOW = 4;
+constexpr int WINDOW_ROWS_MAX = 128;  // the widest decode window (forward.zig:21)
+constexpr int DNG_BIG = 2;  // the same for the larger items: more blocks for fewer items (4: 1 % slower at 512 rows)
+constexpr int DNG_BIG_LONG = 4;   // passes of more than LONG_ROWS rows: 1.5 % faster at 2048 rows
+constexpr int LONG_ROWS = 1024;
+constexpr int GU_SPLIT = 2;                       // K splits of a larger item's gate|up (4 and 8 measured slower)
+// The number of K splits of a larger item's gate|up over K (at most one a chunk).
+static int gu_splits(int K) { return K / (PK * 16) < GU_SPLIT ? K / (PK * 16) : GU_SPLIT; }
+constexpr int DXS = 2 * PK * 16 + 8;              // down matrix: LDS row stride of the activations (K up to 256)
+
+// An activation piece (8 halves: column 8 q8 .. +7 of a chunk row) into LDS. Within each 32-k step of the row
+// (16 words) word d goes to 4 (d & 3) + (d >> 2), so the words of a lane's MFMA operand (g, g + 4, g + 8, g + 12 of
+// the step: the k order in which the trellis quads fill the B operand) are one 16-byte read.
+__device__ __forceinline__ void put_a(uint16_t* row, int q8, const u4v& v) {
+    uint32_t* w = reinterpret_cast<uint32_t*>(row) + 16 * (q8 >> 2) + (q8 & 3);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w[4 * r] = v[r];
+}
+
+// One chunk (PK k tiles) of a wave: its two column tiles times the item's first mts (<= MT) row tiles. The trellis
+// words are staged in st (tile (t, j) at word (2 t + j) * 4 K2), the activations in xa (row stride xs halves, laid
+// out by put_a); each tile pair decodes once and feeds all row tiles.
+template <int CB, int K2, int MT>
+__device__ __forceinline__ void item_chunk(const uint32_t* st, const TileLane<K2, CB>& tl, const uint16_t* xa, int mts,
+                                           int lane, f4v (&acc)[MT][2], int xs) {
+    constexpr int TW = 4 * K2, NWD = TileLane<K2, CB>::NW;
+    const uint16_t* xr = xa + (lane & 15) * xs + 8 * ((lane >> 4) & 3);
+#pragma unroll
+    for (int t = 0; t < PK; t += 2) {
+        h8v bb[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            uint32_t w[2][NWD], s[8];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                tl.staged(st + (2 * (t + h) + j) * TW, w[h]);
+                tl.states(w[h], s + 4 * h);
+            }
+            // pair by pair: with the accumulators of several row tiles, eight states at once cost registers
+            bb[j] = __builtin_bit_cast(h8v, (u4v{cb_pair<CB>(s[0], s[1]), cb_pair<CB>(s[2], s[3]),
+                                                 cb_pair<CB>(s[4], s[5]), cb_pair<CB>(s[6], s[7])}));
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            if (mt >= mts) break;  // the item's occupied row tiles only (uniform)
+            const h8v a = *reinterpret_cast<const h8v*>(xr + mt * 16 * xs + t * 16);
+            acc[mt][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bb[0], acc[mt][0], 0, 0, 0);
+            acc[mt][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bb[1], acc[mt][1], 0, 0, 0);
+        }
+    }
+}
+
+// One chunk for a single row tile with the LDS reads one k step ahead: the trellis words and the activation operand
+// of k step t + 1 are read before k step t decodes, so each read's latency overlaps a step of decoding.
+template <int CB, int K2>
+__device__ __forceinline__ void item_chunk1(const uint32_t* st, const TileLane<K2, CB>& tl, const uint16_t* xa, int lane,
+                                            f4v (&acc)[1][2], int xs) {
+    constexpr int TW = 4 * K2, NWD = TileLane<K2, CB>::NW;
+    const uint16_t* xr = xa + (lane & 15) * xs + 8 * ((lane >> 4) & 3);
+    uint32_t w[2][4][NWD];  // [buffer][tile: (t, j0), (t + 1, j0), (t, j1), (t + 1, j1)][word]
+    h8v a[2];
+    auto read = [&](int t, int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) tl.staged(st + (2 * (t + h) + j) * TW, w[b][2 * j + h]);
+        a[b] = *reinterpret_cast<const h8v*>(xr + t * 16);
+    };
+    read(0, 0);
+#pragma unroll
+    for (int t = 0; t < PK; t += 2) {
+        const int b = (t >> 1) & 1;
+        if (t + 2 < PK) read(t + 2, b ^ 1);
+        issued();
+        h8v bb[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            bb[j] = __builtin_bit_cast(h8v, tl.decode2(w[b][2 * j], w[b][2 * j + 1]));
+        }
+        acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b], bb[0], acc[0][0], 0, 0, 0);
+        acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[b], bb[1], acc[0][1], 0, 0, 0);
+    }
+}
+
+// The chunk loop of a gate|up block for one width: the activations one chunk ahead, the trellis two, two barriers a
+// chunk (the activations are shared by the block's waves). Loads complete in issue order and every load is issued (a
+// chunk past the last re-reads the last), so the waits stay exact.
+template <int CB, int K2, int MT>
+__device__ __forceinline__ void gu_loop(__amdgpu_buffer_rsrc_t xrs, const uint32_t (&aoff)[MT], const int (&lofs)[MT],
+                                        const TileSpan& sp, uint16_t* xa, uint32_t* st, int lane, int q8, int mts,
+                                        int c0, int nch, f4v (&acc)[MT][2]) {
+    constexpr int NL = stage_loads_k<PK, K2>();
+    const TileLane<K2, CB> tl(lane);
+    u4v av[MT], ta[NL], tb[NL];
+    auto issue_a = [&](int c) __attribute__((always_inline)) {
+        c = c0 + (c < nch ? c : nch - 1);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            av[i] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(xrs, aoff[i], c * PK * 32, 0));
+    };
+    auto issue_t = [&](int c, u4v (&tv)[NL]) __attribute__((always_inline)) {
+        c = c0 + (c < nch ? c : nch - 1);
+        TileSpan sc = sp;
+        sc.off = sp.off + c * PK * sp.kstride;
+        stage_issue_k<PK, K2>(sc, lane, tv);
+    };
+    auto step = [&](int c, u4v (&tv)[NL]) __attribute__((always_inline)) {
+        __syncthreads();  // the previous chunk's reads of xa are done
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            if (i < mts) put_a(xa + lofs[i], q8, av[i]);
+        stage_store_k<PK, K2>(st, lane, tv);  // only this wave reads its region, in order
+        issue_a(c + 1);
+        issue_t(c + 2, tv);
+        __syncthreads();  // the chunk's activations are in LDS
+        item_chunk<CB, K2, MT>(st, tl, xa, mts, lane, acc, PXS);
+    };
+    issue_t(0, ta);
+    issue_t(1, tb);
+    issue_a(0);
+    // two steps an iteration with no exit between them, so every load's wait is counted the same on each pass
+    int c = 0;
+    for (; c + 1 < nch; c += 2) {
+        step(c, ta);
+        step(c + 1, tb);
+    }
+    if (c < nch) step(c, ta);  // uniform
+}
+
+// Block b of a launch over (items, C column blocks, Z slices) in XCD order. Blocks are dispatched to the 8 XCDs in
+// turn (block b on XCD b mod 8); group g = item Z + slice takes blocks on XCD g mod 8 for all C of its column blocks
+// (the item's activations of the slice come into that XCD's L2 once), and slice z of an expert's consecutive items
+// lands on the XCDs (i Z + z) mod 8, 8 / gcd(Z, 8) of them (two for Z = 4 or 12), whose L2s then hold its trellis
+// for the expert's later items. 2048 rows: 719 -> 691 us a layer (item order: a slice's blocks on all 8 XCDs, each
+// fetching the slice). Blocks: ceil(items Z / 8) 8 C, those past the list's count return at once.
+__device__ __forceinline__ void xcd_order(int b, int C, int Z, int& item, int& cb, int& z) {
+    const int q = b >> 3;
+    cb = q % C;
+    const int g = (q / C) * 8 + (b & 7);
+    item = g / Z;
+    z = g % Z;
+}
+static unsigned xcd_blocks(int items, int C, int Z) { return (unsigned)((items * Z + 7) / 8 * 8 * C); }
+
+// Block (item of the larger items' list, 128 columns, (matrix, K split)), in XCD order: the item's rows (up to
+// IPM_TILES row tiles) times its expert's matrix over split s of K's chunks of 128 (splits [s nch / nsplit,
+// (s + 1) nch / nsplit)).
+// A chunk's activations go to LDS once for the block's four waves; each wave's two column tiles of the chunk come in
+// as 16-byte loads staged in the wave's own LDS region. Only the item's occupied row tiles are loaded and multiplied;
+// rows past the item's count read the item's first pair and are not stored (MFMA rows do not mix). Split 0 goes to
+// Z[mat][pair][n], split s > 0 to Zp[s - 1][mat][pair][n] (fp32), each accumulated from zero (stored as 0 + sum).
+template <int CB, int MK>
+__global__ void __launch_bounds__(PW * 64) __attribute__((amdgpu_waves_per_eu(2)))
+item_gu_kernel(const uint16_t* __restrict__ X0, const uint16_t* __restrict__ X1, const int64_t* __restrict__ TP0,
+               const int64_t* __restrict__ TP1, const int* __restrict__ K2_0, const int* __restrict__ K2_1,
+               const int* __restrict__ sorted, const int* __restrict__ items, const int* __restrict__ item_count,
+               float* __restrict__ Z, float* __restrict__ Zp, int K, int N, int P, int nsplit, int mats, int max_items,
+               int* __restrict__ status) {
+    constexpr int MT = IPM_TILES;
+    int e, first, cnt;
+    int item, cb, zs;
+    xcd_order((int)blockIdx.x, N / (16 * 2 * PW), mats * nsplit, item, cb, zs);
+    if (!item_at(items, item_count, 1, max_items, item, e, first, cnt)) return;
+    const int mat = zs / nsplit, split = zs % nsplit;
+    const uint16_t* X = mat ? X1 : X0;
+    const uint32_t* T = reinterpret_cast<const uint32_t*>(mat ? TP1[e] : TP0[e]);
+    const int k2 = mat ? K2_1[e] : K2_0[e];
+    // the wave index in a scalar register: the trellis offsets built from it are then scalar (a buffer load's soffset)
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    __shared__ int pair_sh[MT * 16];
+    __shared__ __attribute__((aligned(16))) uint16_t xa[MT * 16 * PXS];
+    __shared__ __attribute__((aligned(16))) uint32_t st[PW][pstage(MK)];
+    if (tid < MT * 16) pair_sh[tid] = tid < cnt ? sorted[first + tid] : -1;
+    __syncthreads();
+    // this thread's activation pieces of every chunk: piece i is row 16 i + (tid >> 4), halves 8 (tid & 15) .. +7;
+    // a piece past the item's row tiles reads row tile 0's address (a cache hit) and is not stored
+    const int mts = (cnt + 15) >> 4;
+    uint32_t aoff[MT];
+    int lofs[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int row = i * 16 + (tid >> 4);
+        const int rr = i < mts ? row : (tid >> 4);
+        const int p = pair_sh[rr] >= 0 ? pair_sh[rr] : pair_sh[0];
+        aoff[i] = ((uint32_t)p * (uint32_t)K + 8u * (tid & 15)) * 2u;
+        lofs[i] = row * PXS;
+    }
+    const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(X, (uint32_t)((size_t)P * K * 2));
+    const int nt0 = cb * (2 * PW) + 2 * wave;
+    const int ns = N >> 4, TWB = 16 * k2;
+    TileSpan sp;
+    sp.r = buffer_rsrc(T, (uint32_t)((K >> 4) * ns * TWB));
+    sp.off = nt0 * TWB;
+    sp.kstride = ns * TWB;
+    f4v acc[MT][2];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = f4v{0.f, 0.f, 0.f, 0.f};
+    const int nch = K / (PK * 16);
+    const int c0 = split * nch / nsplit, nc = (split + 1) * nch / nsplit - c0;  // nsplit <= nch: nc >= 1
+    const bool ok = EA_K2_SWITCH(
+        k2, 2, MK, (gu_loop<CB, K2V, MT>(xrs, aoff, lofs, sp, xa, st[wave], lane, tid & 15, mts, c0, nc, acc)));
+    if (!ok) {
+        if (lane == 0) record_error(status, DEV_UNSUPPORTED_WIDTH);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = nan4();
+    }
+    float* Zm = (split ? Zp + (size_t)(split - 1) * 2 * P * N : Z) + (size_t)mat * P * N;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int p = pair_sh[mt * 16 + 4 * (lane >> 4) + i];
+            if (p < 0) continue;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) Zm[(size_t)p * N + (nt0 + j) * 16 + (lane & 15)] = 0.f + acc[mt][j][i];
+        }
+}
+
+// Items of at most 16 pairs: a block is NW waves, one a column-tile pair of one matrix, over all of K. The block's
+// waves share each chunk of activations through a ring of RING_S chunk slots in LDS, filled and freed with LDS
+// counters instead of barriers, so a wave can run up to RING_S - RING_L - 1 chunks ahead of the slowest:
+//   filled[s]: pieces stored into slot s, over all the chunks it has held (NW a chunk);
+//   done[s]:   waves that have finished a chunk of slot s, over all its chunks (NW a chunk).
+// At its step c a wave stores its piece of chunk p = c + RING_L into slot p % RING_S once every wave is done with
+// that slot's previous chunk (done >= NW (p / RING_S)), waits until chunk c is complete in its slot
+// (filled >= NW (c / RING_S + 1)), computes it, and counts itself done. The slowest wave can always go on (every
+// chunk it waits for was stored at a step no later than its own, and every slot it stores into was freed before),
+// so every wait ends. Each wave's trellis goes through its own LDS region as in gu_loop; the activation piece of a
+// chunk (1/NW of it) and the trellis are loaded two chunks ahead. K is split as the larger items' is, over the same
+// chunk ranges and into the same planes, so a pair's sums do not depend on which list its item is in. (Decode windows
+// are bound by the waves there are, not by their work: 37 rows touch about 112 experts, and one block an (item, 128
+// columns, matrix) over all of K left 1.75 blocks a CU: 118 us, against 67 with the
+// two splits. Prompts of 512 and 2048 rows measured the same either way.)
+constexpr int RING_S = 6;  // activation chunk slots
+constexpr int RING_L = 2;  // a wave stores its piece of chunk c + RING_L at its step c
+
+template <int NW>
+struct RingPiece {  // a lane's words of a chunk: 16 rows x 64 words over NW waves
+    static constexpr int WORDS = 16 * 64 / (NW * 64);
+};
+
+__device__ __forceinline__ int lds_load_acquire(const int* p) {
+    return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// One count for the whole wave: only its first lane adds (the wait before the add covers every lane's accesses).
+__device__ __forceinline__ void lds_add_release(int* p, int v, int lane) {
+    if (lane == 0) __hip_atomic_fetch_add(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// Wait until *p >= target. Every count waited for is reached (see above); the wait is still bounded (about 2^20
+// sleeps, tens of milliseconds): past the bound it gives up, returns false and the kernel reports EA_SYNC_TIMEOUT.
+__device__ __forceinline__ bool lds_wait_geq(const int* p, int target) {
+    for (int n = 0; lds_load_acquire(p) < target; ++n) {
+        if (n >= (1 << 20)) return false;
+        __builtin_amdgcn_s_sleep(1);
+    }
+    return true;
+}
+
+template <int CB, int K2, int NW>
+__device__ __forceinline__ void ring_loop(__amdgpu_buffer_rsrc_t xrs, uint32_t aoff, int lofs, const TileSpan& sp,
+                                          uint16_t* ring, int* filled, int* done, uint32_t* st, int lane, int c0,
+                                          int nch, f4v (&acc)[1][2], bool& synced) {
+    constexpr int NL = stage_loads_k<PK, K2>();
+    constexpr int W = RingPiece<NW>::WORDS;  // 2 or 4
+    constexpr int SLOT = 16 * PXS;
+    using pv = uint32_t __attribute__((ext_vector_type(W)));
+    const TileLane<K2, CB> tl(lane);
+    pv pa, pb;
+    u4v ta[NL], tb[NL];
+    auto issue_p = [&](int c, pv& v) __attribute__((always_inline)) {
+        c = c0 + (c < nch ? c : nch - 1);
+        if constexpr (W == 4)
+            v = __builtin_bit_cast(pv, __builtin_amdgcn_raw_buffer_load_b128(xrs, aoff, c * PK * 32, 0));
+        else
+            v = __builtin_bit_cast(pv, __builtin_amdgcn_raw_buffer_load_b64(xrs, aoff, c * PK * 32, 0));
+    };
+    auto issue_t = [&](int c, u4v (&tv)[NL]) __attribute__((always_inline)) {
+        c = c0 + (c < nch ? c : nch - 1);
+        TileSpan sc = sp;
+        sc.off = sp.off + c * PK * sp.kstride;
+        stage_issue_k<PK, K2>(sc, lane, tv);
+    };
+    // the piece's words d .. d + W - 1 of its row (d = lofs & 63) at their transposed places (see put_a)
+    auto put = [&](int p, const pv& v) __attribute__((always_inline)) {
+        const int sl = p % RING_S;
+        synced = synced && lds_wait_geq(&done[sl], NW * (p / RING_S));  // after a give-up no more waits
+        uint32_t* w = reinterpret_cast<uint32_t*>(ring + sl * SLOT + (lofs >> 6) * PXS);
+        const int d = lofs & 63;
+#pragma unroll
+        for (int r = 0; r < W; ++r) {
+            const int dd = (d & 15) + r;  // word within its 32-k step
+            w[16 * (d >> 4) + 4 * (dd & 3) + (dd >> 2)] = v[r];
+        }
+        lds_add_release(&filled[sl], 1, lane);
+    };
+    auto step = [&](int c, u4v (&tv)[NL], pv& v) __attribute__((always_inline)) {
+        if (c + RING_L < nch) put(c + RING_L, v);  // uniform
+        issue_p(c + RING_L + 2, v);
+        stage_store_k<PK, K2>(st, lane, tv);
+        issue_t(c + 2, tv);
+        const int sl = c % RING_S;
+        synced = synced && lds_wait_geq(&filled[sl], NW * (c / RING_S + 1));
+        item_chunk1<CB, K2>(st, tl, ring + sl * SLOT, lane, acc, PXS);
+        lds_add_release(&done[sl], 1, lane);  // after the chunk's reads of the slot have returned
+    };
+    // chunks 0 .. RING_L - 1 go in before the loop; pa / pb then carry chunks RING_L and RING_L + 1
+    for (int p = 0; p < RING_L && p < nch; ++p) {
+        pv v;
+        issue_p(p, v);
+        put(p, v);
+    }
+    issue_p(RING_L, pa);
+    issue_t(0, ta);
+    issue_p(RING_L + 1, pb);
+    issue_t(1, tb);
+    int c = 0;
+    for (; c + 1 < nch; c += 2) {  // two steps an iteration with no exit between them
+        step(c, ta, pa);
+        step(c + 1, tb, pb);
+    }
+    if (c < nch) step(c, ta, pa);  // uniform
+}
+
+template <int CB, int MK, int NW>
+__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(4)))
+item_ring_kernel(const uint16_t* __restrict__ X0, const uint16_t* __restrict__ X1, const int64_t* __restrict__ TP0,
+                 const int64_t* __restrict__ TP1, const int* __restrict__ K2_0, const int* __restrict__ K2_1,
+                 const int* __restrict__ sorted, const int* __restrict__ items, const int* __restrict__ item_count,
+                 float* __restrict__ Z, float* __restrict__ Zp, int K, int N, int P, int nsplit, int max_items,
+                 int* __restrict__ status) {
+    int e, first, cnt;
+    if (!item_at(items, item_count, 0, max_items, blockIdx.x, e, first, cnt)) return;
+    const int mat = blockIdx.z / nsplit, split = blockIdx.z % nsplit;
+    const uint16_t* X = mat ? X1 : X0;
+    const uint32_t* T = reinterpret_cast<const uint32_t*>(mat ? TP1[e] : TP0[e]);
+    const int k2 = mat ? K2_1[e] : K2_0[e];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    __shared__ int pair_sh[16];
+    __shared__ int filled[RING_S], done[RING_S];
+    __shared__ __attribute__((aligned(16))) uint16_t ring[RING_S * 16 * PXS];
+    __shared__ __attribute__((aligned(16))) uint32_t st[NW][pstage(MK)];
+    if (threadIdx.x < 16) pair_sh[threadIdx.x] = (int)threadIdx.x < cnt ? sorted[first + threadIdx.x] : -1;
+    if (threadIdx.x < RING_S) filled[threadIdx.x] = done[threadIdx.x] = 0;
+    __syncthreads();
+    // this lane's piece of every chunk: words [d, d + W) of row r (word index lofs = 64 r + d over the chunk);
+    // a row past the count reads the first pair's row
+    constexpr int W = RingPiece<NW>::WORDS;
+    const int lofs = (wave * 64 + lane) * W;
+    const int row = lofs >> 6;
+    const int p = pair_sh[row] >= 0 ? pair_sh[row] : pair_sh[0];
+    const uint32_t aoff = ((uint32_t)p * (uint32_t)K + 2u * (uint32_t)(lofs & 63)) * 2u;
+    const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(X, (uint32_t)((size_t)P * K * 2));
+    const int nt0 = blockIdx.y * (2 * NW) + 2 * wave;
+    const int ns = N >> 4, TWB = 16 * k2;
+    TileSpan sp;
+    sp.r = buffer_rsrc(T, (uint32_t)((K >> 4) * ns * TWB));
+    sp.off = nt0 * TWB;
+    sp.kstride = ns * TWB;
+    f4v acc[1][2];
+    acc[0][0] = acc[0][1] = f4v{0.f, 0.f, 0.f, 0.f};
+    const int nch = K / (PK * 16);
+    const int c0 = split * nch / nsplit, nc = (split + 1) * nch / nsplit - c0;  // nsplit <= nch: nc >= 1
+    bool synced = true;
+    const bool ok = EA_K2_SWITCH(k2, 2, MK,
+                                 (ring_loop<CB, K2V, NW>(xrs, aoff, lofs, sp, ring, filled, done, st[wave], lane, c0,
+                                                         nc, acc, synced)));
+    if (!ok || !synced) {
+        if (lane == 0) record_error(status, ok ? DEV_SYNC_TIMEOUT : DEV_UNSUPPORTED_WIDTH);
+        acc[0][0] = acc[0][1] = nan4();
+    }
+    float* Zm = (split ? Zp + (size_t)(split - 1) * 2 * P * N : Z) + (size_t)mat * P * N;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int pp = pair_sh[4 * (lane >> 4) + i];
+        if (pp < 0) continue;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) Zm[(size_t)pp * N + (nt0 + j) * 16 + (lane & 15)] = 0.f + acc[0][j][i];
+    }
+}
+
+// The column blocks of a down block for one width: step s is column block s / nch, chunk s % nch; the trellis two
+// steps ahead; each column block's rows are stored when its last chunk is done.
+template <int CB, int K2, int MT, int NG>
+__device__ __forceinline__ void dn_loop(const TileSpan& sp, const uint16_t* xa, uint32_t* st, int lane, int wave,
+                                        int mts, int nch, int nb0, const int* pair_sh, const PairPlane& plane) {
+    constexpr int NL = stage_loads_k<PK, K2>();
+    constexpr int TWB = 16 * K2;
+    const TileLane<K2, CB> tl(lane);
+    const int steps = NG * nch;  // even (NG even, or nch = 2: the caller's choice): two steps an iteration
+    u4v ta[NL], tb[NL];
+    f4v acc[MT][2];
+    auto issue_t = [&](int s2, u4v (&tv)[NL]) __attribute__((always_inline)) {
+        s2 = s2 < steps ? s2 : steps - 1;
+        TileSpan sc = sp;
+        sc.off = sp.off + (s2 / nch) * 8 * TWB + (s2 % nch) * PK * sp.kstride;
+        stage_issue_k<PK, K2>(sc, lane, tv);
+    };
+    auto step = [&](int s2, u4v (&tv)[NL]) __attribute__((always_inline)) {
+        const int c = s2 % nch;
+        if (c == 0) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[mt][0] = acc[mt][1] = f4v{0.f, 0.f, 0.f, 0.f};
+        }
+        stage_store_k<PK, K2>(st, lane, tv);  // only this wave reads its region, in order
+        issue_t(s2 + 2, tv);
+        item_chunk<CB, K2, MT>(st, tl, xa + c * PK * 16, mts, lane, acc, DXS);
+        if (c == nch - 1) {
+            const int nt0 = (nb0 + s2 / nch) * 8 + 2 * wave;
+            float* Z = plane.base(nt0 * 16);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int p = pair_sh[mt * 16 + 4 * (lane >> 4) + i];
+                    if (p < 0) continue;
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        Z[(size_t)p * plane.stride + (nt0 + j) * 16 + (lane & 15)] = acc[mt][j][i];
+                }
+        }
+    };
+    issue_t(0, ta);
+    issue_t(1, tb);
+    for (int s2 = 0; s2 < steps; s2 += 2) {  // steps = NG nch is even: two steps an iteration, no exit between
+        step(s2, ta);
+        step(s2 + 1, tb);
+    }
+}
+
+// The down matrix (K = I of 128 or 256: one or two chunks): a block (item of list MT > 2, NG column blocks of 128)
+// loads the item's activations for all of K into LDS once, then its waves run the column blocks independently. WB = 8
+// (the larger items): two groups of four waves, each over NG / 2 of the column blocks, share one copy
+// of the activations, so two blocks fit a CU's LDS at four waves a SIMD (four-wave blocks: three at three).
+template <int CB, int MK, int MT, int NG, int WB = PW>
+__global__ void __launch_bounds__(WB * 64) __attribute__((amdgpu_waves_per_eu(MT > 2 && WB == PW ? 2 : 4)))
+item_dn_kernel(const uint16_t* __restrict__ X, const int64_t* __restrict__ TP, const int* __restrict__ K2T,
+               const int* __restrict__ sorted, const int* __restrict__ items, const int* __restrict__ item_count,
+               PairPlane plane, int K, int N, int P, int max_items, int* __restrict__ status) {
+    int e, first, cnt;
+    // the larger items' blocks in XCD order (a column group's slice of an expert on the same XCDs for all of the
+    // expert's items); the small items' (one item an expert) item by item
+    int item = blockIdx.x, grp = blockIdx.y;
+    if constexpr (MT > 2) {
+        int cb_unused;
+        xcd_order((int)blockIdx.x, 1, N / 128 / NG, item, cb_unused, grp);
+    }
+    if (!item_at(items, item_count, MT > 2, max_items, item, e, first, cnt)) return;
+    const uint32_t* T = reinterpret_cast<const uint32_t*>(TP[e]);
+    const int k2 = K2T[e];
+    // the wave index in a scalar register: the trellis offsets built from it are then scalar (a buffer load's soffset)
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    __shared__ int pair_sh[MT * 16];
+    __shared__ __attribute__((aligned(16))) uint16_t xa[MT * 16 * DXS];
+    static_assert(WB == PW || (WB == 2 * PW && NG % 2 == 0), "two wave groups: half the column blocks each");
+    __shared__ __attribute__((aligned(16))) uint32_t st[WB][pstage(MK)];
+    if (tid < MT * 16) pair_sh[tid] = tid < cnt ? sorted[first + tid] : -1;
+    __syncthreads();
+    const int mts = (cnt + 15) >> 4;
+    const int nch = K / (PK * 16);  // 1 or 2
+    {
+        // 256 threads cover a chunk of a row tile; with eight waves each half of the block loads one chunk
+        constexpr int CPT = WB == PW ? 2 : 1;  // chunks a thread loads
+        const int lt = tid & 255, c0 = WB == PW ? 0 : tid >> 8;
+        const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(X, (uint32_t)((size_t)P * K * 2));
+        u4v av[CPT][MT];
+#pragma unroll
+        for (int q = 0; q < CPT; ++q)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                const int rr = i < mts ? i * 16 + (lt >> 4) : (lt >> 4);
+                const int p = pair_sh[rr] >= 0 ? pair_sh[rr] : pair_sh[0];
+                const int cc = c0 + q < nch ? c0 + q : 0;
+                av[q][i] = __builtin_bit_cast(
+                    u4v, __builtin_amdgcn_raw_buffer_load_b128(
+                             xrs, ((uint32_t)p * (uint32_t)K + (uint32_t)(cc * PK * 16 + 8 * (lt & 15))) * 2u, 0, 0));
+            }
+#pragma unroll
+        for (int q = 0; q < CPT; ++q)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                if (c0 + q < nch && i < mts)
+                    put_a(xa + (i * 16 + (lt >> 4)) * DXS + (c0 + q) * PK * 16, lt & 15, av[q][i]);
+    }
+    constexpr int NGW = WB == PW ? NG : NG / 2;  // column blocks a wave group runs
+    const int ns = N >> 4, TWB = 16 * k2;
+    const int w4 = wave & (PW - 1);
+    const int nb0 = grp * NG + (wave / PW) * NGW;  // the wave group's first column block
+    TileSpan sp;
+    sp.r = buffer_rsrc(T, (uint32_t)((K >> 4) * ns * TWB));
+    sp.off = (nb0 * 8 + 2 * w4) * TWB;
+    sp.kstride = ns * TWB;
+    __syncthreads();  // the activations are in LDS
+    const bool ok = EA_K2_SWITCH(
+        k2, 2, MK, (dn_loop<CB, K2V, MT, NGW>(sp, xa, st[wave], lane, w4, mts, nch, nb0, pair_sh, plane)));
+    if (!ok) {  // no product ran: the item's outputs of the block's column blocks are NaN
+        if (lane == 0) record_error(status, DEV_UNSUPPORTED_WIDTH);
+        for (int g = 0; g < NGW; ++g)
+            for (int i = 0; i < MT * 16; ++i) {
+                const int p = pair_sh[i];
+                if (p < 0) continue;
+                const int o = (nb0 + g) * 128 + w4 * 32 + (lane & 31);
+                plane.base(o)[(size_t)p * plane.stride + o] = __builtin_nanf("");
+            }
+    }
+}
+
+// What one item list's pass reads and writes: the rotated activations, the three matrices' trellis tables and
+// widths, the items, the pair classes and the per-pair planes (z and zp: gate|up partial sums, xd: down inputs,
+// plane: down outputs). The two lists' pairs are disjoint, so their passes touch disjoint rows of every plane.
+struct ListPass {
+    const uint16_t *xg, *xu;
+    const int64_t* tp[3];
+    const int* k2[3];
+    const int *sorted, *items, *count, *pclass, *pick;
+    const uint16_t *svh_g, *svh_u, *suh_d;
+    float *z, *zp;
+    PairPlane plane;
+    uint16_t* xd;
+    int D, I, P, rows, slots, E, mi;
+    int* status;
+};
+
+// One item list from its gate|up product to its down product, in order on q: big = 1 takes the larger items (the
+// gate|up K split into zp; the down matrix by blocks of DNG_BIG column blocks), big = 0 the items of at most
+// SMALL_ROWS pairs (the ring kernel; DNG column blocks). The down matrix takes the resident-activation kernel when
+// its K and N fit, the chunked ones otherwise. The two lists run on two streams: the small items' blocks leave room
+// on many CUs, the larger items' blocks are few and long, and each list's down product starts when its own
+// epilogue is done.
+template <int CB, int MK>
+static int list_pass(hipStream_t q, const ListPass& a, int big) {
+    const int ns = gu_splits(a.D);
+    if (big)
+        item_gu_kernel<CB, MK><<<xcd_blocks(a.mi, a.I / (16 * 2 * PW), 2 * ns), PW * 64, 0, q>>>(
+            a.xg, a.xu, a.tp[0], a.tp[1], a.k2[0], a.k2[1], a.sorted, a.items, a.count, a.z, a.zp, a.D, a.I, a.P, ns,
+            2, a.mi, a.status);
+    else  // blocks of 4 waves over 128 columns (8 waves over 256 measured 1 % slower at 512 rows, the same at 2048)
+        item_ring_kernel<CB, MK, 4><<<dim3(a.mi, a.I / 128, 2 * ns), 4 * 64, 0, q>>>(
+            a.xg, a.xu, a.tp[0], a.tp[1], a.k2[0], a.k2[1], a.sorted, a.items, a.count, a.z, a.zp, a.D, a.I, a.P, ns,
+            a.mi, a.status);
+    int r = launched();
+    if (r) return r;
+    r = launch_gateup_epilogue(q, a.z, a.pick, a.svh_g, a.svh_u, a.suh_d, a.xd, (uint32_t)a.rows, (uint32_t)a.P,
+                               (uint32_t)a.I, (uint32_t)ns, (uint32_t)a.slots, (uint32_t)a.E, __builtin_inff(), 1, a.zp, a.pclass,
+                               big);
+    if (r) return r;
+    const int nb = a.D / 128;
+    if (a.I <= 2 * PK * 16 && nb % 2 == 0) {
+#define EA_DN(MT_, NG_, WB_, grid)                                                                                    \
+    item_dn_kernel<CB, MK, MT_, NG_, WB_><<<grid, (WB_) * 64, 0, q>>>(a.xd, a.tp[2], a.k2[2], a.sorted, a.items, a.count,  \
+                                                                  a.plane, a.I, a.D, a.P, a.mi, a.status)
+        if (big && a.rows > LONG_ROWS && nb % DNG_BIG_LONG == 0)
+            EA_DN(IPM_TILES, DNG_BIG_LONG, 2 * PW, xcd_blocks(a.mi, 1, nb / DNG_BIG_LONG));
+        else if (big && a.I == 2 * PK * 16)  // two chunks of K: a wave group's one column block is an even step count
+            EA_DN(IPM_TILES, DNG_BIG, 2 * PW, xcd_blocks(a.mi, 1, nb / DNG_BIG));
+        else if (big)
+            EA_DN(IPM_TILES, DNG_BIG, PW, xcd_blocks(a.mi, 1, nb / DNG_BIG));
+        else if (a.rows <= WINDOW_ROWS_MAX && nb % DNG_WINDOW == 0)
+            EA_DN(SMALL_ROWS / 16, DNG_WINDOW, PW, dim3(a.mi, nb / DNG_WINDOW, 1));
+        else if (nb % DNG == 0)
+            EA_DN(SMALL_ROWS / 16, DNG, PW, dim3(a.mi, nb / DNG, 1));
+        else
+            EA_DN(SMALL_ROWS / 16, 2, PW, dim3(a.mi, nb / 2, 1));
+#undef EA_DN
+    } else if (big) {
+        item_gu_kernel<CB, MK><<<xcd_blocks(a.mi, a.D / (16 * 2 * PW), 1), PW * 64, 0, q>>>(
+            a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, nullptr, a.I, a.D,
+            a.P, 1, 1, a.mi, a.status);
+    } else {
+        item_ring_kernel<CB, MK, 4><<<dim3(a.mi, a.D / 128, 1), 4 * 64, 0, q>>>(
+            a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, nullptr, a.I, a.D, a.P,
+            1, a.mi, a.status);
+    }
+    return launched();
+}
+
+// The same for a layer with experts above width 10 (ea_prompt_wide.hip).
+int list_pass_wide(hipStream_t q, const ListPass& a, int big, uint32_t cb);
+
+}  // namespace ea

@@ -273,6 +273,25 @@ def test_prompt_experts_narrow_widths_resident_down(ea, k2, R, E, planes):
     assert device.device_status() == 0
 
 
+@pytest.mark.parametrize("k2,cb,R,E,I", [(13, 1, 20, 64, 256), (15, 2, 100, 24, 256), (16, 0, 100, 24, 128), (11, 0, 300, 24, 256)])
+def test_prompt_experts_wide_widths_resident_down(ea, k2, cb, R, E, I):
+    """Widths above 10 (three trellis words a lane) through both item lists and the resident-activation down kernel,
+    every codebook; both plane modes give the same bits."""
+    device, _, _, pe, synth = ea
+    D = 2048
+    host, ex, sc, x, pick, wts, dx, dp, dw = _prompt_case(ea, R, E, D, I, k2, 970 + k2, zipf=False, cb=cb)
+    want = orc.prompt_experts(x, pick, wts, oracle_routed(host), R, 8, bf16=True)
+    got = []
+    for planes in (True, False):
+        out = device.zeros((R, D), torch.float32)
+        pe.run(device.stream(), dx.data_ptr(), D, dp.data_ptr(), dw.data_ptr(), ex, pe.Scratch(ex, R, 8, planes=planes),
+               out.data_ptr(), R, do_round=False)
+        got.append(device.download(out))
+        assert_close_rms(got[-1], want, 2e-3, f"wide widths, K2 {k2}, planes={planes}")
+    np.testing.assert_array_equal(got[0], got[1])
+    assert device.device_status() == 0
+
+
 @pytest.mark.parametrize("planes", [True, False])
 def test_prompt_experts_f32_activations(ea, planes):
     """fp32 activations (x_dtype 2: the rotation launch reads them and rounds the rotated rows to fp16 as for 16-bit
