@@ -209,9 +209,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, 
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
 
-// Dispatch a runtime K2 to wave_tiles<..., K2, ...> for K2 in [LO, HI]; false when outside.
+// Dispatch a runtime K2 to wave_tiles<..., K2, ...> for K2 in [LO, HI]; false when outside. Always inlined: as a called
+// function it holds its captures in scratch memory and wave-uniform values in vector registers.
 #define EA_K2_SWITCH(k2, LO, HI, CALL)                                        \
-    [&]() -> bool {                                                           \
+    [&]() __attribute__((always_inline)) -> bool {                            \
         switch (k2) {                                                         \
             EA_K2_CASE(2, LO, HI, CALL) EA_K2_CASE(3, LO, HI, CALL)           \
             EA_K2_CASE(4, LO, HI, CALL) EA_K2_CASE(5, LO, HI, CALL)           \

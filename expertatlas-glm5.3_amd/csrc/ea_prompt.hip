@@ -388,15 +388,29 @@ int ea_prompt_experts_run(ea_stream_t stream, const void* x, int x_dtype, uint32
                                                                   dptr<int>(sc->pclass), (int)max_items, IPM);
         int r = launched();
         if (r) return r;
-        r = launch_rot_in(s, xs, x_dtype, xstride, pk, dptr<const uint16_t>(ex->suh_g), dptr<const uint16_t>(ex->suh_u),
-                          dptr<uint16_t>(sc->xg), dptr<uint16_t>(sc->xu), n, D, S, E);
-        if (r) return r;
+        const uint16_t *suh_g = dptr<const uint16_t>(ex->suh_g), *suh_u = dptr<const uint16_t>(ex->suh_u);
+        // Long passes rotate inside the larger items' products (rotate_fits says when they can): 2048 rows 666 -> 601 us,
+        // bound by memory; 1024 rows 423 with the launch and 419 without it, 512 rows 306 and 335 (few blocks, each with the
+        // rotation on its chain). Widths above 10 keep the rotation launch: their kernel with the rotation inside came
+        // out of the compiler with the width switch as a called function, and hung in a test.
+        const bool fuse = !wide && n > (uint32_t)LONG_ROWS && rotate_fits(xs, x_dtype, xstride, suh_g, suh_u, n, I);
+        if (!fuse) {
+            r = launch_rot_in(s, xs, x_dtype, xstride, pk, suh_g, suh_u, dptr<uint16_t>(sc->xg), dptr<uint16_t>(sc->xu), n,
+                              D, S, E);
+            if (r) return r;
+        }
         const int dh = (int)(D / 2);
         const PairPlane plane = split ? PairPlane{dptr<float>(sc->xg), dptr<float>(sc->xu) - dh, dh, dh}
                                       : PairPlane{dptr<float>(sc->plane), dptr<float>(sc->plane), dh, (int)D};
         ListPass a{};
-        a.xg = dptr<const uint16_t>(sc->xg);
-        a.xu = dptr<const uint16_t>(sc->xu);
+        a.x = xs;
+        a.x_dtype = x_dtype;
+        a.x_stride = (int)xstride;
+        a.fuse = fuse;
+        a.suh_g = suh_g;
+        a.suh_u = suh_u;
+        a.xg = dptr<uint16_t>(sc->xg);
+        a.xu = dptr<uint16_t>(sc->xu);
         for (int m = 0; m < 3; ++m) {
             a.tp[m] = dptr<const int64_t>(ex->ptr[m]);
             a.k2[m] = dptr<const int>(ex->k2[m]);

@@ -61,6 +61,10 @@ constexpr int WINDOW_ROWS_MAX = 128;  // the widest decode window (forward.zig:2
 constexpr int DNG_BIG = 2;  // the same for the larger items: more blocks for fewer items (4: 1 % slower at 512 rows)
 constexpr int DNG_BIG_LONG = 4;   // passes of more than LONG_ROWS rows: 1.5 % faster at 2048 rows
 constexpr int LONG_ROWS = 1024;
+// Rows a pass up to which the larger items' gate|up stages its activations in two buffers (two blocks a CU), above which in
+// one (four). 300 rows 254 us with two and 282 with one, 512 rows 306 and 315, 640 rows 351 and 347, 1024 rows 447 and 423:
+// few blocks wait on each chunk's round trip, many on each other for a place.
+constexpr int MID_ROWS = 600;
 constexpr int GU_SPLIT = 2;                       // K splits of a larger item's gate|up (4 and 8 measured slower)
 // The number of K splits of a larger item's gate|up over K (at most one a chunk).
 static int gu_splits(int K) { return K / (PK * 16) < GU_SPLIT ? K / (PK * 16) : GU_SPLIT; }
@@ -140,21 +144,69 @@ __device__ __forceinline__ void item_chunk1(const uint32_t* st, const TileLane<K
     }
 }
 
-// The chunk loop of a gate|up block for one width: the activations one chunk ahead, the trellis two, two barriers a
-// chunk (the activations are shared by the block's waves). Loads complete in issue order and every load is issued (a
-// chunk past the last re-reads the last), so the waits stay exact.
+// The same with the LDS reads ahead: the next k step's trellis words are read before this step decodes, and a row tile's
+// activations before the products of the one before. Costs registers that the rotating kernel does not have.
 template <int CB, int K2, int MT>
-__device__ __forceinline__ void gu_loop(__amdgpu_buffer_rsrc_t xrs, const uint32_t (&aoff)[MT], const int (&lofs)[MT],
-                                        const TileSpan& sp, uint16_t* xa, uint32_t* st, int lane, int q8, int mts,
+__device__ __forceinline__ void item_chunk_ahead(const uint32_t* st, const TileLane<K2, CB>& tl, const uint16_t* xa,
+                                                 int mts, int lane, f4v (&acc)[MT][2]) {
+    constexpr int TW = 4 * K2, NWD = TileLane<K2, CB>::NW;
+    const uint16_t* xr = xa + (lane & 15) * PXS + 8 * ((lane >> 4) & 3);
+    uint32_t w[2][2][2][NWD];  // [buffer][column tile][k tile][word]
+    auto read = [&](int t, int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) tl.staged(st + (2 * (t + h) + j) * TW, w[b][j][h]);
+    };
+    read(0, 0);
+#pragma unroll
+    for (int t = 0; t < PK; t += 2) {
+        const int b = (t >> 1) & 1;
+        h8v a = *reinterpret_cast<const h8v*>(xr + t * 16);
+        if (t + 2 < PK) read(t + 2, b ^ 1);
+        issued();
+        h8v bb[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) bb[j] = __builtin_bit_cast(h8v, tl.decode2(w[b][j][0], w[b][j][1]));
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            if (mt >= mts) break;  // the item's occupied row tiles only (uniform)
+            const h8v an = *reinterpret_cast<const h8v*>(xr + (mt + 1 < MT ? mt + 1 : mt) * 16 * PXS + t * 16);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bb[j], acc[mt][j], 0, 0, 0);
+            a = an;
+        }
+    }
+}
+
+// Where a gate|up block's activations come from: rotated already (fp16 [pairs, K], a buffer over them), or the raw rows
+// (16-bit, a buffer over them, with the expert's suh row) that the block rotates while staging them.
+struct GuSrc {
+    __amdgpu_buffer_rsrc_t x, suh;
+    int bf16;
+};
+
+// The chunk loop of a gate|up block for one width. With TWO activation buffers they are staged for the block's waves a
+// chunk ahead: a step stores (ROT: rotates and stores) the next chunk's and issues the loads of the one after, computes
+// its own, and meets the other waves once. With one, two barriers a chunk (MID_ROWS says which; above width 10, whose
+// staging regions are larger, always one: 777 rows 428 us, with two 437). The trellis is loaded two chunks ahead into the wave's own region. Loads
+// complete in issue order and every load is issued (a chunk past the last re-reads the last), so the waits stay exact.
+// Thread tid's piece i of a chunk is row (i NT + tid) / 16; aoff: its byte offset in the source.
+template <int CB, int K2, int MT, int NT, bool ROT, bool TWO>
+__device__ __forceinline__ void gu_loop(const GuSrc& src, const uint32_t (&aoff)[(MT * 256 + NT - 1) / NT],
+                                        const TileSpan& sp, uint16_t* xa, uint32_t* st, int lane, int rows, int mts,
                                         int c0, int nch, f4v (&acc)[MT][2]) {
-    constexpr int NL = stage_loads_k<PK, K2>();
+        constexpr int NL = stage_loads_k<PK, K2>(), NP = (MT * 256 + NT - 1) / NT, BUF = MT * 16 * PXS;
     const TileLane<K2, CB> tl(lane);
-    u4v av[MT], ta[NL], tb[NL];
+    const int row0 = (int)threadIdx.x >> 4, q8 = ROT ? h8_group(lane) : lane & 15;
+    u4v av[NP], sv = u4v{0u, 0u, 0u, 0u}, ta[NL], tb[NL];
     auto issue_a = [&](int c) __attribute__((always_inline)) {
         c = c0 + (c < nch ? c : nch - 1);
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
-            av[i] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(xrs, aoff[i], c * PK * 32, 0));
+        for (int i = 0; i < NP; ++i)
+            av[i] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(src.x, aoff[i], c * PK * 32, 0));
+        if constexpr (ROT)
+            sv = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(src.suh, q8 * 16, c * PK * 32, 0));
     };
     auto issue_t = [&](int c, u4v (&tv)[NL]) __attribute__((always_inline)) {
         c = c0 + (c < nch ? c : nch - 1);
@@ -162,27 +214,65 @@ __device__ __forceinline__ void gu_loop(__amdgpu_buffer_rsrc_t xrs, const uint32
         sc.off = sp.off + c * PK * sp.kstride;
         stage_issue_k<PK, K2>(sc, lane, tv);
     };
-    auto step = [&](int c, u4v (&tv)[NL]) __attribute__((always_inline)) {
-        __syncthreads();  // the previous chunk's reads of xa are done
+    auto put = [&](uint16_t* buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
-            if (i < mts) put_a(xa + lofs[i], q8, av[i]);
-        stage_store_k<PK, K2>(st, lane, tv);  // only this wave reads its region, in order
-        issue_a(c + 1);
-        issue_t(c + 2, tv);
-        __syncthreads();  // the chunk's activations are in LDS
-        item_chunk<CB, K2, MT>(st, tl, xa, mts, lane, acc, PXS);
+        for (int i = 0; i < NP; ++i) {
+            const int row = i * (NT / 16) + row0;
+            if (row >= rows) continue;  // uniform over a wave (rows % 16 == 0)
+            u4v v = av[i];
+            if constexpr (ROT) {
+                float f[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const uint16_t h = (uint16_t)(v[j >> 1] >> (16 * (j & 1)));
+                    f[j] = (src.bf16 ? bf2f(h) : h2f(h)) * h2f((uint16_t)(sv[j >> 1] >> (16 * (j & 1))));
+                }
+                const float sc = fwht128_x8(f, lane) * HAD_SCALE;  // the values' sign folded into the scale (exact)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    v[j] = f2h2(__builtin_fmaf(f[2 * j], sc, 0.f), __builtin_fmaf(f[2 * j + 1], sc, 0.f));
+            }
+            put_a(buf + row * PXS, q8, v);
+        }
     };
-    issue_t(0, ta);
-    issue_t(1, tb);
-    issue_a(0);
+    auto step = [&](int c, u4v (&tv)[NL], int b) __attribute__((always_inline)) {
+        if constexpr (TWO) {
+            stage_store_k<PK, K2>(st, lane, tv);  // only this wave reads its region, in order
+            put(xa + (b ^ 1) * BUF);              // the chunk before the one in that buffer was read before the barrier
+            issue_t(c + 2, tv);
+            issue_a(c + 2);
+            if constexpr (ROT) item_chunk<CB, K2, MT>(st, tl, xa + b * BUF, mts, lane, acc, PXS);
+            else item_chunk_ahead<CB, K2, MT>(st, tl, xa + b * BUF, mts, lane, acc);
+            __syncthreads();
+        } else {
+            __syncthreads();  // the previous chunk's reads of xa are done
+            put(xa);
+            stage_store_k<PK, K2>(st, lane, tv);
+            issue_a(c + 1);
+            issue_t(c + 2, tv);
+            __syncthreads();
+            item_chunk_ahead<CB, K2, MT>(st, tl, xa, mts, lane, acc);
+        }
+    };
+    if constexpr (TWO) {
+        issue_a(0);
+        issue_t(0, ta);
+        put(xa);
+        issue_a(1);
+        issue_t(1, tb);
+        __syncthreads();
+    } else {
+        issue_t(0, ta);
+        issue_t(1, tb);
+        issue_a(0);
+    }
     // two steps an iteration with no exit between them, so every load's wait is counted the same on each pass
     int c = 0;
     for (; c + 1 < nch; c += 2) {
-        step(c, ta);
-        step(c + 1, tb);
+        step(c, ta, 0);
+        step(c + 1, tb, 1);
     }
-    if (c < nch) step(c, ta);  // uniform
+    if (c < nch) step(c, ta, 0);  // uniform
 }
 
 // Block b of a launch over (items, C column blocks, Z slices) in XCD order. Blocks are dispatched to the 8 XCDs in
@@ -200,51 +290,57 @@ __device__ __forceinline__ void xcd_order(int b, int C, int Z, int& item, int& c
 }
 static unsigned xcd_blocks(int items, int C, int Z) { return (unsigned)((items * Z + 7) / 8 * 8 * C); }
 
-// Block (item of the larger items' list, 128 columns, (matrix, K split)), in XCD order: the item's rows (up to
-// IPM_TILES row tiles) times its expert's matrix over split s of K's chunks of 128 (splits [s nch / nsplit,
-// (s + 1) nch / nsplit)).
-// A chunk's activations go to LDS once for the block's four waves; each wave's two column tiles of the chunk come in
-// as 16-byte loads staged in the wave's own LDS region. Only the item's occupied row tiles are loaded and multiplied;
-// rows past the item's count read the item's first pair and are not stored (MFMA rows do not mix). Split 0 goes to
+// Block (item of the larger items' list, 32 WB columns, (matrix, K split)), in XCD order: the item's rows (up to IPM_TILES
+// row tiles) times its expert's matrix over split s of K's chunks of 128 (splits [s nch / nsplit, (s + 1) nch / nsplit)).
+// A chunk's activations go to LDS once for the block's WB waves; each wave's two column tiles of the chunk come in as
+// 16-byte loads staged in the wave's own LDS region. Only the item's occupied row tiles are staged and multiplied; rows
+// past the item's count repeat the item's first pair and are not stored (MFMA rows do not mix). Split 0 goes to
 // Z[mat][pair][n], split s > 0 to Zp[s - 1][mat][pair][n] (fp32), each accumulated from zero (stored as 0 + sum).
-template <int CB, int MK>
-__global__ void __launch_bounds__(PW * 64) __attribute__((amdgpu_waves_per_eu(2)))
-item_gu_kernel(const uint16_t* __restrict__ X0, const uint16_t* __restrict__ X1, const int64_t* __restrict__ TP0,
+// ROT (WB 8, so that one block covers a rank's 256 columns): X0 is x [rows, K] (16-bit, x_stride apart) and suh0 / suh1
+// the stacked scales; the block rotates its rows as rot_in_kernel does, same bits. A pass over the larger items is bound
+// by memory (2048 rows: 3.8 TB/s of the 5.2 a copy reaches), and the rotated pairs were a quarter of its bytes.
+template <int CB, int MK, bool ROT, bool TWO, int WB>
+__global__ void __launch_bounds__(WB * 64) __attribute__((amdgpu_waves_per_eu(ROT ? 4 : 2)))
+item_gu_kernel(const void* __restrict__ X0, const void* __restrict__ X1, const int64_t* __restrict__ TP0,
                const int64_t* __restrict__ TP1, const int* __restrict__ K2_0, const int* __restrict__ K2_1,
                const int* __restrict__ sorted, const int* __restrict__ items, const int* __restrict__ item_count,
                float* __restrict__ Z, float* __restrict__ Zp, int K, int N, int P, int nsplit, int mats, int max_items,
-               int* __restrict__ status) {
-    constexpr int MT = IPM_TILES;
+               int* __restrict__ status, const uint16_t* __restrict__ suh0, const uint16_t* __restrict__ suh1, int x_bf16,
+               int x_stride, int slots) {
+    constexpr int MT = IPM_TILES, NT = WB * 64, NP = (MT * 256 + NT - 1) / NT;
     int e, first, cnt;
     int item, cb, zs;
-    xcd_order((int)blockIdx.x, N / (16 * 2 * PW), mats * nsplit, item, cb, zs);
+    xcd_order((int)blockIdx.x, N / (32 * WB), mats * nsplit, item, cb, zs);
     if (!item_at(items, item_count, 1, max_items, item, e, first, cnt)) return;
     const int mat = zs / nsplit, split = zs % nsplit;
-    const uint16_t* X = mat ? X1 : X0;
     const uint32_t* T = reinterpret_cast<const uint32_t*>(mat ? TP1[e] : TP0[e]);
     const int k2 = mat ? K2_1[e] : K2_0[e];
     // the wave index in a scalar register: the trellis offsets built from it are then scalar (a buffer load's soffset)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     __shared__ int pair_sh[MT * 16];
-    __shared__ __attribute__((aligned(16))) uint16_t xa[MT * 16 * PXS];
-    __shared__ __attribute__((aligned(16))) uint32_t st[PW][pstage(MK)];
+    __shared__ __attribute__((aligned(16))) uint16_t xa[(TWO ? 2 : 1) * MT * 16 * PXS];
+    __shared__ __attribute__((aligned(16))) uint32_t st[WB][pstage(MK)];
     if (tid < MT * 16) pair_sh[tid] = tid < cnt ? sorted[first + tid] : -1;
     __syncthreads();
-    // this thread's activation pieces of every chunk: piece i is row 16 i + (tid >> 4), halves 8 (tid & 15) .. +7;
-    // a piece past the item's row tiles reads row tile 0's address (a cache hit) and is not stored
-    const int mts = (cnt + 15) >> 4;
-    uint32_t aoff[MT];
-    int lofs[MT];
+    // a piece past the item's row tiles reads a row of the first one (a cache hit) and is not stored
+    const int mts = (cnt + 15) >> 4, rows = mts * 16;
+    uint32_t aoff[NP];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        const int row = i * 16 + (tid >> 4);
-        const int rr = i < mts ? row : (tid >> 4);
+    for (int i = 0; i < NP; ++i) {
+        const int row = (i * NT + tid) >> 4, rr = row < rows ? row : row & 15;
         const int p = pair_sh[rr] >= 0 ? pair_sh[rr] : pair_sh[0];
-        aoff[i] = ((uint32_t)p * (uint32_t)K + 8u * (tid & 15)) * 2u;
-        lofs[i] = row * PXS;
+        aoff[i] = ROT ? ((uint32_t)(p / slots) * (uint32_t)x_stride + 8u * (uint32_t)h8_group(lane)) * 2u
+                      : ((uint32_t)p * (uint32_t)K + 8u * (tid & 15)) * 2u;
     }
-    const __amdgpu_buffer_rsrc_t xrs = buffer_rsrc(X, (uint32_t)((size_t)P * K * 2));
-    const int nt0 = cb * (2 * PW) + 2 * wave;
+    GuSrc src;
+    src.bf16 = x_bf16;
+    if constexpr (ROT) {
+        src.x = buffer_rsrc(X0, (uint32_t)(((size_t)(P / slots - 1) * x_stride + K) * 2));
+        src.suh = buffer_rsrc((mat ? suh1 : suh0) + (size_t)e * K, (uint32_t)K * 2u);
+    } else {
+        src.x = src.suh = buffer_rsrc(mat ? X1 : X0, (uint32_t)((size_t)P * K * 2));
+    }
+    const int nt0 = cb * (2 * WB) + 2 * wave;
     const int ns = N >> 4, TWB = 16 * k2;
     TileSpan sp;
     sp.r = buffer_rsrc(T, (uint32_t)((K >> 4) * ns * TWB));
@@ -256,7 +352,7 @@ item_gu_kernel(const uint16_t* __restrict__ X0, const uint16_t* __restrict__ X1,
     const int nch = K / (PK * 16);
     const int c0 = split * nch / nsplit, nc = (split + 1) * nch / nsplit - c0;  // nsplit <= nch: nc >= 1
     const bool ok = EA_K2_SWITCH(
-        k2, 2, MK, (gu_loop<CB, K2V, MT>(xrs, aoff, lofs, sp, xa, st[wave], lane, tid & 15, mts, c0, nc, acc)));
+        k2, 2, MK, (gu_loop<CB, K2V, MT, NT, ROT, TWO>(src, aoff, sp, xa, st[wave], lane, rows, mts, c0, nc, acc)));
     if (!ok) {
         if (lane == 0) record_error(status, DEV_UNSUPPORTED_WIDTH);
 #pragma unroll
@@ -436,6 +532,50 @@ item_ring_kernel(const uint16_t* __restrict__ X0, const uint16_t* __restrict__ X
     }
 }
 
+// The small items' pairs rotated for the ring kernel, when the larger items' products rotate their own: block (item,
+// matrix, 2048 columns), 16 lanes a 128-block (rot_in_kernel's arithmetic); the expert's suh is read once for the item's
+// rows, eight rows' loads in flight. (2048 rows: 601 us a pass, against 617 with rot_in_kernel over all rows, its other
+// pairs skipped.)
+static __global__ void __launch_bounds__(256) item_rot_kernel(const uint16_t* __restrict__ x, int x_bf16, int x_stride,
+                                                       const int* __restrict__ sorted, const int* __restrict__ items,
+                                                       const int* __restrict__ item_count,
+                                                       const uint16_t* __restrict__ suh0, const uint16_t* __restrict__ suh1,
+                                                       uint16_t* __restrict__ out0, uint16_t* __restrict__ out1, int K,
+                                                       int slots, int max_items) {
+    int e, first, cnt;
+    if (!item_at(items, item_count, 0, max_items, blockIdx.x, e, first, cnt)) return;
+    const int lane = threadIdx.x & 63, k = blockIdx.z * 2048 + 128 * ((int)threadIdx.x >> 4) + 8 * h8_group(lane);
+    if (k >= K) return;  // whole 16-lane groups (K % 128 == 0)
+    const u4v sv = *reinterpret_cast<const u4v*>((blockIdx.y ? suh1 : suh0) + (size_t)e * K + k);
+    uint16_t* out = blockIdx.y ? out1 : out0;
+    constexpr int QB = 8;
+    for (int i0 = 0; i0 < cnt; i0 += QB) {
+        int p[QB];
+        u4v xv[QB];
+#pragma unroll
+        for (int i = 0; i < QB; ++i) p[i] = sorted[first + (i0 + i < cnt ? i0 + i : i0)];
+#pragma unroll
+        for (int i = 0; i < QB; ++i) xv[i] = *reinterpret_cast<const u4v*>(x + (size_t)(p[i] / slots) * x_stride + k);
+        issued();
+#pragma unroll
+        for (int i = 0; i < QB; ++i) {
+            if (i0 + i >= cnt) break;  // uniform
+            float f[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const uint16_t h = (uint16_t)(xv[i][j >> 1] >> (16 * (j & 1)));
+                f[j] = (x_bf16 ? bf2f(h) : h2f(h)) * h2f((uint16_t)(sv[j >> 1] >> (16 * (j & 1))));
+            }
+            const float sc = fwht128_x8(f, lane) * HAD_SCALE;  // the values' sign folded into the scale (exact)
+            u4v w;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                w[j] = f2h2(__builtin_fmaf(f[2 * j], sc, 0.f), __builtin_fmaf(f[2 * j + 1], sc, 0.f));
+            *reinterpret_cast<u4v*>(out + (size_t)p[i] * K + k) = w;
+        }
+    }
+}
+
 // The column blocks of a down block for one width: step s is column block s / nch, chunk s % nch; the trellis two
 // steps ahead; each column block's rows are stored when its last chunk is done.
 template <int CB, int K2, int MT, int NG>
@@ -566,7 +706,11 @@ item_dn_kernel(const uint16_t* __restrict__ X, const int64_t* __restrict__ TP, c
 // widths, the items, the pair classes and the per-pair planes (z and zp: gate|up partial sums, xd: down inputs,
 // plane: down outputs). The two lists' pairs are disjoint, so their passes touch disjoint rows of every plane.
 struct ListPass {
-    const uint16_t *xg, *xu;
+    const void* x;  // the pass's rows, and how they lie
+    int x_dtype, x_stride;
+    bool fuse;      // the larger items' products rotate x themselves (rotate_fits); only the small items' pairs go through xg / xu
+    const uint16_t *suh_g, *suh_u;
+    uint16_t *xg, *xu;
     const int64_t* tp[3];
     const int* k2[3];
     const int *sorted, *items, *count, *pclass, *pick;
@@ -578,6 +722,15 @@ struct ListPass {
     int* status;
 };
 
+// Whether the larger items' products can rotate x themselves: 16-bit rows on 16-byte boundaries within 32-bit offsets, and
+// one block over all of a matrix's columns (two would rotate twice).
+static bool rotate_fits(const void* x, int x_dtype, uint32_t x_stride, const uint16_t* suh_g, const uint16_t* suh_u,
+                        uint32_t rows, uint32_t I) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(suh_g) |
+                         reinterpret_cast<uintptr_t>(suh_u) | (uintptr_t)x_stride * 2;
+    return I == 256 && (x_dtype == F16 || x_dtype == BF16) && (at & 15) == 0 && (uint64_t)rows * x_stride * 2 < (1ull << 32);
+}
+
 // One item list from its gate|up product to its down product, in order on q: big = 1 takes the larger items (the
 // gate|up K split into zp; the down matrix by blocks of DNG_BIG column blocks), big = 0 the items of at most
 // SMALL_ROWS pairs (the ring kernel; DNG column blocks). The down matrix takes the resident-activation kernel when
@@ -587,14 +740,30 @@ struct ListPass {
 template <int CB, int MK>
 static int list_pass(hipStream_t q, const ListPass& a, int big) {
     const int ns = gu_splits(a.D);
-    if (big)
-        item_gu_kernel<CB, MK><<<xcd_blocks(a.mi, a.I / (16 * 2 * PW), 2 * ns), PW * 64, 0, q>>>(
-            a.xg, a.xu, a.tp[0], a.tp[1], a.k2[0], a.k2[1], a.sorted, a.items, a.count, a.z, a.zp, a.D, a.I, a.P, ns,
-            2, a.mi, a.status);
-    else  // blocks of 4 waves over 128 columns (8 waves over 256 measured 1 % slower at 512 rows, the same at 2048)
+#define EA_GU(ROT_, TWO_, WB_, X0_, X1_)                                                                                \
+    item_gu_kernel<CB, MK, ROT_, TWO_, WB_><<<xcd_blocks(a.mi, a.I / (32 * (WB_)), 2 * ns), (WB_) * 64, 0, q>>>(             \
+        X0_, X1_, a.tp[0], a.tp[1], a.k2[0], a.k2[1], a.sorted, a.items, a.count, a.z, a.zp, a.D, a.I, a.P, ns, 2, a.mi, \
+        a.status, a.suh_g, a.suh_u, a.x_dtype == BF16, a.x_stride, a.slots)
+    if (big && a.fuse) {
+        if constexpr (MK <= 10) EA_GU(true, true, 8, a.x, a.x);  // fuse is for these widths only (ea_prompt_experts_run)
+    } else if (big && (MK > 10 || a.rows > MID_ROWS)) {
+        EA_GU(false, false, 4, a.xg, a.xu);
+    } else if (big) {
+        if constexpr (MK <= 10) EA_GU(false, true, 4, a.xg, a.xu);
+    } else {
+        if (a.fuse) {  // the small items' pairs, on their own stream
+            item_rot_kernel<<<dim3(a.mi, 2, (a.D + 2047) / 2048), 256, 0, q>>>(
+                static_cast<const uint16_t*>(a.x), a.x_dtype == BF16, a.x_stride, a.sorted, a.items, a.count, a.suh_g,
+                a.suh_u, a.xg, a.xu, a.D, a.slots, a.mi);
+            const int r = launched();
+            if (r) return r;
+        }
+        // blocks of 4 waves over 128 columns (8 waves over 256 measured 1 % slower at 512 rows, the same at 2048)
         item_ring_kernel<CB, MK, 4><<<dim3(a.mi, a.I / 128, 2 * ns), 4 * 64, 0, q>>>(
             a.xg, a.xu, a.tp[0], a.tp[1], a.k2[0], a.k2[1], a.sorted, a.items, a.count, a.z, a.zp, a.D, a.I, a.P, ns,
             a.mi, a.status);
+    }
+#undef EA_GU
     int r = launched();
     if (r) return r;
     r = launch_gateup_epilogue(q, a.z, a.pick, a.svh_g, a.svh_u, a.suh_d, a.xd, (uint32_t)a.rows, (uint32_t)a.P,
@@ -620,9 +789,9 @@ static int list_pass(hipStream_t q, const ListPass& a, int big) {
             EA_DN(SMALL_ROWS / 16, 2, PW, dim3(a.mi, nb / 2, 1));
 #undef EA_DN
     } else if (big) {
-        item_gu_kernel<CB, MK><<<xcd_blocks(a.mi, a.D / (16 * 2 * PW), 1), PW * 64, 0, q>>>(
+        item_gu_kernel<CB, MK, false, false, 4><<<xcd_blocks(a.mi, a.D / 128, 1), 256, 0, q>>>(
             a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, nullptr, a.I, a.D,
-            a.P, 1, 1, a.mi, a.status);
+            a.P, 1, 1, a.mi, a.status, nullptr, nullptr, 0, 0, 1);
     } else {
         item_ring_kernel<CB, MK, 4><<<dim3(a.mi, a.D / 128, 1), 4 * 64, 0, q>>>(
             a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, nullptr, a.I, a.D, a.P,

@@ -292,6 +292,32 @@ def test_prompt_experts_wide_widths_resident_down(ea, k2, cb, R, E, I):
     assert device.device_status() == 0
 
 
+@pytest.mark.parametrize("x_dtype,pad,planes", [(0, 0, True), (1, 8, False), (1, 2, False)])
+def test_prompt_experts_long_pass_rotations(ea, x_dtype, pad, planes):
+    """More than 1,024 rows: the larger items' products rotate x themselves (16-bit rows on 16-byte boundaries, strided or
+    not) or, for rows that do not lie so (pad 2), read rotated pairs: the oracle's bar, and a row's bits are those of the
+    same row in a shorter pass, which always takes the rotation launch."""
+    device, _, moe, pe, synth = ea
+    R, E, D, I, short = 1030, 48, 512, 256, 200
+    pick, wts = synth.picks_zipf(990, R, 1.1, E, 8), synth.routing_weights(991, R, 8)
+    pick[3, 2] = -1  # a slot without an expert
+    host = synth.HostLayer(992, experts=E, dims=D, width=I, k2=synth.mixed_widths(5, E), cb=1, only=np.unique(pick[pick >= 0]))
+    x = synth.activations(993, R, D, ["f16", "bf16"][x_dtype])
+    wide = np.zeros((R, D + pad), np.uint16)
+    wide[:, :D] = x
+    ex = moe.Routed(host)
+    dx, dp, dw = device.upload(wide), device.upload(pick), device.upload(wts)
+    out, head = device.zeros((R, D), torch.float32), device.zeros((short, D), torch.float32)
+    pe.run(device.stream(), dx.data_ptr(), D + pad, dp.data_ptr(), dw.data_ptr(), ex, pe.Scratch(ex, R, 8, planes=planes),
+           out.data_ptr(), R, do_round=False, x_dtype=x_dtype)
+    pe.run(device.stream(), dx.data_ptr(), D + pad, dp.data_ptr(), dw.data_ptr(), ex,
+           pe.Scratch(ex, short, 8, planes=planes), head.data_ptr(), short, do_round=False, x_dtype=x_dtype)
+    got = device.download(out)
+    assert_close_rms(got, orc.prompt_experts(x, pick, wts, oracle_routed(host), R, 8, bf16=x_dtype == 1), 2e-3, "long pass")
+    np.testing.assert_array_equal(got[:short], device.download(head))
+    assert device.device_status() == 0
+
+
 @pytest.mark.parametrize("planes", [True, False])
 def test_prompt_experts_f32_activations(ea, planes):
     """fp32 activations (x_dtype 2: the rotation launch reads them and rounds the rotated rows to fp16 as for 16-bit
