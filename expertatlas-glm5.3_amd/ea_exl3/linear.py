@@ -58,11 +58,18 @@ class Scratch:
             self.c.z[i] = self.z[i].data_ptr()
 
 
+_ADDRS = tuple(U64 * n for n in range(MAX_JOBS + 1))
+_CODES = tuple(C.c_int * n for n in range(MAX_JOBS + 1))
+
+
+def _addrs(v):
+    return (_ADDRS[len(v)] if len(v) <= MAX_JOBS else U64 * len(v))(*v)
+
+
 def _arrays(ls, outs, dtypes):
-    arr = (C.POINTER(_Linear) * len(ls))(*[C.pointer(l.c) for l in ls])
-    o = (U64 * len(outs))(*outs)
-    d = (C.c_int * len(dtypes))(*dtypes)
-    return arr, o, d
+    """The layers' addresses, the output addresses and the dtype codes as C arrays."""
+    codes = _CODES[len(dtypes)] if len(dtypes) <= MAX_JOBS else C.c_int * len(dtypes)
+    return _addrs([C.addressof(l.c) for l in ls]), _addrs(outs), codes(*dtypes)
 
 
 def call(stream: int, s: Scratch, ls, x: int, x_dtype: int, m: int, outs, out_dtypes) -> None:
