@@ -1,10 +1,11 @@
-// Library set-up, status words, trellis dequantisation, the router's top-8 and the shared expert's SwiGLU.
+// Library set-up, status words, trellis dequantisation and the shared expert's SwiGLU.
 #include <hip/hip_runtime.h>
 
 #include <mutex>
 #include <vector>
 
 #include "ea_device.hpp"
+#include "ea_experts.hpp"
 #include "ea_gemm.hpp"
 #include "ea_host.hpp"
 
@@ -48,62 +49,6 @@ __global__ void __launch_bounds__(256) unpack_kernel(const uint32_t* __restrict_
     const uint32_t* tile = T + kt * stride_k + (nt >> 3) * stride_nb + (nt & 7) * 4 * k2;
     const bool ok = EA_K2_SWITCH(k2, 2, 16, (unpack_tile<CB, K2V>(tile, W, N, kt, nt, lane)));
     (void)ok;
-}
-
-// ---- router top-8 ----------------------------------------------------------------------------------------------
-// One block a row, a thread an expert (E = 256). Eight rounds of a block arg-max over the ranking key of choice =
-// sigmoid + bias (order_key: NaN below every number), the lower id winning ties; the winner's key becomes 0, below
-// every choice (native_ops.cu:1015-1068).
-__global__ void __launch_bounds__(256) topk8_kernel(const float* __restrict__ logits, const float* __restrict__ bias,
-                                                    int32_t* __restrict__ pick, float* __restrict__ wts, float scale,
-                                                    uint8_t* __restrict__ log) {
-    __shared__ uint32_t s_key[4];
-    __shared__ int s_idx[4];
-    __shared__ float s_wts[8];
-    __shared__ int s_pick[8];
-    const int r = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const float score = 1.0f / (expf_path(0.0f - logits[(size_t)r * 256 + t]) + 1.0f);
-    uint32_t key = order_key(score + bias[t]);
-    for (int k = 0; k < 8; ++k) {
-        uint32_t v = key;
-        int i = t;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const uint32_t ov = (uint32_t)__shfl_xor((int)v, o, 64);
-            const int oi = __shfl_xor(i, o, 64);
-            if (ov > v || (ov == v && oi < i)) {
-                v = ov;
-                i = oi;
-            }
-        }
-        if (lane == 0) {
-            s_key[wave] = v;
-            s_idx[wave] = i;
-        }
-        __syncthreads();
-        uint32_t bv = s_key[0];
-        int bi = s_idx[0];
-#pragma unroll
-        for (int w = 1; w < 4; ++w)
-            if (s_key[w] > bv || (s_key[w] == bv && s_idx[w] < bi)) {
-                bv = s_key[w];
-                bi = s_idx[w];
-            }
-        __syncthreads();  // every thread has read the winners before the next round writes them
-        if (t == bi) {
-            s_pick[k] = bi;
-            s_wts[k] = score;
-            key = 0u;
-        }
-    }
-    __syncthreads();
-    if (t < 8) {
-        float total = 0.0f;
-        for (int k = 0; k < 8; ++k) total = total + s_wts[k];
-        pick[(size_t)r * 8 + t] = s_pick[t];
-        wts[(size_t)r * 8 + t] = s_wts[t] / (total + 1e-20f) * scale;
-        if (log) log[(size_t)r * 8 + t] = (uint8_t)s_pick[t];
-    }
 }
 
 // ---- SwiGLU of the shared expert ------------------------------------------------------------------------------
@@ -293,8 +238,7 @@ int ea_topk8(ea_stream_t stream, const float* logits, const float* bias, int32_t
     EA_REQUIRE_CTX(c);
     if (!logits || !bias || !pick || !wts) return EA_BAD_ARGUMENT;
     if (rows == 0) return EA_OK;
-    topk8_kernel<<<rows, 256, 0, as_stream(stream)>>>(logits, bias, pick, wts, scale, log);
-    return launched();
+    return launch_topk8(as_stream(stream), logits, bias, pick, wts, rows, scale, log);
 }
 
 int ea_swiglu2(ea_stream_t stream, const void* g, const void* u, void* out, uint32_t rows, uint32_t width) {

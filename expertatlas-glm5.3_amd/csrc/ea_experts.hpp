@@ -39,6 +39,10 @@ int decode_layer(hipStream_t s, const void* x, int x_dtype, uint32_t x_stride, c
                  const ea_linear* const* shared, const ea_moe_scratch* sc, float* out, uint32_t R,
                  const void* router_w = nullptr);
 
+// ops.topk (ea_decode_layer.hip): the top-8 of each row's 256 logits; log: null or a byte a pick.
+int launch_topk8(hipStream_t s, const float* logits, const float* bias, int32_t* pick, float* wts, uint32_t rows,
+                 float scale, uint8_t* log);
+
 // The router's logits (ea_router.hip): out fp32 [m, ne] = x [m, d] @ w^T, eight slices added in order.
 int launch_router(hipStream_t s, const void* x, int x_dtype, uint32_t x_stride, const void* w, float* part, float* out,
                   uint32_t m, uint32_t d, uint32_t ne);
