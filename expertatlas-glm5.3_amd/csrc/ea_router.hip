@@ -7,8 +7,10 @@
 // c = l, l + 64, l + 128, .. of the slice (c < kw / 4) in ascending order, each chunk's values in order, by fp32 fma;
 // then the 64 lane sums are added by a butterfly over lane distances 32, 16, 8, 4, 2, 1. Products of 16-bit operands
 // are exact in fp32, so an fma and a multiply-then-add give the same bits. A block holds the eight slices of its
-// experts and rows (a wave a slice) and adds them in slice order, so the logits need no second launch.
+// expert and rows (a wave a slice) and adds them in slice order, so the logits need no second launch.
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "ea_device.hpp"
 #include "ea_gemm.hpp"
@@ -17,17 +19,36 @@
 namespace ea {
 
 constexpr int RT_SLICES = 8;  // ops.zig:133
-constexpr int RT_ROWS = 16;   // rows a block
 
-// The lane sums of a wave added by the butterfly; every lane ends with the total.
-__device__ __forceinline__ float wave_sum_butterfly(float v) {
-    v = v + lane_xor<32>(v);
-    v = v + lane_xor<16>(v);
-    v = v + lane_xor<8>(v);
-    v = v + lane_xor<4>(v);
-    v = v + lane_xor<2>(v);
-    v = v + lane_xor<1>(v);
-    return v;
+// The lane sums of a wave added by the butterfly, for N (a power of two, at most 32) values: in the first steps a lane keeps
+// half of its values and hands its partner the others, so that each value is summed once (the two halves' sum has the same
+// bits on either side). v[0] ends as the total of value wave_sums() of the lane, the same in 64 / N neighbouring lanes.
+template <int N>
+__device__ __forceinline__ int wave_sums(float (&v)[N], int lane) {
+    int mine = 0;
+    auto step = [&](auto dist_, auto half_) __attribute__((always_inline)) {
+        constexpr int D = decltype(dist_)::value, H = decltype(half_)::value;
+        if constexpr (H > 0) {
+            const bool up = (lane & D) != 0;
+#pragma unroll
+            for (int i = 0; i < H; ++i) {
+                const float keep = up ? v[i + H] : v[i], give = up ? v[i] : v[i + H];
+                v[i] = keep + lane_xor<D>(give);
+            }
+            mine += up ? H : 0;
+        } else {
+            v[0] = v[0] + lane_xor<D>(v[0]);
+        }
+    };
+#define EA_STEP(D_, H_) step(std::integral_constant<int, D_>{}, std::integral_constant<int, H_>{})
+    EA_STEP(32, N / 2);
+    EA_STEP(16, N / 4);
+    EA_STEP(8, N / 8);
+    EA_STEP(4, N / 16);
+    EA_STEP(2, N / 32);
+    EA_STEP(1, 0);
+#undef EA_STEP
+    return mine;
 }
 
 __device__ __forceinline__ void act4(uint2 u, bool bf, float (&v)[4]) {
@@ -37,97 +58,68 @@ __device__ __forceinline__ void act4(uint2 u, bool bf, float (&v)[4]) {
     for (int i = 0; i < 4; ++i) v[i] = bf ? bf2f(h[i]) : h2f(h[i]);
 }
 
-// Block (expert group of EB, row group of RT_ROWS): wave s computes slice s of every (row, expert) of the block.
-// ONE (m = 1): the lane's chunks four at a time, every weight and activation load of the four issued before the
-// first product (a chunk past the slice re-reads the slice's last chunk and is not added); the same sums in the same
-// order as the general form, whose loads of a row under `r < rows` wait chunk by chunk.
-template <int EB, bool ONE>
-__global__ void __launch_bounds__(64 * RT_SLICES) router_kernel(const uint16_t* __restrict__ x, int x_bf16,
-                                                                int x_stride, const uint16_t* __restrict__ w,
-                                                                float* __restrict__ part, float* __restrict__ out,
-                                                                int m, int d, int ne) {
-    __shared__ float sums[RT_SLICES][RT_ROWS][EB];
-    const int lane = threadIdx.x & 63, s = threadIdx.x >> 6;
-    const int e0 = blockIdx.x * EB, m0 = blockIdx.y * RT_ROWS;
-    const int rows = min(RT_ROWS, m - m0), kw = d / RT_SLICES, nc = kw / 4;
-    const bool bf = x_bf16 != 0;
-    float acc[RT_ROWS][EB];
+// Block (expert, row group of ROWS), wave s: slice s of the expert and the group's rows. What bounds it at few rows is round
+// trips (3.1 MB of weights at 256 x 6144 are 0.5 us of HBM, a block's rows come from L2), with more the rows' unpacking and
+// products. So the loads of RT_BATCH chunks of the weight and of every row are issued before the first product (a row past
+// m re-reads the last one, a chunk past the slice the slice's last, and is not added), the type is fixed at compile time,
+// and the rows' lane sums share their steps (wave_sums). The form before read each row under a condition of its own, which
+// waited for its load, and took four experts a block above 16 rows. 256 x 6144, distinct weights: 1 row 3.5 -> 2.9 us, 2 rows
+// 6.6 -> 3.2, 5 rows 8.6 -> 4.5, 16 rows 16.2 -> 6.7, 37 rows 19.6 -> 12.7, 128 rows 38 -> 26.5, 512 rows 190 -> 94.
+constexpr int RT_BATCH = 3;  // the chunks of a lane's slice at d = 6144
+template <int ROWS, bool BF>
+__global__ void __launch_bounds__(64 * RT_SLICES) router_kernel(const uint16_t* __restrict__ x, int x_stride,
+                                                                    const uint16_t* __restrict__ w,
+                                                                    float* __restrict__ part, float* __restrict__ out,
+                                                                    int m, int d, int ne) {
+    __shared__ float sums[RT_SLICES][ROWS];
+    const int lane = threadIdx.x & 63, s = threadIdx.x >> 6, e = blockIdx.x, m0 = (int)blockIdx.y * ROWS;
+    const int rows = min(ROWS, m - m0);
+    const int kw = d / RT_SLICES, nc = kw / 4;
+    float acc[ROWS];
 #pragma unroll
-    for (int r = 0; r < RT_ROWS; ++r)
+    for (int r = 0; r < ROWS; ++r) acc[r] = 0.0f;
+    const uint16_t* wr = w + (size_t)e * d + (size_t)s * kw;
+    const uint16_t* xr = x + (size_t)m0 * x_stride + (size_t)s * kw;
+    for (int c0 = 0; c0 < nc; c0 += RT_BATCH * 64) {
+        uint2 wu[RT_BATCH], xu[RT_BATCH][ROWS];
 #pragma unroll
-        for (int j = 0; j < EB; ++j) acc[r][j] = 0.0f;
-    const size_t k_lo = (size_t)s * kw;
-    if constexpr (ONE) {
-        static_assert(EB == 1, "one row: one expert a block");
-        const uint16_t* wr = w + (size_t)e0 * d + k_lo;  // e0 < ne: a block per expert
-        const uint16_t* xr = x + (size_t)m0 * x_stride + k_lo;
-        for (int c0 = 0; c0 < nc; c0 += 4 * 64) {
-            uint2 wu[4], xu[4];
+        for (int i = 0; i < RT_BATCH; ++i) {
+            const size_t k = 4 * (size_t)min(c0 + i * 64 + lane, nc - 1);
+            wu[i] = *reinterpret_cast<const uint2*>(wr + k);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int c = min(c0 + i * 64 + lane, nc - 1);
-                wu[i] = *reinterpret_cast<const uint2*>(wr + 4 * (size_t)c);
-                xu[i] = *reinterpret_cast<const uint2*>(xr + 4 * (size_t)c);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float wv[4], xv[4];
-                act4(wu[i], true, wv);
-                act4(xu[i], bf, xv);
-                if (c0 + i * 64 + lane < nc)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) acc[0][0] = __builtin_fmaf(xv[q], wv[q], acc[0][0]);
-            }
+            for (int r = 0; r < ROWS; ++r)
+                xu[i][r] = *reinterpret_cast<const uint2*>(xr + (size_t)min(r, rows - 1) * x_stride + k);
         }
-    } else {
-#pragma unroll 3
-        for (int c = lane; c < nc; c += 64) {
-            const size_t k = k_lo + 4 * (size_t)c;
-            uint2 wu[EB];
+        issued();
 #pragma unroll
-            for (int j = 0; j < EB; ++j)
-                wu[j] = e0 + j < ne ? *reinterpret_cast<const uint2*>(w + (size_t)(e0 + j) * d + k) : uint2{0u, 0u};
-            float wv[EB][4];
+        for (int i = 0; i < RT_BATCH; ++i) {
+            float wv[4];
+            act4(wu[i], true, wv);
+            const bool in = c0 + i * 64 + lane < nc;
 #pragma unroll
-            for (int j = 0; j < EB; ++j) act4(wu[j], true, wv[j]);
+            for (int r = 0; r < ROWS; ++r) {
+                float xv[4], t = acc[r];
+                act4(xu[i][r], BF, xv);
 #pragma unroll
-            for (int r = 0; r < RT_ROWS; ++r) {
-                if (r < rows) {
-                    float xv[4];
-                    act4(*reinterpret_cast<const uint2*>(x + (size_t)(m0 + r) * x_stride + k), bf, xv);
-#pragma unroll
-                    for (int j = 0; j < EB; ++j)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[r][j] = __builtin_fmaf(xv[i], wv[j][i], acc[r][j]);
-                }
+                for (int q = 0; q < 4; ++q) t = __builtin_fmaf(xv[q], wv[q], t);
+                acc[r] = in ? t : acc[r];
             }
         }
     }
-#pragma unroll
-    for (int r = 0; r < RT_ROWS; ++r) {
-        if (r < rows) {
-#pragma unroll
-            for (int j = 0; j < EB; ++j) {
-                const float t = wave_sum_butterfly(acc[r][j]);
-                if (lane == 0) sums[s][r][j] = t;
-            }
-        }
-    }
+    const int mine = wave_sums<ROWS>(acc, lane);
+    if ((lane & (64 / ROWS - 1)) == 0) sums[s][mine] = acc[0];
     __syncthreads();
-    const int t = threadIdx.x;
-    if (t < rows * EB) {
-        const int r = t / EB, j = t % EB, e = e0 + j;
-        if (e < ne) {
-            float tot = sums[0][r][j];
-            if (part) part[(size_t)(m0 + r) * ne + e] = tot;
+    const int r = threadIdx.x;
+    if (r < rows) {
+        float tot = sums[0][r];
+        if (part) part[(size_t)(m0 + r) * ne + e] = tot;
 #pragma unroll
-            for (int q = 1; q < RT_SLICES; ++q) {
-                const float p = sums[q][r][j];
-                if (part) part[((size_t)q * m + m0 + r) * ne + e] = p;
-                tot = tot + p;
-            }
-            out[(size_t)(m0 + r) * ne + e] = tot;
+        for (int q = 1; q < RT_SLICES; ++q) {
+            const float p = sums[q][r];
+            if (part) part[((size_t)q * m + m0 + r) * ne + e] = p;
+            tot = tot + p;
         }
+        out[(size_t)(m0 + r) * ne + e] = tot;
     }
 }
 
@@ -141,19 +133,19 @@ int launch_router(hipStream_t s, const void* x, int x_dtype, uint32_t x_stride, 
     if (x_stride < d || x_stride % 4 != 0) return EA_BAD_ROW_STRIDE;
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) & 7) return EA_BAD_ARGUMENT;
     if (m == 0 || ne == 0) return EA_OK;
-    const unsigned gy = (m + RT_ROWS - 1) / RT_ROWS;
     const auto* xs = static_cast<const uint16_t*>(x);
     const auto* ws = static_cast<const uint16_t*>(w);
-    if (m == 1)
-        router_kernel<1, true><<<dim3(ne, gy), 64 * RT_SLICES, 0, s>>>(xs, x_dtype == BF16, (int)x_stride, ws, part,
-                                                                        out, (int)m, (int)d, (int)ne);
-    else if (m <= RT_ROWS)
-        router_kernel<1, false><<<dim3(ne, gy), 64 * RT_SLICES, 0, s>>>(xs, x_dtype == BF16, (int)x_stride, ws, part,
-                                                                         out, (int)m, (int)d, (int)ne);
-    else
-        router_kernel<4, false><<<dim3((ne + 3) / 4, gy), 64 * RT_SLICES, 0, s>>>(xs, x_dtype == BF16, (int)x_stride,
-                                                                                   ws, part, out, (int)m, (int)d,
-                                                                                   (int)ne);
+    // rows a block (the least power of two that holds m, at most 16): a block's rows share one read of its weights
+#define EA_RF(ROWS_)                                                                                                   \
+    (x_dtype == BF16 ? router_kernel<ROWS_, true> : router_kernel<ROWS_, false>)                                       \
+        <<<dim3(ne, (m + (ROWS_) - 1) / (ROWS_)), 64 * RT_SLICES, 0, s>>>(xs, (int)x_stride, ws, part, out, (int)m,    \
+                                                                          (int)d, (int)ne)
+    if (m == 1) EA_RF(1);
+    else if (m == 2) EA_RF(2);
+    else if (m <= 4) EA_RF(4);
+    else if (m <= 8) EA_RF(8);
+    else EA_RF(16);
+#undef EA_RF
     return launched();
 }
 

@@ -120,6 +120,13 @@ def test_gpu_router_bit_exact(ea, m, d, ne, x_dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("d", [512, 1536, 6144, 7168])  # a lane's chunks: none for most, none or one, three, three or four
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9, 15, 16, 17])  # the row groups' sizes and remainders
+def test_gpu_router_row_groups(ea, m, d):
+    test_gpu_router_bit_exact(ea, m, d, 5, m & 1)
+
+
+@pytest.mark.gpu
 def test_gpu_router_errors(ea):
     torch, device, ops = ea
     from ea_exl3._lib import EaError
