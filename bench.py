@@ -11,7 +11,7 @@ A step is one pass of the hot path over one batch of synthetic input, with every
   stack (config 5): 75 resident layers (3-bit for 70 % of the experts), one token through all of them (us / token);
   linear (config 1): one 4-bit EXL3 linear 6144 x 2048 at one row (linear.call);
   prefill512 / prefill2048 (config 4): prompt_experts.run over 512 / 2048 rows with Zipf(1.1) routing (a _planes0
-      suffix: without the pair plane, the reference's default atomic mode).
+      suffix: without the pair plane, the reference's default).
 The default run times config 2 and then, into the same line as objects of their own, the workloads named by --legs
 (the other BASELINE configs). Every GPU leg runs before any CPU work: a leg spins up on its own work (--spin-up
 seconds of untimed calls), runs one layer outside the timed region whose output it keeps, does its W warm-up steps,
@@ -72,7 +72,7 @@ def parse():
                     help="decode configs: ea_ffn_moe_decode, or the reference's launch sequence (topk, "
                          "moe.routed's six launches, the shared expert's linears, swiglu2, add)")
     ap.add_argument("--planes", type=int, default=1, choices=[0, 1],
-                    help="prefill legs without a _planes0 suffix: 1 the pair plane and slot-ordered combine, 0 atomics")
+                    help="prefill legs without a _planes0 suffix: 1 the pair plane, 0 none")
     ap.add_argument("--spin-up", type=float, default=0.3,
                     help="seconds of untimed calls of each leg's own work before its warm-up steps")
     ap.add_argument("--cpu-budget", type=float, default=8.0, help="seconds of CPU work each leg's CPU baseline samples")
@@ -1010,7 +1010,7 @@ def run_prefill(args, torch, np, R: int, planes: int = 1) -> Leg:
     t_hbm, t_mfma = b / (HBM_PEAK_GBS * 1e9) * 1e6, f / (FP16_PEAK_TFLOPS * 1e12) * 1e6
     gbs, tfs = b / (us * 1e-6) / 1e9, f / (us * 1e-6) / 1e12
     mode = ("planes 1: the pair plane and the slot-ordered combine (the same bits every run)" if planes else
-            "planes 0: down items add into out with fp32 atomics in arrival order (the reference's default mode 0)")
+            "planes 0: no pair plane, the down rows over the pairs' rotated inputs (the reference's default mode 0)")
     config = {"workload": f"config 4: prefill chunk of {R} tokens x 6144 through prompt_experts.run, Zipf(1.1) top-8 "
                           "routing over 256 4-bit experts", "mode": mode, "distinct_experts": len(distinct),
               "step_bytes": b, "step_flops": f, "step_roofline_us": round(max(t_hbm, t_mfma), 3),
