@@ -66,8 +66,12 @@ constexpr int LONG_ROWS = 1024;
 // few blocks wait on each chunk's round trip, many on each other for a place.
 constexpr int MID_ROWS = 600;
 constexpr int GU_SPLIT = 2;                       // K splits of a larger item's gate|up (4 and 8 measured slower)
-// The number of K splits of a larger item's gate|up over K (at most one a chunk).
-static int gu_splits(int K) { return K / (PK * 16) < GU_SPLIT ? K / (PK * 16) : GU_SPLIT; }
+// The number of K splits of an item's gate|up over K (at most one a chunk). A layer that holds a width above 10 keeps one sum
+// over all of K in ascending order: two splits change its bits and measured no faster (777 rows of 5, 6 and 8 bits: 428 us
+// with one, 430 with two).
+static int gu_splits(int K, bool wide = false) {
+    return wide ? 1 : K / (PK * 16) < GU_SPLIT ? K / (PK * 16) : GU_SPLIT;
+}
 constexpr int DXS = 2 * PK * 16 + 8;              // down matrix: LDS row stride of the activations (K up to 256)
 
 // An activation piece (8 halves: column 8 q8 .. +7 of a chunk row) into LDS. Within each 32-k step of the row
@@ -739,7 +743,7 @@ static bool rotate_fits(const void* x, int x_dtype, uint32_t x_stride, const uin
 // epilogue is done.
 template <int CB, int MK>
 static int list_pass(hipStream_t q, const ListPass& a, int big) {
-    const int ns = gu_splits(a.D);
+    const int ns = gu_splits(a.D, MK > 10);
 #define EA_GU(ROT_, TWO_, WB_, X0_, X1_)                                                                                \
     item_gu_kernel<CB, MK, ROT_, TWO_, WB_><<<xcd_blocks(a.mi, a.I / (32 * (WB_)), 2 * ns), (WB_) * 64, 0, q>>>(             \
         X0_, X1_, a.tp[0], a.tp[1], a.k2[0], a.k2[1], a.sorted, a.items, a.count, a.z, a.zp, a.D, a.I, a.P, ns, 2, a.mi, \

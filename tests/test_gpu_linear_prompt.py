@@ -292,6 +292,45 @@ def test_prompt_experts_wide_widths_resident_down(ea, k2, cb, R, E, I):
     assert device.device_status() == 0
 
 
+@pytest.mark.parametrize("planes", [True, False])
+@pytest.mark.parametrize("R,k2,cb", [(40, 12, 1), (300, 11, 2), (300, 16, 0), (1100, "wide-mixed", 1)])
+def test_prompt_experts_wide_layers_sum_k_in_order(ea, R, k2, cb, planes):
+    """A layer that holds a width above 10 sums gate and up over all of K in ascending order, in one accumulator. Block 0
+    of K (128 columns) puts one large product into every sum and block 2, with block 0's tiles and the opposite sign, takes
+    it out again: in that order exactly, so the last block's small products leave the same bits as without the two. Sums of
+    K's halves, added at the end, lose the small products' low bits against the large one (2^-24 of 4e4 is 1 % of them)."""
+    device, _, moe, pe, synth = ea
+    E, D, I = 24, 512, 256
+    k2v = np.array([(12, 8, 6, 16, 10, 11, 4, 14)[e % 8] for e in range(E)], np.int32) if k2 == "wide-mixed" else k2
+    pick, wts = synth.picks_zipf(810 + R, R, 1.1, E, 8), synth.routing_weights(811, R, 8)
+    host = synth.HostLayer(812, experts=E, dims=D, width=I, k2=k2v, cb=cb, only=np.unique(pick))
+    for m in (0, 1):
+        for t in host.trellis[m]:
+            if t is not None:
+                rows = t.reshape(D // 16, -1)
+                rows[16:24] = rows[0:8]
+    host.suh_g = host.suh_u = synth.f16_bits(np.ones(E * D))
+    small = np.zeros((R, D), np.float32)
+    small[:, 384:] = synth.bf16_to_f32(synth.bf16_bits(0.015 * synth.activations(813, R, D, "f32")[:, 384:]))
+    had = np.array([[(-1.0) ** bin(i & j).count("1") for j in range(128)] for i in range(128)], np.float32)
+    both = small.copy()
+    both[:, 0:128] = 4096.0 * had[np.arange(R) % 128]  # rotated: one entry of 4096 sqrt(128), the others exactly zero
+    both[:, 256:384] = -both[:, 0:128]
+    ex = moe.Routed(host)
+    sc = pe.Scratch(ex, R, 8, planes=planes)
+    dp, dw = device.upload(pick), device.upload(wts)
+    got = []
+    for x in (small, both):
+        dx = device.upload(synth.bf16_bits(x))
+        out = device.zeros((R, D), torch.float32)
+        pe.run(device.stream(), dx.data_ptr(), D, dp.data_ptr(), dw.data_ptr(), ex, sc, out.data_ptr(), R, do_round=False)
+        got.append(device.download(out))
+    want = orc.prompt_experts(synth.bf16_bits(small), pick, wts, oracle_routed(host), R, 8, bf16=True)
+    assert_close_rms(got[0], want, 2e-3, f"wide layer, small rows, K2 {k2}")
+    np.testing.assert_array_equal(got[1], got[0])
+    assert device.device_status() == 0
+
+
 @pytest.mark.parametrize("x_dtype,pad,planes", [(0, 0, True), (1, 8, False), (1, 2, False)])
 def test_prompt_experts_long_pass_rotations(ea, x_dtype, pad, planes):
     """More than 1,024 rows: the larger items' products rotate x themselves (16-bit rows on 16-byte boundaries, strided or
