@@ -297,6 +297,8 @@ static void launch_rows_k2(hipStream_t s, ea_jobs jobs, const ea_rot_jobs& rj, b
 
 constexpr int LR_ROT_ROWS = 32;  // rows a rotating block takes at most
 
+static bool overlap(uint64_t a, size_t an, uint64_t b, size_t bn) { return a < b + bn && b < a + an; }
+
 int launch_linear_rows(hipStream_t s, const ea_jobs& jobs, const ea_rot_jobs* rot, int M, int K, uint32_t k2,
                        uint32_t cb, const void* x, int x_dtype) {
     EA_REQUIRE_CTX(c);
@@ -307,8 +309,14 @@ int launch_linear_rows(hipStream_t s, const ea_jobs& jobs, const ea_rot_jobs* ro
     for (int i = 0; i < jobs.n; ++i) blocks += jobs.j[i].SK > 1 ? jobs.j[i].N / 64 * jobs.j[i].SK : jobs.j[i].N / 128;
     bool fuse = rot && (M <= LR_ROT_ROWS || blocks * ((M + LR_ROT_ROWS - 1) / LR_ROT_ROWS) <= c->cus) && (x_dtype == F16 || x_dtype == BF16) &&
                 (reinterpret_cast<uintptr_t>(x) & 15) == 0;
-    for (int i = 0; fuse && i < jobs.n; ++i)
-        fuse = K / jobs.j[i].SK % 128 == 0 && (rot->suh[i] & 15) == 0 && (rot->xh[i] & 15) == 0;
+    // and x is left alone meanwhile (an output, or xh, in its place: the rotation is done before the products start then)
+    const uint64_t xa = reinterpret_cast<uintptr_t>(x);
+    for (int i = 0; fuse && i < jobs.n; ++i) {
+        const ea_job& j = jobs.j[i];
+        const size_t xb = (size_t)M * K * 2, yb = (size_t)M * j.N * (j.y_dtype == F32 ? 4 : 2);
+        fuse = K / j.SK % 128 == 0 && (rot->suh[i] & 15) == 0 && (rot->xh[i] & 15) == 0 && !overlap(xa, xb, j.y, yb) &&
+               !overlap(xa, xb, rot->xh[i], xb);
+    }
     if (rot && !fuse) {
         const int r = launch_lin_rot_in(s, x, x_dtype, rot, (uint32_t)jobs.n, (uint32_t)M, (uint32_t)K);
         if (r) return r;

@@ -166,6 +166,38 @@ def test_linear_many_rows(ea, M, K, Ns, k2, cb, x_dtype):
     assert device.device_status() == 0 and all(np.isfinite(f).all() for f in first)
 
 
+@pytest.mark.parametrize("M,K,N,jobs", [(1, 512, 512, 1), (20, 512, 512, 2), (128, 896, 896, 1), (70, 768, 256, 2),
+                                        (33, 256, 1024, 1)])
+def test_linear_output_in_place_of_the_input(ea, M, K, N, jobs):
+    """One K split: the first output takes the input's place (from its first byte on, shorter or longer than it), and the
+    rotated rows are taken before any of it is stored: every output's bits are those of a call that leaves x alone."""
+    device, linear, _, _, synth = ea
+    lins = []
+    for i in range(jobs):
+        T = synth.trellis(190 + i, 0, 0, 0, K, N, 8)
+        lins.append(linear.Linear(T, synth.scales(191 + i, K, 1.0), synth.scales(192 + i, N, 0.02), K, N, 8, 1))
+        assert lins[-1].sk == 1
+    x = synth.activations(193, M, K, "bf16")
+    sc = linear.Scratch(M, K, 1)
+    apart, got = [device.zeros((M, N), torch.int16) for _ in lins], [device.zeros((M, N), torch.int16) for _ in lins]
+    dx = device.upload(x)
+    linear.call(device.stream(), sc, lins, dx.data_ptr(), 1, M, [o.data_ptr() for o in apart], [1] * jobs)
+    both = device.zeros((M * max(K, N),), torch.int16)
+    both[: M * K] = device.upload(x).view(torch.int16).reshape(-1)
+    linear.call(device.stream(), sc, lins, both.data_ptr(), 1, M, [both.data_ptr()] + [o.data_ptr() for o in got[1:]],
+                [1] * jobs)
+    np.testing.assert_array_equal(device.download(both)[: M * N].reshape(M, N), device.download(apart[0]))
+    for a, b in zip(got[1:], apart[1:]):
+        np.testing.assert_array_equal(device.download(a), device.download(b))
+    # xh in the input's place: the rotation alone writes there
+    dx2 = device.upload(x)
+    sc.c.xh[0] = dx2.data_ptr()
+    y = device.zeros((M, N), torch.int16)
+    linear.call(device.stream(), sc, lins[:1], dx2.data_ptr(), 1, M, [y.data_ptr()], [1])
+    np.testing.assert_array_equal(device.download(y), device.download(apart[0]))
+    assert device.device_status() == 0
+
+
 def test_linear_errors(ea):
     device, linear, _, _, synth = ea
     from ea_exl3._lib import EaError
