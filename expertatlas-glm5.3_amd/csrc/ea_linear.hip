@@ -471,6 +471,9 @@ static bool launch_small(const ea_jobs& jobs, const ea_rot_jobs* rj, hipStream_t
         if (j.SK < 2 || (K >> 4) % (j.SK * wk) != 0 || (K >> 4) / j.SK / wk != nkt) return false;
         if (!rj && (!j.xh || (j.xh & 15))) return false;
         if (rj && ((rj->suh[i] & 15) || (rj->xh[i] & 3))) return false;
+        // its trellis offsets are 32-bit (the kernel for more rows takes any strides)
+        const int64_t span = (int64_t)((j.N >> 7) - 1) * j.stride_nb + (int64_t)(K >> 4) * j.stride_k;
+        if (j.stride_k < 0 || j.stride_nb < 0 || span >= (1ll << 29)) return false;
     }
     if (nkt < 2 || nkt > LS_MAXNKT || (nkt & 1)) return false;
     const ea_rot_jobs r = rj ? *rj : ea_rot_jobs{};

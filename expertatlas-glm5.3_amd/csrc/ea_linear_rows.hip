@@ -18,6 +18,7 @@ namespace ea {
 // 16 bytes that are only 4-byte aligned (a caller's xh), and two fp16 that are only 2-byte aligned (svh, bias)
 typedef u4v u4v_a4 __attribute__((aligned(4)));
 typedef uint32_t u32_a2 __attribute__((aligned(2)));
+typedef const __attribute__((address_space(1))) u4v_a4* gptr_u4;
 
 constexpr int LR_WAVES = 8;
 constexpr int LR_KT = 4;  // k tiles a wave multiplies of each chunk
@@ -38,8 +39,9 @@ __device__ __forceinline__ void lr_put(uint16_t* row, int q8, const u4v& v) {
 // sums are then added in LDS. CW 4: one split, the block holds whole 128-column blocks and finishes them; CW 2: 64-column
 // blocks, twice as many, the sums to Z[split]. ROT: the block rotates its chunk itself while staging it (16 lanes a
 // Hadamard block, fwht128_x8), column group 0 also writing xh; worth it while the rows are few (a block repeats the
-// rotation that every column group needs).
-template <int CB, int K2, int MT, int CW, bool ROT>
+// rotation that every column group needs). FAR: 64-bit trellis offsets, for a caller's k stride (ea_exl3_linear) that 32 bits
+// do not hold or that is negative; 4 % slower, so a build of its own.
+template <int CB, int K2, int MT, int CW, bool ROT, bool FAR>
 __global__ void __launch_bounds__(LR_WAVES * 64) lin_rows_kernel(ea_jobs jobs, ea_rot_jobs rj, int M, int K,
                                                                  const void* __restrict__ x, int x_bf16) {
     constexpr int KW = LR_WAVES / CW, CK = 64 * KW, XS = CK + 8, ROWS = 16 * MT, COLS = 32 * CW;
@@ -80,8 +82,11 @@ __global__ void __launch_bounds__(LR_WAVES * 64) lin_rows_kernel(ea_jobs jobs, e
         for (int i = 0; i < NL; ++i) {
             constexpr int cpr = 2 * K2, last = LR_KT * cpr - 1;
             const int q = min(64 * i + lane, last), t = q / cpr, col = q - t * cpr;
-            tv[i] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(
-                                                trs, min(t0 + t, kt - 1) * kstride + cw * 2 * TW * 4 + col * 16, 0, 0));
+            if constexpr (FAR)
+                tv[i] = *(gptr_u4)(tb + min(t0 + t, kt - 1) * J.stride_k + cw * 2 * TW + col * 4);
+            else
+                tv[i] = __builtin_bit_cast(u4v, __builtin_amdgcn_raw_buffer_load_b128(
+                                                    trs, min(t0 + t, kt - 1) * kstride + cw * 2 * TW * 4 + col * 16, 0, 0));
         }
     };
 
@@ -266,7 +271,7 @@ __global__ void __launch_bounds__(256) lin_finish_kernel(ea_jobs jobs, int M) {
 
 // The jobs of one kind (one split, or several) as one launch of the products: columns a block COLS = 32 CW.
 template <int CB, int K2, int CW>
-static void launch_rows_k2(hipStream_t s, ea_jobs jobs, const ea_rot_jobs& rj, bool rot, int M, int K, const void* x,
+static void launch_rows_k2(hipStream_t s, ea_jobs jobs, const ea_rot_jobs& rj, bool rot, bool far, int M, int K, const void* x,
                            int x_bf16, int cus) {
     int nb = 0;
     for (int i = 0; i < jobs.n; ++i) {
@@ -280,17 +285,19 @@ static void launch_rows_k2(hipStream_t s, ea_jobs jobs, const ea_rot_jobs& rj, b
     int mt = rot ? tiles == 1 || nb * tiles <= cus ? 1 : 2 : CW == 4 ? 4 : 8;
     while (!rot && mt > 1 && (mt / 2 >= tiles || nb * ((tiles + mt - 1) / mt) < cus * 7 / 4)) mt /= 2;
     const auto grid = [&](int t) { return dim3((unsigned)nb, (unsigned)((tiles + t - 1) / t)); };
-#define EA_LR(MT_, ROT_) \
-    lin_rows_kernel<CB, K2, MT_, CW, ROT_><<<grid(MT_), LR_WAVES * 64, 0, s>>>(jobs, rj, M, K, x, x_bf16)
-    if (rot) {
-        if (mt == 1) EA_LR(1, true);
-        else EA_LR(2, true);
+#define EA_LR(MT_, ROT_, FAR_) \
+    lin_rows_kernel<CB, K2, MT_, CW, ROT_, FAR_><<<grid(MT_), LR_WAVES * 64, 0, s>>>(jobs, rj, M, K, x, x_bf16)
+    if (far) {  // not with rot (launch_linear_rows)
+        EA_LR(2, false, true);
+    } else if (rot) {
+        if (mt == 1) EA_LR(1, true, false);
+        else EA_LR(2, true, false);
     } else if (mt <= 2) {
-        EA_LR(2, false);
+        EA_LR(2, false, false);
     } else if (CW == 4 || mt == 4) {
-        EA_LR(4, false);
+        EA_LR(4, false, false);
     } else {
-        if constexpr (CW == 2) EA_LR(8, false);
+        if constexpr (CW == 2) EA_LR(8, false, false);
     }
 #undef EA_LR
 }
@@ -302,12 +309,14 @@ static bool overlap(uint64_t a, size_t an, uint64_t b, size_t bn) { return a < b
 int launch_linear_rows(hipStream_t s, const ea_jobs& jobs, const ea_rot_jobs* rot, int M, int K, uint32_t k2,
                        uint32_t cb, const void* x, int x_dtype) {
     EA_REQUIRE_CTX(c);
+    bool far = false;
+    for (int i = 0; i < jobs.n; ++i) far = far || jobs.j[i].stride_k < 0 || (K >> 4) * jobs.j[i].stride_k >= (1ll << 29);
     // the rotation inside the products while its blocks fit the GPU at once (or the rows one block), a launch of its own
     // above: the shared expert's gate|up (6144 x 256, two jobs) at 64 rows 14.5 -> 11.3 us, 6144 x 2048 at 64 rows 17.2
     // with the launch and 17.8 without
     int blocks = 0;
     for (int i = 0; i < jobs.n; ++i) blocks += jobs.j[i].SK > 1 ? jobs.j[i].N / 64 * jobs.j[i].SK : jobs.j[i].N / 128;
-    bool fuse = rot && (M <= LR_ROT_ROWS || blocks * ((M + LR_ROT_ROWS - 1) / LR_ROT_ROWS) <= c->cus) && (x_dtype == F16 || x_dtype == BF16) &&
+    bool fuse = rot && !far && (M <= LR_ROT_ROWS || blocks * ((M + LR_ROT_ROWS - 1) / LR_ROT_ROWS) <= c->cus) && (x_dtype == F16 || x_dtype == BF16) &&
                 (reinterpret_cast<uintptr_t>(x) & 15) == 0;
     // and x is left alone meanwhile (an output, or xh, in its place: the rotation is done before the products start then)
     const uint64_t xa = reinterpret_cast<uintptr_t>(x);
@@ -336,8 +345,8 @@ int launch_linear_rows(hipStream_t s, const ea_jobs& jobs, const ea_rot_jobs* ro
         if (sj.n == 0) continue;
 #define EA_LV(K2_, CB_)                                                                               \
     if (k2 == K2_ && cb == CB_) {                                                                     \
-        if (split) launch_rows_k2<CB_, K2_, 2>(s, sj, rj, fuse, M, K, x, x_dtype == BF16, c->cus);    \
-        else launch_rows_k2<CB_, K2_, 4>(s, sj, rj, fuse, M, K, x, x_dtype == BF16, c->cus);          \
+        if (split) launch_rows_k2<CB_, K2_, 2>(s, sj, rj, fuse, far, M, K, x, x_dtype == BF16, c->cus);    \
+        else launch_rows_k2<CB_, K2_, 4>(s, sj, rj, fuse, far, M, K, x, x_dtype == BF16, c->cus);          \
     }
         EA_LV(10, 2) EA_LV(12, 2) EA_LV(8, 1) EA_LV(8, 2) EA_LV(6, 1) EA_LV(4, 1)
 #undef EA_LV

@@ -198,6 +198,46 @@ def test_linear_output_in_place_of_the_input(ea, M, K, N, jobs):
     assert device.device_status() == 0
 
 
+def _raw_jobs(specs):
+    """ea_exl3_linear's jobs from dicts of Job fields (device addresses and strides in words)."""
+    from ea_exl3._lib import Jobs
+
+    jobs = Jobs()
+    jobs.n = len(specs)
+    for j, spec in zip(jobs.j, specs):
+        for name, v in spec.items():
+            setattr(j, name, v)
+    return jobs
+
+
+@pytest.mark.parametrize("M,SK", [(5, 1), (40, 2)])
+@pytest.mark.parametrize("stride", [1 << 27, 1 << 20, -(1 << 20)])
+def test_linear_k_strides_of_any_size(ea, M, SK, stride):
+    """ea_exl3_linear takes 64-bit tile strides: k tiles half a gigabyte apart (8 GB in all, past 32-bit offsets) and k
+    tiles laid out backwards."""
+    device, linear, _, _, synth = ea
+    K, N, k2, cb = 256, 128, 8, 1
+    tw, kt = 4 * k2, K // 16
+    T = synth.trellis(600, 0, 0, 0, K, N, k2)
+    svh = synth.scales(601, N, 0.02)
+    xh = synth.f16_bits(np.random.default_rng(602).standard_normal((M, K)))
+    want = orc.exl3_linear(xh, T, 8 * tw, kt * 8 * tw, svh, M, K, N, k2, cb, SK, 2)
+    words = torch.empty(kt * abs(stride), dtype=torch.int32, device="cuda")
+    first = words.data_ptr() + (0 if stride > 0 else (kt - 1) * -stride * 4)
+    tiles = device.upload(T.view(np.int32).reshape(kt, 8 * tw))
+    for t in range(kt):
+        at = t * stride if stride > 0 else (kt - 1 - t) * -stride
+        words[at:at + 8 * tw] = tiles[t]
+    dx, dsv = device.upload(xh), device.upload(svh)
+    z, cnt = device.zeros(SK * M * N, torch.float32), device.zeros(8 * (N // 128), torch.int32)
+    y = device.zeros((M, N), torch.float32)
+    jobs = _raw_jobs([dict(xh=dx.data_ptr(), T=first, stride_k=stride, stride_nb=0, svh=dsv.data_ptr(), bias=0,
+                           y=y.data_ptr(), Z=z.data_ptr() if SK > 1 else 0, counters=cnt.data_ptr(), y_dtype=2, N=N, SK=SK)])
+    linear.Kernels().linear(device.stream(), jobs, M, K, k2, cb, 2)
+    assert_close_rms(device.download(y), want, 1e-4, f"k stride {stride}")
+    assert device.device_status() == 0
+
+
 def test_linear_errors(ea):
     device, linear, _, _, synth = ea
     from ea_exl3._lib import EaError
