@@ -171,11 +171,29 @@ int ea_fini(void) {
 
 namespace ea {
 static std::mutex g_fork_mu;
+
+// The capture a stream takes part in: its status and id (none where the query fails; its error is not a launch's).
+static hipStreamCaptureStatus capture_of(hipStream_t s, unsigned long long& id) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    id = 0;
+    if (hipStreamGetCaptureInfo(s, &st, &id) == hipSuccess) return st;
+    (void)hipGetLastError();
+    return hipStreamCaptureStatusNone;
+}
+
 int fork_join(hipStream_t s, const std::function<int(hipStream_t)>& side_work,
               const std::function<int(hipStream_t)>& main_work) {
     DevCtx* c = ctx();
     if (!c || !c->ready) return EA_NOT_INITIALIZED;
     std::lock_guard<std::mutex> lk(g_fork_mu);
+    // A capture that forked holds the side stream until it ends (only here, under the lock, does one take it): what another
+    // stream launched there would become part of it. A call outside that capture runs both parts on its own stream.
+    unsigned long long own = 0, held = 0;
+    const hipStreamCaptureStatus cs = capture_of(c->side, held);
+    if (cs != hipStreamCaptureStatusNone && (cs != capture_of(s, own) || own != held)) {
+        const int a = side_work(s), b = main_work(s);
+        return a ? a : b;
+    }
     int r = hip_status(hipEventRecord(c->fork, s));
     if (r) return r;
     r = hip_status(hipStreamWaitEvent(c->side, c->fork, 0));

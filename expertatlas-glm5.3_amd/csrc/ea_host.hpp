@@ -30,7 +30,8 @@ struct DevCtx {
 int dl_static_setup(DevCtx& c);
 
 // Run `side_work(side stream)` beside `main_work(s)`: both start after everything already on s, and s waits for
-// both before anything later. Serialised per device (the side stream and events are shared).
+// both before anything later. The side stream and events are shared: calls of several threads enqueue one after the other,
+// and one that finds the side stream held by another capture runs both parts on s, in turn.
 int fork_join(hipStream_t s, const std::function<int(hipStream_t)>& side_work,
               const std::function<int(hipStream_t)>& main_work);
 

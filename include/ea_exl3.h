@@ -194,9 +194,10 @@ int ea_prompt_scratch_init(ea_stream_t stream, ea_prompt_scratch* s, void* base,
 /* out [R, D] fp32 (fp16 with half_sums) = sum over slots of wts * expert(x), rounded through bf16 when do_round.
  * Replaces prompt_experts.run (prompt_experts.zig:146-248). Without a pair plane (s->plane 0) out is 4-byte
  * aligned; half_sums with a plane is EA_INVALID (prompt_experts.zig:155), as is half_sums with do_round (:147). The
- * two item lists run side by side: the call forks one per-device side stream off `stream` with events and joins it back before returning, so the call stays capturable;
- * calls on one device therefore must not run or be captured concurrently from several host threads (the side stream
- * and its events are shared; a mutex orders the forks, not the streams' work). */
+ * two item lists run side by side: the call forks one per-device side stream off `stream` with events and joins it back
+ * before returning, so the call stays capturable. Several host threads may call, or capture, at once, each with its own
+ * scratch and stream: their launches on the side stream follow one another, and while one thread's capture holds the side
+ * stream the calls outside it run the lists in turn on their own stream. */
 int ea_prompt_experts_run(ea_stream_t stream, const void* x, int x_dtype, uint32_t xstride, const int32_t* pick,
                           const float* wts, const ea_routed* ex, const ea_prompt_scratch* s, void* out, uint32_t R,
                           int do_round, int half_sums);

@@ -61,6 +61,83 @@ def test_prefill_graph_replays(ea):
                                                  out.data_ptr(), R, do_round=False), out)
 
 
+@pytest.mark.parametrize("k2", [8, 12])
+def test_prefill_calls_beside_an_open_capture(ea, k2):
+    """While a capture of a prefill pass is open (it holds the library's side stream), an eager pass on another stream and
+    another capture do not become part of it: the eager pass has run, each graph replays its own calls, all with the same
+    bits. The first capture takes a second pass after the others."""
+    import ctypes as C
+
+    from ea_exl3._lib import lib
+
+    device, _, moe, pe, synth = ea
+    R, E, D, I, slots = 130, 48, 512, 256, 8
+    pick = synth.picks_zipf(930, R, 1.1, E, slots)
+    host = synth.HostLayer(931, experts=E, dims=D, width=I, k2=k2, only=np.unique(pick))
+    ex = moe.Routed(host)
+    dx, dp = device.upload(synth.activations(932, R, D, "bf16")), device.upload(pick)
+    dw = device.upload(synth.routing_weights(933, R, slots))
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    scs = [pe.Scratch(ex, R, slots) for _ in range(4)]
+    outs = [device.zeros((R, D), torch.float32) for _ in range(4)]
+
+    def run(i, stream):
+        pe.run(device.stream(stream), dx.data_ptr(), D, dp.data_ptr(), dw.data_ptr(), ex, scs[i], outs[i].data_ptr(), R,
+               do_round=False)
+
+    run(0, torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    want = outs[0].cpu().numpy()
+    for o in outs:
+        o.fill_(float("nan"))
+    torch.cuda.synchronize()
+    L = lib()  # the HIP runtime's own calls, through the library that links it
+
+    def hip(name, *args):
+        assert getattr(L, name)(*args) == 0, name
+
+    def begin(s):
+        hip("hipStreamBeginCapture", C.c_void_p(s.cuda_stream), 2)  # relaxed
+
+    def end(s):
+        g, e = C.c_void_p(), C.c_void_p()
+        hip("hipStreamEndCapture", C.c_void_p(s.cuda_stream), C.byref(g))
+        hip("hipGraphInstantiate", C.byref(e), g, None, None, C.c_size_t(0))
+        return g, e
+
+    a, b, c = streams
+    begin(a)
+    run(0, a)
+    run(1, b)  # eager
+    begin(c)
+    run(2, c)
+    graph_c = end(c)
+    run(3, a)
+    graph_a = end(a)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(outs[1].cpu().numpy(), want)
+    assert all(torch.isnan(outs[i]).all() for i in (0, 2, 3)), "captured passes have not run"
+    for rep in range(2):
+        for (_, e), s, which in ((graph_a, a, (0, 3)), (graph_c, c, (2,))):
+            for o in outs:
+                o.fill_(float("nan"))
+            torch.cuda.synchronize()
+            hip("hipGraphLaunch", e, C.c_void_p(s.cuda_stream))
+            torch.cuda.synchronize()
+            for i in range(4):
+                if i in which:
+                    np.testing.assert_array_equal(outs[i].cpu().numpy(), want, err_msg=f"pass {i}, replay {rep}")
+                else:
+                    assert torch.isnan(outs[i]).all()
+    for g, e in (graph_a, graph_c):
+        hip("hipGraphExecDestroy", e)
+        hip("hipGraphDestroy", g)
+    run(0, torch.cuda.current_stream())  # the side stream is free again
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(outs[0].cpu().numpy(), want)
+    assert device.device_status() == 0
+
+
 @pytest.mark.parametrize("R", [1, 4])
 def test_decode_layer_graph_replays(ea, R):
     device, linear, moe, pe, synth = ea
