@@ -174,11 +174,13 @@ __device__ __forceinline__ u4v cb_quads(const uint32_t (&s)[8]) {
             const uint32_t x = (CB == CB_MCG) ? s[i] * 0xCBAC1FEDu : s[i] * 89226354u + 64248484u;
             y[i] = __builtin_amdgcn_bitop3_b32(x, 0x8FFF8FFFu, 0x3B603B60u, 0x6A);
         }
+        // early clobber: the first halves are written before the second operands are read, so these keep registers of their
+        // own even where the compiler knows that a pair's two states are equal
 #define EA_ADD_LO(r) "v_add_f16_sdwa " r ", " r ", " r " dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:WORD_0 src1_sel:WORD_1\n\t"
 #define EA_ADD_HI(r, b) "v_add_f16_sdwa " r ", " b ", " b " dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:WORD_0 src1_sel:WORD_1\n\t"
         asm(EA_ADD_LO("%0") EA_ADD_LO("%1") EA_ADD_LO("%2") EA_ADD_LO("%3") EA_ADD_HI("%0", "%4") EA_ADD_HI("%1", "%5")
                 EA_ADD_HI("%2", "%6") EA_ADD_HI("%3", "%7") "s_nop 1"
-            : "+v"(y[0]), "+v"(y[2]), "+v"(y[4]), "+v"(y[6])
+            : "+&v"(y[0]), "+&v"(y[2]), "+&v"(y[4]), "+&v"(y[6])
             : "v"(y[1]), "v"(y[3]), "v"(y[5]), "v"(y[7]));
 #undef EA_ADD_LO
 #undef EA_ADD_HI
