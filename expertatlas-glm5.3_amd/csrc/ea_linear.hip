@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(256) lin_rot_in_kernel(const void* __restrict_
         (uint32_t)f2h(v0 * HAD_SCALE) | ((uint32_t)f2h(v1 * HAD_SCALE) << 16);
 }
 
-// ---- the small-row linear: up to 16 rows, K split, every CU busy ----------------------------------------------------
+// ---- the small-row linear: few rows (launch_small), K split, every CU busy ---------------------------------------
 // Block (job, group g of 32 columns, split s) with WK waves: wave w multiplies k tiles [s KS + w NKT, + NKT) of the
 // group's two column tiles (KS = WK NKT, the split's tiles), the trellis staged in LDS by 16-byte loads; the waves'
 // sums are added in order into Z[s] (agent-scope stores), and the last of the 4 SK blocks of a 128-column block to
@@ -44,7 +44,6 @@ __global__ void __launch_bounds__(256) lin_rot_in_kernel(const void* __restrict_
 // round trip for the data. The tag is a signalling-NaN bit pattern: no fp32 result has it (arithmetic quiets NaNs),
 // so partial sums the flag form left in the same buffer are never taken for tagged slots, and Z needs no clearing
 // between the two forms. A Z buffer must not hold the tag when first used (zero, as the counters start, is fine).
-constexpr int LS_MAXR = 16;
 constexpr int LS_MAXNKT = 16;
 constexpr int LS_FLAGS = 32;  // flag bytes a 128-column block has in the counters (int32 [8 N / 128], zero between calls)
 constexpr int LS_MAXTS = 8;   // tagged splits the finisher polls at once (two slots a lane each)
@@ -134,7 +133,7 @@ __global__ void __launch_bounds__(1024) lin_small_kernel(ea_jobs jobs, ea_rot_jo
     constexpr int TW = 4 * K2;
     EA_STAMP(0, threadIdx.x == 0);  // the block's start
     // the tagged form takes the call's rows in passes of LS_PASS side by side (blockIdx.y): rows m0 .. m0 + M - 1 of
-    // M_all; the flag form all of them (at most LS_MAXR) in one
+    // M_all; the flag form all of them (fewer than LS_PASS) in one
     const int m0 = TAG ? (int)blockIdx.y * LS_PASS : 0;
     const int M = TAG ? min(LS_PASS, M_all - m0) : M_all;
     int ji = 0;
@@ -457,8 +456,8 @@ static int small_grid(ea_jobs& sj) {
     return nb;
 }
 
-// The small-row kernel when it applies (few rows, see below; every job split (SK > 1) with the same even per-wave tile count up to
-// 16, a width the staged decode takes, 16-bit activations when rotating); false otherwise, and nothing is launched.
+// The small-row kernel when it applies (few rows, see below; every job split (SK > 1) with the same even per-wave tile count
+// up to 16, a width the staged decode takes, 16-bit activations when rotating); false otherwise, and nothing is launched.
 static bool launch_small(const ea_jobs& jobs, const ea_rot_jobs* rj, hipStream_t s, int M, int K, uint32_t k2,
                          uint32_t cb, int wk, const void* x, int x_dtype, int* status, int cus) {
     if (M > 128 || k2 > (uint32_t)STAGE_MAXK2) return false;
@@ -494,7 +493,7 @@ static bool launch_small(const ea_jobs& jobs, const ea_rot_jobs* rj, hipStream_t
     for (int i = 0; i < jobs.n; ++i) one = one && jobs.j[i].SK == 2;
     const int passes = (M + LS_PASS - 1) / LS_PASS;
     const bool few = tag && (one ? tb * passes <= cus : tb * passes < cus / 2);
-    if (M >= (tag && tb > cus ? 4 : 8) && !few) return false;
+    if (M >= (tag && tb > cus ? 4 : LS_PASS) && !few) return false;
     // the tagged form on sixteen waves a block (four a SIMD) when its waves' k tiles halve evenly once more: the
     // same decode over twice the waves (config 1: 8.64 -> 8.55 us)
     int tw = 2 * wk, tn = nkt;
@@ -502,18 +501,19 @@ static bool launch_small(const ea_jobs& jobs, const ea_rot_jobs* rj, hipStream_t
         tw *= 2;
         tn /= 2;
     }
-    // the tagged form on sixteen waves; above LS_MAXR rows, when its block's LDS is too large for a pass's rows, on
-    // eight; the flag form up to LS_MAXR rows; otherwise not this kernel
+    // the tagged form on sixteen waves; from a whole pass of rows on, when its block's LDS is too large for them, on eight;
+    // the flag form below a pass (1792 x 256 at 12 rows: 15.7 us with it, 10.9 with the kernel for more rows); otherwise not
+    // this kernel
 #define EA_SV(K2_, CB_)                                                                                            \
     if (k2 == K2_ && cb == CB_) {                                                                                  \
         if (tag && (rj ? launch_small_k2<CB_, K2_, true, true>(tj, r, tb, s, M, K, tw, tn, x, bf, status)          \
                        : launch_small_k2<CB_, K2_, false, true>(tj, r, tb, s, M, K, tw, tn, x, bf, status)))       \
             return true;                                                                                           \
-        if (tag && M > LS_MAXR && tw != 2 * wk &&                                                                  \
+        if (tag && M >= LS_PASS && tw != 2 * wk &&                                                                 \
             (rj ? launch_small_k2<CB_, K2_, true, true>(tj, r, tb, s, M, K, 2 * wk, nkt, x, bf, status)            \
                 : launch_small_k2<CB_, K2_, false, true>(tj, r, tb, s, M, K, 2 * wk, nkt, x, bf, status)))         \
             return true;                                                                                           \
-        if (M > LS_MAXR) return false;                                                                             \
+        if (M >= LS_PASS) return false;                                                                            \
         return rj ? launch_small_k2<CB_, K2_, true, false>(sj, r, nb, s, M, K, wk, nkt, x, bf, status)             \
                   : launch_small_k2<CB_, K2_, false, false>(sj, r, nb, s, M, K, wk, nkt, x, bf, status);           \
     }

@@ -51,24 +51,28 @@ def test_config1_linear_6144x2048_one_row(ea):
     assert device.device_status() == 0
 
 
-def test_config1_linear_flag_and_tagged_forms_share_z(ea):
-    """16 rows take the flag form (fp32 partial sums left in Z), then 1 and 4 rows the tagged form on the same Z: the
-    stale partial sums are never taken for tagged slots (the tag is a NaN pattern no fp32 result has)."""
+@pytest.mark.parametrize("K,N,k2,cb,rows", [
+    (6144, 2048, 8, 1, (16, 1, 4, 16, 1)),     # 16 rows: the kernel for more rows; 1 and 4: the tagged form
+    (1792, 256, 10, 2, (7, 1, 16, 7, 17, 1)),  # 7 rows: the flag form (the tagged block's LDS is too large for them)
+    (16384, 128, 8, 1, (7, 1, 9, 3)),          # 32 splits: the flag form with a counter; 9: the kernel for more rows
+])
+def test_linear_forms_share_z(ea, K, N, k2, cb, rows):
+    """The kernels that leave fp32 partial sums in Z (the flag form, and the one for more rows) and the tagged form on one
+    Z in turn: stale partial sums are never taken for tagged slots (the tag is a NaN pattern no fp32 result has)."""
     device, linear, _, _, synth = ea
-    K, N, k2, cb = 6144, 2048, 8, 1
     T = synth.trellis(1011, 0, 0, 0, K, N, k2)
     suh, svh = synth.scales(1012, K, 1.0), synth.scales(1013, N, 0.02)
     lin = linear.Linear(T, suh, svh, K, N, k2, cb)
     tw = 4 * k2
-    sc = linear.Scratch(16, K, lin.sk * 16 * N)
-    for M in (16, 1, 4, 16, 1):
+    sc = linear.Scratch(max(rows), K, lin.sk * max(rows) * N)
+    for M in rows:
         x = synth.activations(1014 + M, M, K, "f16")
         want = orc.exl3_linear(orc.exl3_rot_in(x, suh, M, K), linear.strips(T, K, N, k2), 8 * tw, (K // 16) * 8 * tw,
                                svh, M, K, N, k2, cb, lin.sk, lin.wk, y_dtype=2)
         dx = device.upload(x)
         y = device.zeros((M, N), torch.float32)
         linear.call(device.stream(), sc, [lin], dx.data_ptr(), 0, M, [y.data_ptr()], [2])
-        assert_close_rms(device.download(y), want, 1e-4, f"config 1 shape, {M} rows after other row counts")
+        assert_close_rms(device.download(y), want, 1e-4, f"{K} x {N}, {M} rows after other row counts")
         assert int(device.download(lin.counters).sum()) == 0
     assert device.device_status() == 0
 

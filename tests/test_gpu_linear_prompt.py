@@ -210,6 +210,44 @@ def _raw_jobs(specs):
     return jobs
 
 
+@pytest.mark.parametrize("M", [1, 7, 8, 40])
+@pytest.mark.parametrize("K,wk,jobs", [
+    (768, 4, ((256, 3, True),)),                                # an odd split count: the flag form below eight rows
+    (512, 8, ((128, 2, False), (384, 2, True))),                # eight waves a split: likewise
+    (512, 2, ((256, 1, True), (128, 4, True), (384, 1, False))),  # jobs of one split and of several in one call
+    (256, 2, ((128, 1, False), (256, 2, True))),
+])
+def test_linear_bias_and_mixed_splits(ea, M, K, wk, jobs):
+    """ea_exl3_linear with a bias, split counts that no plan gives, and jobs of one and of several K splits in one call."""
+    device, linear, _, _, synth = ea
+    k2, cb = 8, 1
+    tw = 4 * k2
+    xh = synth.f16_bits(np.random.default_rng(620 + M).standard_normal((M, K)))
+    dx = device.upload(xh)
+    specs, wants, outs, keep = [], [], [], [dx]
+    for i, (N, SK, biased) in enumerate(jobs):
+        T = synth.trellis(621 + i, 0, 0, 0, K, N, k2)
+        svh = synth.scales(622 + i, N, 0.02)
+        bias = synth.scales(623 + i, N, 0.5) if biased else None
+        strips = linear.strips(T, K, N, k2)
+        wants.append(orc.exl3_linear(xh, strips, 8 * tw, (K // 16) * 8 * tw, svh, M, K, N, k2, cb, SK, wk, bias=bias))
+        t, sv, z = device.upload(strips), device.upload(svh), device.zeros(SK * M * N, torch.float32)
+        cnt, y = device.zeros(8 * (N // 128), torch.int32), device.zeros((M, N), torch.float32)
+        b = device.upload(bias) if biased else None
+        keep += [t, sv, z, b, cnt]
+        outs.append((y, cnt))
+        specs.append(dict(xh=dx.data_ptr(), T=t.data_ptr(), stride_k=8 * tw, stride_nb=(K // 16) * 8 * tw, svh=sv.data_ptr(),
+                          bias=b.data_ptr() if biased else 0, y=y.data_ptr(), Z=z.data_ptr() if SK > 1 else 0,
+                          counters=cnt.data_ptr(), y_dtype=2, N=N, SK=SK))
+    for rep in range(2):
+        linear.Kernels().linear(device.stream(), _raw_jobs(specs), M, K, k2, cb, wk)
+        for (y, cnt), want in zip(outs, wants):
+            assert_close_rms(device.download(y), want, 1e-4, f"M={M} rep {rep}")
+            assert int(device.download(cnt).sum()) == 0
+            y.fill_(float("nan"))
+    assert device.device_status() == 0
+
+
 @pytest.mark.parametrize("M,SK", [(5, 1), (40, 2)])
 @pytest.mark.parametrize("stride", [1 << 27, 1 << 20, -(1 << 20)])
 def test_linear_k_strides_of_any_size(ea, M, SK, stride):
