@@ -454,11 +454,6 @@ __global__ void __launch_bounds__(DL_ROUTE_THREADS) route_kernel(DLArgs a) {
 
 // ---- the MFMA core of an item ------------------------------------------------------------------------------------
 
-// Where word d (values 2 d, 2 d + 1) of a row of staged activations goes: within each 32-k step (16 words) to 4 (d & 3) +
-// (d >> 2), so that a lane's MFMA operand of the step (words g, g + 4, g + 8, g + 12: the k order of the decoded quads) is
-// one 16-byte read.
-__device__ __forceinline__ int a_word(int d) { return (d & ~15) + 4 * (d & 3) + ((d >> 2) & 3); }
-
 // The wave's two column tiles times the activation rows in xs (laid out by a_word) over NKT k tiles: acc[j] += A (rows of
 // xs, the MFMA's 16 rows; rows past the unit's members hold zeros) x B (tile pair (t, t + 1) of column tile j). The tiles'
 // words are staged in LDS (st: tile (t, j) at word (2 t + j) * 4 K2); each lane reads the two words its four values come

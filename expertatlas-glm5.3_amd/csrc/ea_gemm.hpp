@@ -46,13 +46,6 @@ struct TileLane {
         w[1] = gload(tile + w1);
         if constexpr (NW == 3) w[2] = gload(tile + w2);
     }
-    // The same through a buffer resource: the tile starts `soff` bytes into it (a scalar offset), so the addressing
-    // costs no vector registers beyond the lane's word offsets.
-    __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t r, int soff, uint32_t (&w)[NW]) const {
-        w[0] = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * w0, soff, 0);
-        w[1] = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * w1, soff, 0);
-        if constexpr (NW == 3) w[2] = __builtin_amdgcn_raw_buffer_load_b32(r, 4 * w2, soff, 0);
-    }
     // The same from LDS.
     __device__ __forceinline__ void staged(const uint32_t* tile, uint32_t (&w)[NW]) const {
         w[0] = tile[w0];
@@ -99,6 +92,34 @@ __device__ __forceinline__ h4v load_a4(const uint16_t* __restrict__ xrow, int k0
     const uint16_t* xk = xrow + k0 + 2 * ((lane >> 4) & 3);
     const u2v au = {*reinterpret_cast<const uint32_t*>(xk), *reinterpret_cast<const uint32_t*>(xk + 8)};
     return __builtin_bit_cast(h4v, au);
+}
+
+// Where word d (values 2 d, 2 d + 1) of a row of activations staged in LDS goes: within each 32-k step (16 words) to
+// 4 (d & 3) + (d >> 2), so that a lane's MFMA operand of the step (words g, g + 4, g + 8, g + 12: the k order of the decoded
+// quads) is one 16-byte read.
+__device__ __forceinline__ int a_word(int d) { return (d & ~15) + 4 * (d & 3) + ((d >> 2) & 3); }
+
+// An activation piece (8 values: columns 8 q8 .. + 7 of the row) to its places in LDS.
+__device__ __forceinline__ void put_a(uint16_t* row, int q8, const u4v& v) {
+    uint32_t* w = reinterpret_cast<uint32_t*>(row) + 16 * (q8 >> 2) + (q8 & 3);  // a_word(4 q8)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w[4 * r] = v[r];
+}
+
+// Eight values of a 128-k block rotated (16 lanes a block, lane l the values 8 h8_group(l) .. + 7): x (16-bit) * suh through
+// the Hadamard butterflies in the order of rot_in_kernel, rounded to fp16.
+__device__ __forceinline__ u4v rot8(const u4v& x, const u4v& suh, int bf16, int lane) {
+    float f[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint16_t h = (uint16_t)(x[j >> 1] >> (16 * (j & 1)));
+        f[j] = (bf16 ? bf2f(h) : h2f(h)) * h2f((uint16_t)(suh[j >> 1] >> (16 * (j & 1))));
+    }
+    const float sc = fwht128_x8(f, lane) * HAD_SCALE;  // the values' sign folded into the scale (exact)
+    u4v v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = f2h2(__builtin_fmaf(f[2 * j], sc, 0.f), __builtin_fmaf(f[2 * j + 1], sc, 0.f));
+    return v;
 }
 
 // acc[m][j] += rows(m) @ tiles: tile (t, j) of the strip at base + t * kstride + j * TW words for t in [0, nkt);

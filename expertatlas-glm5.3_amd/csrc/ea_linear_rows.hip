@@ -23,15 +23,6 @@ typedef const __attribute__((address_space(1))) u4v_a4* gptr_u4;
 constexpr int LR_WAVES = 8;
 constexpr int LR_KT = 4;  // k tiles a wave multiplies of each chunk
 
-// An activation piece (8 halves, columns 8 q8 .. +7 of a chunk row) into LDS: within each 32-k step (16 words) word d goes
-// to 4 (d & 3) + (d >> 2), so a lane's MFMA operand (words g, g + 4, g + 8, g + 12: the k order of the decoded quads) is
-// one 16-byte read.
-__device__ __forceinline__ void lr_put(uint16_t* row, int q8, const u4v& v) {
-    uint32_t* w = reinterpret_cast<uint32_t*>(row) + 16 * (q8 >> 2) + (q8 & 3);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) w[4 * r] = v[r];
-}
-
 // Block (job, group g of 32 CW columns, split; rows m0 = 16 MT blockIdx.y .. + 16 MT - 1) of eight waves: CW column waves
 // of two column tiles each times KW = 8 / CW k waves. The split's k range is walked in chunks of 64 KW: the rows' chunk
 // staged in LDS for all waves (row tiles past the call's rows are skipped, rows past it repeat the last row and are not
@@ -125,21 +116,12 @@ __global__ void __launch_bounds__(LR_WAVES * 64) lin_rows_kernel(ea_jobs jobs, e
             const int kk = c * CK + 8 * pq;
             u4v v = av[i];
             if constexpr (ROT) {
-                float f[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const uint16_t h = (uint16_t)(v[j >> 1] >> (16 * (j & 1)));
-                    f[j] = (x_bf16 ? bf2f(h) : h2f(h)) * h2f((uint16_t)(sv[j >> 1] >> (16 * (j & 1))));
-                }
-                const float sc = fwht128_x8(f, lane) * HAD_SCALE;  // the values' sign folded into the scale (exact)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    v[j] = f2h2(__builtin_fmaf(f[2 * j], sc, 0.f), __builtin_fmaf(f[2 * j + 1], sc, 0.f));
+                v = rot8(v, sv, x_bf16, lane);
                 if (g == 0 && xh && kk < kn && prow < rows)
                     *reinterpret_cast<u4v*>(xh + (size_t)(m0 + prow) * K + lo + kk) = v;
             }
             if (kk >= kn) v = u4v{0u, 0u, 0u, 0u};
-            if (PIECES % (LR_WAVES * 64) == 0 || prow < ROWS) lr_put(xa + prow * XS, pq, v);
+            if (PIECES % (LR_WAVES * 64) == 0 || prow < ROWS) put_a(xa + prow * XS, pq, v);
         }
     };
 

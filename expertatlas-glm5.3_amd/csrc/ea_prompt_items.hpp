@@ -55,7 +55,7 @@ constexpr int PW = 4;                             // waves a block: 8 column til
 constexpr int pstage(int mk) { return PK * 2 * 4 * mk; }  // a wave's staged trellis words a chunk
 constexpr int DNG = 16;  // down matrix: column blocks of 128 a block, small items (8, 24 and 48 measured slower at 512 rows)
 // the same in a decode window, whose items are too few to fill the GPU with blocks that long (37 rows, 112 experts: 336
-// blocks of 16 column blocks took 71 us, 1,344 of 4 take 39)
+// blocks of 16 column blocks took 71 us, 1,344 of 4 take 39; passes of 129 to 511 rows were not measured with 4)
 constexpr int DNG_WINDOW = 4;
 constexpr int WINDOW_ROWS_MAX = 128;  // the widest decode window (forward.zig:21)
 constexpr int DNG_BIG = 2;  // the same for the larger items: more blocks for fewer items (4: 1 % slower at 512 rows)
@@ -63,7 +63,8 @@ constexpr int DNG_BIG_LONG = 4;   // passes of more than LONG_ROWS rows: 1.5 % f
 constexpr int LONG_ROWS = 1024;
 // Rows a pass up to which the larger items' gate|up stages its activations in two buffers (two blocks a CU), above which in
 // one (four). 300 rows 254 us with two and 282 with one, 512 rows 306 and 315, 640 rows 351 and 347, 1024 rows 447 and 423:
-// few blocks wait on each chunk's round trip, many on each other for a place.
+// few blocks wait on each chunk's round trip, many on each other for a place. (Rows of 8 slots over 256 experts, as for the
+// other row counts here.)
 constexpr int MID_ROWS = 600;
 constexpr int GU_SPLIT = 2;                       // K splits of a larger item's gate|up (4 and 8 measured slower)
 // The number of K splits of an item's gate|up over K (at most one a chunk). A layer that holds a width above 10 keeps one sum
@@ -73,15 +74,6 @@ static int gu_splits(int K, bool wide = false) {
     return wide ? 1 : K / (PK * 16) < GU_SPLIT ? K / (PK * 16) : GU_SPLIT;
 }
 constexpr int DXS = 2 * PK * 16 + 8;              // down matrix: LDS row stride of the activations (K up to 256)
-
-// An activation piece (8 halves: column 8 q8 .. +7 of a chunk row) into LDS. Within each 32-k step of the row
-// (16 words) word d goes to 4 (d & 3) + (d >> 2), so the words of a lane's MFMA operand (g, g + 4, g + 8, g + 12 of
-// the step: the k order in which the trellis quads fill the B operand) are one 16-byte read.
-__device__ __forceinline__ void put_a(uint16_t* row, int q8, const u4v& v) {
-    uint32_t* w = reinterpret_cast<uint32_t*>(row) + 16 * (q8 >> 2) + (q8 & 3);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) w[4 * r] = v[r];
-}
 
 // One chunk (PK k tiles) of a wave: its two column tiles times the item's first mts (<= MT) row tiles. The trellis
 // words are staged in st (tile (t, j) at word (2 t + j) * 4 K2), the activations in xa (row stride xs halves, laid
@@ -224,18 +216,7 @@ __device__ __forceinline__ void gu_loop(const GuSrc& src, const uint32_t (&aoff)
             const int row = i * (NT / 16) + row0;
             if (row >= rows) continue;  // uniform over a wave (rows % 16 == 0)
             u4v v = av[i];
-            if constexpr (ROT) {
-                float f[8];
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const uint16_t h = (uint16_t)(v[j >> 1] >> (16 * (j & 1)));
-                    f[j] = (src.bf16 ? bf2f(h) : h2f(h)) * h2f((uint16_t)(sv[j >> 1] >> (16 * (j & 1))));
-                }
-                const float sc = fwht128_x8(f, lane) * HAD_SCALE;  // the values' sign folded into the scale (exact)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    v[j] = f2h2(__builtin_fmaf(f[2 * j], sc, 0.f), __builtin_fmaf(f[2 * j + 1], sc, 0.f));
-            }
+            if constexpr (ROT) v = rot8(v, sv, src.bf16, lane);
             put_a(buf + row * PXS, q8, v);
         }
     };
@@ -564,18 +545,7 @@ static __global__ void __launch_bounds__(256) item_rot_kernel(const uint16_t* __
 #pragma unroll
         for (int i = 0; i < QB; ++i) {
             if (i0 + i >= cnt) break;  // uniform
-            float f[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint16_t h = (uint16_t)(xv[i][j >> 1] >> (16 * (j & 1)));
-                f[j] = (x_bf16 ? bf2f(h) : h2f(h)) * h2f((uint16_t)(sv[j >> 1] >> (16 * (j & 1))));
-            }
-            const float sc = fwht128_x8(f, lane) * HAD_SCALE;  // the values' sign folded into the scale (exact)
-            u4v w;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                w[j] = f2h2(__builtin_fmaf(f[2 * j], sc, 0.f), __builtin_fmaf(f[2 * j + 1], sc, 0.f));
-            *reinterpret_cast<u4v*>(out + (size_t)p[i] * K + k) = w;
+            *reinterpret_cast<u4v*>(out + (size_t)p[i] * K + k) = rot8(xv[i], sv, x_bf16, lane);
         }
     }
 }

@@ -1,8 +1,8 @@
 """HIP graph capture of the library's calls through torch.cuda.CUDAGraph: a prefill pass (its two item lists fork
 onto the library's second stream and join back with events, so the capture follows the fork), the decode layer (one
 launch at one row, five at four), moe.routed on a 40-row window (the prefill path in the scratch's prompt region) and
-the EXL3 linear at one row (the tagged split-K slots, zeroed by each call's finisher) and at 40 rows (the per-pass
-counters, reset by each call's last block). Each is captured once after an eager warm-up and replayed several times,
+the EXL3 linear at one row (the tagged split-K slots, zeroed by each call's finisher) and at 40 rows (the products and
+their finish). Each is captured once after an eager warm-up and replayed several times,
 with eager work and synchronizations between the replays; every replay must give the eager result bit for bit (both
 paths are deterministic: splits and slots are summed in a fixed order)."""
 import numpy as np

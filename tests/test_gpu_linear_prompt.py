@@ -44,14 +44,14 @@ def test_unpack_bit_exact(ea, k2, cb):
     (1, 6144, 256, 8, 1, 1),     # the shared expert's gate / up at batch 1 (plan: SK 8, WK 4), bf16 out
     (1, 256, 6144, 8, 1, 2),     # its down (SK 1), fp32 out
     (16, 6144, 256, 10, 2, 2),   # 5-bit mul1 (the real checkpoints' shared expert), 16 rows
-    (40, 1024, 640, 8, 2, 0),    # three row passes, fp16 out
+    (40, 1024, 640, 8, 2, 0),    # five row passes of the tagged form (few blocks), fp16 out
     (128, 512, 384, 6, 1, 2),    # the most rows a call takes
-    (128, 6144, 256, 8, 1, 1),   # the shared expert's gate / up on a 128-row window: 8 row passes x 8 K splits at once
+    (128, 6144, 256, 8, 1, 1),   # the shared expert's gate / up on a 128-row window
     (96, 256, 6144, 8, 1, 2),    # its down on a 96-row window
     (4, 6144, 2048, 8, 1, 2),    # config 1's shape at four rows (the small-row kernel: 32-column groups x 8 splits)
     (7, 2048, 512, 6, 1, 0),     # 3 bits, fp16 out, a ragged row count
     (2, 1024, 384, 4, 1, 2),     # 2 bits
-    (3, 2048, 512, 12, 2, 2),    # 6-bit mul1 (widths above 10: the register-streaming kernel at any row count)
+    (3, 2048, 512, 12, 2, 2),    # 6-bit mul1 (widths above 10: the kernel for more rows at any row count)
     (5, 1024, 384, 8, 2, 1),     # 4-bit mul1, bf16 out
     (1, 8192, 256, 8, 1, 2),     # SK 16: the tagged finisher polls eight splits
     (3, 8192, 512, 6, 1, 1),     # the same at three rows, 3 bits, bf16 out
@@ -313,13 +313,13 @@ def _prompt_case(ea, R, E, D, I, k2, seed, x_dtype=1, zipf=True, cb=1, planes=Tr
 
 @pytest.mark.parametrize("R,E,D,I,k2", [(130, 64, 512, 256, 8), (300, 256, 1024, 256, "mixed"), (40, 32, 256, 128, 6),
                                         (120, 32, 256, 128, 12), (300, 32, 256, 128, 12), (300, 32, 256, 128, 8),
-                                        # widths above 10 take the register-streaming GEMM with items of up to 112
-                                        # pairs; Zipf over 32 experts gives the top experts ~300 pairs: three items
+                                        # widths above 10; Zipf over 32 experts gives the top experts ~300 pairs: four
+                                        # items of up to 80
                                         (300, 32, 256, 128, 11), (300, 32, 256, 128, 14), (300, 32, 256, 128, 16),
                                         (260, 32, 512, 256, "wide-mixed")])
 def test_prompt_experts_run(ea, R, E, D, I, k2):
     device, _, _, pe, synth = ea
-    if k2 == "wide-mixed":  # every width class on the register-streaming path at once
+    if k2 == "wide-mixed":  # two and three trellis words a lane in one layer
         k2v = np.array([(12, 8, 6, 16, 10, 11, 4, 14)[e % 8] for e in range(E)], np.int32)
     else:
         k2v = synth.mixed_widths(5, E) if k2 == "mixed" else k2
@@ -467,6 +467,30 @@ def test_prompt_experts_long_pass_rotations(ea, x_dtype, pad, planes):
     assert device.device_status() == 0
 
 
+def test_prompt_experts_second_chunk(ea):
+    """More than 4,096 rows: the second chunk of rows takes the same scratch after the first. With and without the pair plane
+    (whose down rows then lie where the second chunk's rotated inputs go) the same bits, and those of the second chunk's
+    rows in a call of their own."""
+    device, _, _, pe, synth = ea
+    R, E, D, I, cut = 4300, 32, 256, 128, 4096
+    host, ex, sc, x, pick, wts, dx, dp, dw = _prompt_case(ea, R, E, D, I, 8, 640, planes=False)
+    got = []
+    for s in (sc, pe.Scratch(ex, R, 8, planes=True)):
+        out = device.zeros((R, D), torch.float32)
+        pe.run(device.stream(), dx.data_ptr(), D, dp.data_ptr(), dw.data_ptr(), ex, s, out.data_ptr(), R, do_round=False)
+        got.append(device.download(out))
+    np.testing.assert_array_equal(got[0], got[1])
+    tail = device.zeros((R - cut, D), torch.float32)
+    pe.run(device.stream(), dx.data_ptr() + cut * D * 2, D, dp.data_ptr() + cut * 32, dw.data_ptr() + cut * 32, ex, sc,
+           tail.data_ptr(), R - cut, do_round=False)
+    np.testing.assert_array_equal(device.download(tail), got[0][cut:])
+    rows = np.concatenate([np.arange(0, R, 16), [cut - 1, cut, R - 1]])
+    want = orc.prompt_experts(np.ascontiguousarray(x[rows]), np.ascontiguousarray(pick[rows]), np.ascontiguousarray(wts[rows]),
+                              oracle_routed(host), len(rows), 8, bf16=True)
+    assert_close_rms(got[0][rows], want, 2e-3, "two chunks (sampled rows)")
+    assert device.device_status() == 0
+
+
 @pytest.mark.parametrize("planes", [True, False])
 def test_prompt_experts_f32_activations(ea, planes):
     """fp32 activations (x_dtype 2: the rotation launch reads them and rounds the rotated rows to fp16 as for 16-bit
@@ -486,8 +510,8 @@ def test_prompt_experts_f32_activations(ea, planes):
 
 @pytest.mark.parametrize("cb,I", [(0, 256), (2, 256), (2, 128), (0, 128)])
 def test_prompt_experts_codebooks(ea, cb, I):
-    """3inst and mul1 through both item lists (the small items' ring kernel and the larger items' kernel), both
-    ring widths (8 waves at I = 256, 4 at I = 128)."""
+    """3inst and mul1 through both item lists (the small items' ring kernel and the larger items' kernel), one and two
+    column blocks of 128 in the intermediate."""
     device, _, _, pe, synth = ea
     R, E, D = 160, 48, 512
     host, ex, sc, x, pick, wts, dx, dp, dw = _prompt_case(ea, R, E, D, I, 8, 500 + cb + I, cb=cb)
@@ -499,7 +523,7 @@ def test_prompt_experts_codebooks(ea, cb, I):
 
 
 def test_prompt_unaligned_output_same_bits(ea):
-    """An output 4 bytes off a 16-byte boundary takes the scalar combine: the same bits as the vector one."""
+    """An output 4 bytes off a 16-byte boundary is stored 4 bytes at a time: the same bits as 16 at a time."""
     device, _, _, pe, synth = ea
     R, D = 40, 512
     host, ex, sc, x, pick, wts, dx, dp, dw = _prompt_case(ea, R, 32, D, 128, 8, 400)
@@ -513,10 +537,9 @@ def test_prompt_unaligned_output_same_bits(ea):
 
 
 def test_prompt_half_sums_and_invalid(ea):
-    """half_sums is the reference's mode 1: no pair plane, each slot added into the fp16 out as packed fp16 atomics
-    (prompt_experts.zig:150-155, prompt_experts.cu:785-797). Refused with rounding (prompt_experts.zig:147) and with a
-    pair plane (:155). fp16 sums of 8 slots: each slot's value is rounded to fp16 and every add rounds, so the bar is
-    1e-2 * RMS here (2e-3 for the fp32 modes)."""
+    """half_sums is the reference's mode 1: no pair plane, an fp16 out (prompt_experts.zig:150-155, prompt_experts.cu:785-797,
+    which adds each slot into it; here the fp32 sum of the slots is rounded once). Refused with rounding
+    (prompt_experts.zig:147) and with a pair plane (:155). The bits are those of the fp32 output rounded to fp16."""
     device, _, _, pe, synth = ea
     from ea_exl3._lib import EaError
 
@@ -536,22 +559,23 @@ def test_prompt_half_sums_and_invalid(ea):
     pick2[0, 3] = -1  # a slot that is not an expert adds nothing
     want = orc.prompt_experts(x, pick2, wts, oracle_routed(host), R, 8, bf16=True)
     h = device.zeros((R, D), torch.float16)
-    h.fill_(7.0)  # the pass clears its rows of out before the slots are added
+    h.fill_(7.0)  # what out holds does not matter
     dp2 = device.upload(pick2)
     pe.run(device.stream(), dx.data_ptr(), D, dp2.data_ptr(), dw.data_ptr(), ex, sc, h.data_ptr(), R,
            do_round=False, half_sums=True)
-    got = device.download(h).view(np.float16).astype(np.float32)
-    assert_close_rms(got, want, 1e-2, "half sums (fp16 atomics)")
+    pe.run(device.stream(), dx.data_ptr(), D, dp2.data_ptr(), dw.data_ptr(), ex, sc, out.data_ptr(), R, do_round=False)
+    full = device.download(out)
+    assert_close_rms(full, want, 2e-3, "fp32 sums, no plane, a slot without an expert")
+    np.testing.assert_array_equal(device.download(h).view(np.uint16), synth.f16_bits(full))
     assert device.device_status() == 0
 
 
 @pytest.mark.parametrize("R,E,D,I,k2", [(130, 64, 512, 256, 8), (300, 256, 1024, 256, "mixed"), (40, 32, 256, 128, 6),
                                         (300, 32, 256, 128, 12), (260, 32, 512, 256, "wide-mixed")])
 def test_prompt_experts_no_plane(ea, R, E, D, I, k2):
-    """planes = 0, the reference's default mode 0: no pair plane and no combine; the down items add each pair's slot
-    into out with fp32 atomics in arrival order (bits may differ run to run). Both item lists, the staged and the
-    register-streaming (widths above 10) down GEMMs; out starts dirty and is cleared by the pass; do_round rounds the
-    sums through bf16. Every run meets the oracle's bar and the planes-1 output's."""
+    """planes = 0, the reference's default mode 0: no pair plane, the pairs' down rows over their rotated inputs. Both item
+    lists, widths up to 10 and above; out starts dirty; do_round rounds the sums through bf16. Every run meets the oracle's
+    bar and gives the bits of planes 1 (the same products, the slots added in the same order)."""
     device, _, _, pe, synth = ea
     if k2 == "wide-mixed":
         k2v = np.array([(12, 8, 6, 16, 10, 11, 4, 14)[e % 8] for e in range(E)], np.int32)
@@ -571,7 +595,7 @@ def test_prompt_experts_no_plane(ea, R, E, D, I, k2):
                do_round=False)
         got = device.download(out)
         assert_close_rms(got, want, 2e-3, f"prompt experts, no plane, run {rep}")
-        assert_close_rms(got, device.download(ref), 2e-3, f"no plane against the plane, run {rep}")
+        np.testing.assert_array_equal(got, device.download(ref), err_msg=f"no plane against the plane, run {rep}")
     pe.run(device.stream(), dx.data_ptr(), D, dp.data_ptr(), dw.data_ptr(), ex, sc, out.data_ptr(), R, do_round=True)
     r = device.download(out)
     np.testing.assert_array_equal(r, synth.bf16_to_f32(synth.bf16_bits(r)))  # every value a bf16
