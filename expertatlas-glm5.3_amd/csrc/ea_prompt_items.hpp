@@ -68,8 +68,9 @@ constexpr int LONG_ROWS = 1024;
 constexpr int MID_ROWS = 600;
 constexpr int GU_SPLIT = 2;                       // K splits of a larger item's gate|up (4 and 8 measured slower)
 // The number of K splits of an item's gate|up over K (at most one a chunk). A layer that holds a width above 10 keeps one sum
-// over all of K in ascending order: two splits change its bits and measured no faster (777 rows of 5, 6 and 8 bits: 428 us
-// with one, 430 with two).
+// over all of K in ascending order, the order of the sums it has always had; two splits would round its outputs differently
+// (2e-4 of them, after the bf16 rounding). 5, 6 and 8 bits with one / two: windows of 37 / 128 rows 172 / 146 and 206 / 192 us,
+// prompts of 512, 777 and 2048 rows 368 / 375, 428 / 430 and 752 / 721.
 static int gu_splits(int K, bool wide = false) {
     return wide ? 1 : K / (PK * 16) < GU_SPLIT ? K / (PK * 16) : GU_SPLIT;
 }

@@ -224,7 +224,9 @@ typedef struct ea_rot_jobs {
  * (exl3.zig:78-91; exl3_linear.cu:152-173). */
 int ea_exl3_rot_in(ea_stream_t stream, const void* x, int x_dtype, const ea_rot_jobs* jobs, uint32_t njobs,
                    uint32_t m, uint32_t kdim);
-/* One launch over `jobs`. Replaces exl3.Kernels.linear (exl3.zig:95-121; exl3_linear.cu:231-484). */
+/* y_j = xh_j @ W_j for 1..3 jobs of up to 128 rows: one launch for few rows, else the products and, for jobs of several K
+ * splits, a launch that adds them. T's strides may be of any size and sign. Replaces exl3.Kernels.linear (exl3.zig:95-121;
+ * exl3_linear.cu:231-484). */
 int ea_exl3_linear(ea_stream_t stream, const ea_jobs* jobs, uint32_t m, uint32_t kdim, uint32_t k2, uint32_t cb,
                    uint32_t wk, uint32_t loads);
 
@@ -234,9 +236,10 @@ typedef struct ea_linear {
     uint32_t k, n, k2, cb, sk, wk;
 } ea_linear;
 /* linear.zig:142-154 Scratch: xh fp16 [M, K] and z fp32 [SK, M, N] a layer. z must not hold the small-row kernel's
- * tag when first used (zero it once at allocation, as the counters are): calls of up to about 8 rows, and of 17 to 128
- * rows (in passes of 8), with an even split count hand their partial sums over in z as tagged 8-byte slots and leave
- * every slot they used zero. Two calls
+ * tag when first used (zero it once at allocation, as the counters are): calls of few rows (fewer than 8, or more where
+ * few blocks are needed) with an even split count hand their partial sums over in z as tagged 8-byte slots and leave
+ * every slot they used zero; all others leave fp32 partial sums there. No call needs z cleared after another: a partial
+ * sum never holds the tag. Two calls
  * that run at once on one z race, as in the reference. A call whose status word then reads EA_SYNC_TIMEOUT (a
  * split's block never stored its slot) leaves its slots as they are: zero z again before the next call on it. */
 typedef struct ea_linear_scratch {
@@ -245,7 +248,9 @@ typedef struct ea_linear_scratch {
 
 /* linear.zig:61-79 plan */
 void ea_linear_plan(uint32_t k, uint32_t n, uint32_t* sk, uint32_t* wk);
-/* linear.zig:164-188 call / callRotated: outs[j] = x @ W_j for 1..3 groupable layers, m <= 128 rows (rot_in + one linear launch). */
+/* linear.zig:164-188 call / callRotated: outs[j] = x @ W_j for 1..3 groupable layers, m <= 128 rows: one launch for few
+ * rows, else up to three (rotation, products, the splits' sums). xh holds the rotated rows afterwards. With one K split an
+ * output may take x's place. */
 int ea_linear_call(ea_stream_t stream, const ea_linear_scratch* s, const ea_linear* const* ls, uint32_t nls,
                    const void* x, int x_dtype, uint32_t m, const uint64_t* outs, const int* out_dtypes);
 int ea_linear_call_rotated(ea_stream_t stream, const ea_linear_scratch* s, const ea_linear* const* ls, uint32_t nls,
