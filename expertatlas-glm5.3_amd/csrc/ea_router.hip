@@ -61,12 +61,11 @@ __device__ __forceinline__ void act4(uint2 u, bool bf, float (&v)[4]) {
 // Block (expert, row group of ROWS), wave s: slice s of the expert and the group's rows. What bounds it at few rows is round
 // trips (3.1 MB of weights at 256 x 6144 are 0.5 us of HBM, a block's rows come from L2), with more the rows' unpacking and
 // products. So the loads of RT_BATCH chunks of the weight and of every row are issued before the first product (a row past
-// m re-reads the last one, a chunk past the slice the slice's last, and is not added), the type is fixed at compile time,
-// and the rows' lane sums share their steps (wave_sums). The form before read each row under a condition of its own, which
+// m re-reads the last one, a chunk past the slice the slice's last, and is not added; RT_BATCH follows from d, so that hardly
+// a chunk lies past the slice: router_batch), the type is fixed at compile time, and the rows' lane sums share their steps (wave_sums). The form before read each row under a condition of its own, which
 // waited for its load, and took four experts a block above 16 rows. 256 x 6144, distinct weights: 1 row 3.5 -> 2.9 us, 2 rows
 // 6.6 -> 3.2, 5 rows 8.6 -> 4.5, 16 rows 16.2 -> 6.7, 37 rows 19.6 -> 12.7, 128 rows 38 -> 26.5, 512 rows 190 -> 94.
-constexpr int RT_BATCH = 3;  // the chunks of a lane's slice at d = 6144
-template <int ROWS, bool BF>
+template <int ROWS, bool BF, int RT_BATCH>
 __global__ void __launch_bounds__(64 * RT_SLICES) router_kernel(const uint16_t* __restrict__ x, int x_stride,
                                                                     const uint16_t* __restrict__ w,
                                                                     float* __restrict__ part, float* __restrict__ out,
@@ -123,6 +122,14 @@ __global__ void __launch_bounds__(64 * RT_SLICES) router_kernel(const uint16_t* 
     }
 }
 
+// Chunks of a lane's slice a batch: as few batches as four hold, and no more chunks in each than it takes. (Always three, as
+// d = 6144 takes, multiplied chunks past the slice elsewhere: d = 7168, 384 experts, 33 rows 31.1 us, now 22.5; d = 512, 8
+// experts, 4096 rows 26.3, now 10.7; d = 7168, 256 experts, 128 rows 48.1, now 33.7.)
+static int router_batch(int chunks) {
+    const int n = (chunks + 3) / 4;
+    return n > 0 ? (chunks + n - 1) / n : 1;
+}
+
 int launch_router(hipStream_t s, const void* x, int x_dtype, uint32_t x_stride, const void* w, float* part, float* out,
                   uint32_t m, uint32_t d, uint32_t ne) {
     EA_REQUIRE_CTX(c);
@@ -136,8 +143,11 @@ int launch_router(hipStream_t s, const void* x, int x_dtype, uint32_t x_stride, 
     const auto* xs = static_cast<const uint16_t*>(x);
     const auto* ws = static_cast<const uint16_t*>(w);
     // rows a block (the least power of two that holds m, at most 16): a block's rows share one read of its weights
+    const int chunks = ((int)(d / RT_SLICES / 4) + 63) / 64;
+    const int batch = router_batch(chunks);
+#define EA_RB(ROWS_, BATCH_) (x_dtype == BF16 ? router_kernel<ROWS_, true, BATCH_> : router_kernel<ROWS_, false, BATCH_>)
 #define EA_RF(ROWS_)                                                                                                   \
-    (x_dtype == BF16 ? router_kernel<ROWS_, true> : router_kernel<ROWS_, false>)                                       \
+    (batch == 1 ? EA_RB(ROWS_, 1) : batch == 2 ? EA_RB(ROWS_, 2) : batch == 3 ? EA_RB(ROWS_, 3) : EA_RB(ROWS_, 4))     \
         <<<dim3(ne, (m + (ROWS_) - 1) / (ROWS_)), 64 * RT_SLICES, 0, s>>>(xs, (int)x_stride, ws, part, out, (int)m,    \
                                                                           (int)d, (int)ne)
     if (m == 1) EA_RF(1);
@@ -146,6 +156,7 @@ int launch_router(hipStream_t s, const void* x, int x_dtype, uint32_t x_stride, 
     else if (m <= 8) EA_RF(8);
     else EA_RF(16);
 #undef EA_RF
+#undef EA_RB
     return launched();
 }
 

@@ -120,7 +120,8 @@ def test_gpu_router_bit_exact(ea, m, d, ne, x_dtype):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("d", [512, 1536, 6144, 7168])  # a lane's chunks: none for most, none or one, three, three or four
+# a lane's chunks: none for most, none or one, two, three, three or four, five (two batches of three), six
+@pytest.mark.parametrize("d", [512, 1536, 4096, 6144, 7168, 10240, 12288])
 @pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8, 9, 15, 16, 17])  # the row groups' sizes and remainders
 def test_gpu_router_row_groups(ea, m, d):
     test_gpu_router_bit_exact(ea, m, d, 5, m & 1)
