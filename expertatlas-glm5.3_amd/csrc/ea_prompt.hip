@@ -391,9 +391,10 @@ int ea_prompt_experts_run(ea_stream_t stream, const void* x, int x_dtype, uint32
         const uint16_t *suh_g = dptr<const uint16_t>(ex->suh_g), *suh_u = dptr<const uint16_t>(ex->suh_u);
         // Long passes rotate inside the larger items' products (rotate_fits says when they can): 2048 rows 666 -> 601 us,
         // bound by memory; 1024 rows 423 with the launch and 419 without it, 512 rows 306 and 335 (few blocks, each with the
-        // rotation on its chain). Widths above 10 keep the rotation launch: the one build of their kernel with the rotation
+        // rotation on its chain; a pass of as many rows with fewer slots likewise: 16 experts, 2 slots, 2048 rows 61 us with
+        // the launch and 67 without). Widths above 10 keep the rotation launch: the one build of their kernel with the rotation
         // inside hung in a test and its cause was not found, so no such kernel is built (list_pass).
-        const bool fuse = !wide && n > (uint32_t)LONG_ROWS && rotate_fits(xs, x_dtype, xstride, suh_g, suh_u, n, I);
+        const bool fuse = !wide && n > (uint32_t)LONG_ROWS && pairs > 8u * LONG_ROWS && rotate_fits(xs, x_dtype, xstride, suh_g, suh_u, n, I);
         if (!fuse) {
             r = launch_rot_in(s, xs, x_dtype, xstride, pk, suh_g, suh_u, dptr<uint16_t>(sc->xg), dptr<uint16_t>(sc->xu), n,
                               D, S, E);

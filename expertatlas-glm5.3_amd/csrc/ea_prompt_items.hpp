@@ -61,11 +61,18 @@ constexpr int WINDOW_ROWS_MAX = 128;  // the widest decode window (forward.zig:2
 constexpr int DNG_BIG = 2;  // the same for the larger items: more blocks for fewer items (4: 1 % slower at 512 rows)
 constexpr int DNG_BIG_LONG = 4;   // passes of more than LONG_ROWS rows: 1.5 % faster at 2048 rows
 constexpr int LONG_ROWS = 1024;
-// Rows a pass up to which the larger items' gate|up stages its activations in two buffers (two blocks a CU), above which in
-// one (four). 300 rows 254 us with two and 282 with one, 512 rows 306 and 315, 640 rows 351 and 347, 1024 rows 447 and 423:
-// few blocks wait on each chunk's round trip, many on each other for a place. (Rows of 8 slots over 256 experts, as for the
-// other row counts here.)
+// Up to these rows a pass, and this much work (pairs x intermediate width, which follows the blocks there are), the larger
+// items' gate|up stages its activations in two buffers (two blocks a CU), above either in one (three or four). 300 rows of 8
+// slots over 256 experts of width 256: 254 us with two and 282 with one, 512 rows 306 and 315, 640 rows 351 and 347, 1024 rows
+// 447 and 423: few blocks wait on each chunk's round trip, many on each other for a place. Width 512: 129 rows 394 and 416,
+// 200 rows 432 and 430, 300 rows 471 and 456, 512 rows 528 and 514. (Picks that spread evenly make more of the items large:
+// 512 rows of width 256 then take 333 and 310 us.)
 constexpr int MID_ROWS = 600;
+constexpr int64_t MID_WORK = 512 * 8 * 256;
+// Above this work the one-buffer kernel gives up its reads ahead for a fourth wave a SIMD: 640 rows of width 256 354 us without
+// and 366 with it, 1024 rows 435 and 440; width 512, 800 rows 650 and 619, 4096 rows 1,836 and 1,772.
+constexpr int64_t DENSE_WORK = 1024 * 8 * 256;
+static bool two_buffers(int rows, int pairs, int width) { return rows <= MID_ROWS && (int64_t)pairs * width <= MID_WORK; }
 constexpr int GU_SPLIT = 2;                       // K splits of a larger item's gate|up (4 and 8 measured slower)
 // The number of K splits of an item's gate|up over K (at most one a chunk). A layer that holds a width above 10 keeps one sum
 // over all of K in ascending order, the order of the sums it has always had; two splits would round its outputs differently
@@ -189,7 +196,7 @@ struct GuSrc {
 // staging regions are larger, always one: 777 rows 428 us, with two 437). The trellis is loaded two chunks ahead into the wave's own region. Loads
 // complete in issue order and every load is issued (a chunk past the last re-reads the last), so the waits stay exact.
 // Thread tid's piece i of a chunk is row (i NT + tid) / 16; aoff: its byte offset in the source.
-template <int CB, int K2, int MT, int NT, bool ROT, bool TWO>
+template <int CB, int K2, int MT, int NT, bool ROT, bool TWO, bool DENSE>
 __device__ __forceinline__ void gu_loop(const GuSrc& src, const uint32_t (&aoff)[(MT * 256 + NT - 1) / NT],
                                         const TileSpan& sp, uint16_t* xa, uint32_t* st, int lane, int rows, int mts,
                                         int c0, int nch, f4v (&acc)[MT][2]) {
@@ -237,7 +244,8 @@ __device__ __forceinline__ void gu_loop(const GuSrc& src, const uint32_t (&aoff)
             issue_a(c + 1);
             issue_t(c + 2, tv);
             __syncthreads();
-            item_chunk_ahead<CB, K2, MT>(st, tl, xa, mts, lane, acc);
+            if constexpr (DENSE) item_chunk<CB, K2, MT>(st, tl, xa, mts, lane, acc, PXS);
+            else item_chunk_ahead<CB, K2, MT>(st, tl, xa, mts, lane, acc);
         }
     };
     if constexpr (TWO) {
@@ -285,8 +293,9 @@ static unsigned xcd_blocks(int items, int C, int Z) { return (unsigned)((items *
 // ROT (WB 8, so that one block covers a rank's 256 columns): X0 is x [rows, K] (16-bit, x_stride apart) and suh0 / suh1
 // the stacked scales; the block rotates its rows as rot_in_kernel does, same bits. A pass over the larger items is bound
 // by memory (2048 rows: 3.8 TB/s of the 5.2 a copy reaches), and the rotated pairs were a quarter of its bytes.
-template <int CB, int MK, bool ROT, bool TWO, int WB>
-__global__ void __launch_bounds__(WB * 64) __attribute__((amdgpu_waves_per_eu(ROT ? 4 : 2)))
+// DENSE (one buffer): no reads ahead, so that four waves fit a SIMD instead of three.
+template <int CB, int MK, bool ROT, bool TWO, int WB, bool DENSE>
+__global__ void __launch_bounds__(WB * 64) __attribute__((amdgpu_waves_per_eu(ROT || DENSE ? 4 : 2)))
 item_gu_kernel(const void* __restrict__ X0, const void* __restrict__ X1, const int64_t* __restrict__ TP0,
                const int64_t* __restrict__ TP1, const int* __restrict__ K2_0, const int* __restrict__ K2_1,
                const int* __restrict__ sorted, const int* __restrict__ items, const int* __restrict__ item_count,
@@ -338,7 +347,7 @@ item_gu_kernel(const void* __restrict__ X0, const void* __restrict__ X1, const i
     const int nch = K / (PK * 16);
     const int c0 = split * nch / nsplit, nc = (split + 1) * nch / nsplit - c0;  // nsplit <= nch: nc >= 1
     const bool ok = EA_K2_SWITCH(
-        k2, 2, MK, (gu_loop<CB, K2V, MT, NT, ROT, TWO>(src, aoff, sp, xa, st[wave], lane, rows, mts, c0, nc, acc)));
+        k2, 2, MK, (gu_loop<CB, K2V, MT, NT, ROT, TWO, DENSE>(src, aoff, sp, xa, st[wave], lane, rows, mts, c0, nc, acc)));
     if (!ok) {
         if (lane == 0) record_error(status, DEV_UNSUPPORTED_WIDTH);
 #pragma unroll
@@ -715,16 +724,18 @@ static bool rotate_fits(const void* x, int x_dtype, uint32_t x_stride, const uin
 template <int CB, int MK>
 static int list_pass(hipStream_t q, const ListPass& a, int big) {
     const int ns = gu_splits(a.D, MK > 10);
-#define EA_GU(ROT_, TWO_, WB_, X0_, X1_)                                                                                \
-    item_gu_kernel<CB, MK, ROT_, TWO_, WB_><<<xcd_blocks(a.mi, a.I / (32 * (WB_)), 2 * ns), (WB_) * 64, 0, q>>>(             \
+    const bool dense = (int64_t)a.P * a.I > DENSE_WORK;
+#define EA_GU(ROT_, TWO_, WB_, DENSE_, X0_, X1_)                                                                                \
+    item_gu_kernel<CB, MK, ROT_, TWO_, WB_, DENSE_><<<xcd_blocks(a.mi, a.I / (32 * (WB_)), 2 * ns), (WB_) * 64, 0, q>>>(             \
         X0_, X1_, a.tp[0], a.tp[1], a.k2[0], a.k2[1], a.sorted, a.items, a.count, a.z, a.zp, a.D, a.I, a.P, ns, 2, a.mi, \
         a.status, a.suh_g, a.suh_u, a.x_dtype == BF16, a.x_stride, a.slots)
     if (big && a.fuse) {
-        if constexpr (MK <= 10) EA_GU(true, true, 8, a.x, a.x);  // fuse is for these widths only (ea_prompt_experts_run)
-    } else if (big && (MK > 10 || a.rows > MID_ROWS)) {
-        EA_GU(false, false, 4, a.xg, a.xu);
+        if constexpr (MK <= 10) EA_GU(true, true, 8, false, a.x, a.x);  // fuse is for these widths only (ea_prompt_experts_run)
+    } else if (big && (MK > 10 || !two_buffers(a.rows, a.P, a.I))) {
+        if (MK <= 10 && dense) EA_GU(false, false, 4, MK <= 10, a.xg, a.xu);
+        else EA_GU(false, false, 4, false, a.xg, a.xu);
     } else if (big) {
-        if constexpr (MK <= 10) EA_GU(false, true, 4, a.xg, a.xu);
+        if constexpr (MK <= 10) EA_GU(false, true, 4, false, a.xg, a.xu);
     } else {
         if (a.fuse) {  // the small items' pairs, on their own stream
             item_rot_kernel<<<dim3(a.mi, 2, (a.D + 2047) / 2048), 256, 0, q>>>(
@@ -764,9 +775,13 @@ static int list_pass(hipStream_t q, const ListPass& a, int big) {
             EA_DN(SMALL_ROWS / 16, 2, PW, dim3(a.mi, nb / 2, 1));
 #undef EA_DN
     } else if (big) {
-        item_gu_kernel<CB, MK, false, false, 4><<<xcd_blocks(a.mi, a.D / 128, 1), 256, 0, q>>>(
-            a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, nullptr, a.I, a.D,
-            a.P, 1, 1, a.mi, a.status, nullptr, nullptr, 0, 0, 1);
+        auto down = [&](auto kernel) {
+            kernel<<<xcd_blocks(a.mi, a.D / 128, 1), 256, 0, q>>>(
+                a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, nullptr, a.I, a.D,
+                a.P, 1, 1, a.mi, a.status, nullptr, nullptr, 0, 0, 1);
+        };
+        if (MK <= 10 && dense) down(item_gu_kernel<CB, MK, false, false, 4, MK <= 10>);
+        else down(item_gu_kernel<CB, MK, false, false, 4, false>);
     } else {
         item_ring_kernel<CB, MK, 4><<<dim3(a.mi, a.D / 128, 1), 4 * 64, 0, q>>>(
             a.xd, a.xd, a.tp[2], a.tp[2], a.k2[2], a.k2[2], a.sorted, a.items, a.count, a.plane.lo, nullptr, a.I, a.D, a.P,

@@ -467,6 +467,31 @@ def test_prompt_experts_long_pass_rotations(ea, x_dtype, pad, planes):
     assert device.device_status() == 0
 
 
+@pytest.mark.parametrize("R,D,I,slots,k2", [(270, 256, 512, 8, 8), (520, 256, 512, 8, 6), (300, 512, 1024, 8, 10),
+                                            (1100, 512, 256, 2, 8), (1030, 512, 384, 8, 5)])
+def test_prompt_experts_gate_up_forms(ea, R, D, I, slots, k2):
+    """The larger items' gate|up in two buffers, in one, and in one on four waves a SIMD (chosen by rows and by pairs times the
+    intermediate's width), the down product of intermediates above 256, and more than 1,024 rows of few slots (rotated by
+    a launch): the oracle's bar, and a row's bits are those of the same row in a short pass."""
+    device, _, moe, pe, synth = ea
+    E, short = 24, 60
+    pick, wts = synth.picks_zipf(660 + R, R, 1.1, E, slots), synth.routing_weights(661, R, slots)
+    host = synth.HostLayer(662, experts=E, dims=D, width=I, k2=k2, cb=1)
+    x = synth.activations(663, R, D, "bf16")
+    ex = moe.Routed(host)
+    dx, dp, dw = device.upload(x), device.upload(pick), device.upload(wts)
+    got = []
+    for rows in (R, short):
+        out = device.zeros((rows, D), torch.float32)
+        pe.run(device.stream(), dx.data_ptr(), D, dp.data_ptr(), dw.data_ptr(), ex, pe.Scratch(ex, rows, slots), out.data_ptr(),
+               rows, do_round=False)
+        got.append(device.download(out))
+    want = orc.prompt_experts(x, pick, wts, oracle_routed(host), R, slots, bf16=True)
+    assert_close_rms(got[0], want, 2e-3, f"R={R} I={I} slots={slots}")
+    np.testing.assert_array_equal(got[0][:short], got[1])
+    assert device.device_status() == 0
+
+
 def test_prompt_experts_second_chunk(ea):
     """More than 4,096 rows: the second chunk of rows takes the same scratch after the first. With and without the pair plane
     (whose down rows then lie where the second chunk's rotated inputs go) the same bits, and those of the second chunk's
