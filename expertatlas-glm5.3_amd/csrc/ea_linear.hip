@@ -48,6 +48,7 @@ constexpr int LS_MAXNKT = 16;
 constexpr int LS_FLAGS = 32;  // flag bytes a 128-column block has in the counters (int32 [8 N / 128], zero between calls)
 constexpr int LS_MAXTS = 8;   // tagged splits the finisher polls at once (two slots a lane each)
 constexpr int LS_PASS = 8;    // rows a pass of the tagged form (passes side by side up to 128 rows)
+constexpr int LS_FLAG_ROWS = 12;  // the most rows a call of the flag form has
 constexpr uint32_t LS_TAG = 0x7FB5EA1Du;
 constexpr int LS_POLLS = 1 << 20;  // polls before the finisher gives up (tens of milliseconds)
 
@@ -133,7 +134,7 @@ __global__ void __launch_bounds__(1024) lin_small_kernel(ea_jobs jobs, ea_rot_jo
     constexpr int TW = 4 * K2;
     EA_STAMP(0, threadIdx.x == 0);  // the block's start
     // the tagged form takes the call's rows in passes of LS_PASS side by side (blockIdx.y): rows m0 .. m0 + M - 1 of
-    // M_all; the flag form all of them (fewer than LS_PASS) in one
+    // M_all; the flag form all of them (at most LS_FLAG_ROWS) in one
     const int m0 = TAG ? (int)blockIdx.y * LS_PASS : 0;
     const int M = TAG ? min(LS_PASS, M_all - m0) : M_all;
     int ji = 0;
@@ -489,10 +490,16 @@ static bool launch_small(const ea_jobs& jobs, const ea_rot_jobs* rj, hipStream_t
     // better one. At 6144 x 2048: 4 rows 8.8 against 10.3 us, 8 rows 11.2 against 10.3, 16 rows 19.6 against 10.4. With
     // more blocks a pass than CUs it is earlier (2048 x 6144: 4 rows 11.2 against 10.8). With few blocks the passes run at
     // once and it is later, the later if no split is handed over (1024 x 640: 8.3 against 8.5 us up to 48 rows).
+    // Rows rotated already cost this kernel less (a pass that rotates repeats it in every block), so it stops later: while
+    // all passes' blocks run at once, and for one pass up to 3 / 2 of that (6144 x 2048, 8 rows 7.5 against 9.5 us, 12 rows 11.7
+    // against 9.5; 6144 x 256 twice, 24 rows 7.6 against 10.0, 33 rows 11.8 against 10.1; 2048 x 6144, 8 rows 8.7 against 10.1).
     bool one = tag;
     for (int i = 0; i < jobs.n; ++i) one = one && jobs.j[i].SK == 2;
     const int passes = (M + LS_PASS - 1) / LS_PASS;
-    const bool few = tag && (one ? tb * passes <= cus : tb * passes < cus / 2);
+    const int flag_rows = rj || nb > cus ? LS_PASS - 1 : LS_FLAG_ROWS;  // the most rows the flag form takes
+    const bool few = !tag ? M <= flag_rows
+                     : rj ? (one ? tb * passes <= cus : tb * passes < cus / 2)
+                          : tb * passes <= cus || (M <= LS_PASS && tb <= cus * 3 / 2);
     if (M >= (tag && tb > cus ? 4 : LS_PASS) && !few) return false;
     // the tagged form on sixteen waves a block (four a SIMD) when its waves' k tiles halve evenly once more: the
     // same decode over twice the waves (config 1: 8.64 -> 8.55 us)
@@ -502,8 +509,8 @@ static bool launch_small(const ea_jobs& jobs, const ea_rot_jobs* rj, hipStream_t
         tn /= 2;
     }
     // the tagged form on sixteen waves; from a whole pass of rows on, when its block's LDS is too large for them, on eight;
-    // the flag form below a pass (1792 x 256 at 12 rows: 15.7 us with it, 10.9 with the kernel for more rows); otherwise not
-    // this kernel
+    // the flag form for few rows (rotating below a pass: 1792 x 256 at 12 rows 15.7 us with it, 10.9 with the kernel for more
+    // rows; rotated already, 1792 x 768 at 8 / 12 / 16 rows 8.4 / 10.0 / 11.0 and 10.9); otherwise not this kernel
 #define EA_SV(K2_, CB_)                                                                                            \
     if (k2 == K2_ && cb == CB_) {                                                                                  \
         if (tag && (rj ? launch_small_k2<CB_, K2_, true, true>(tj, r, tb, s, M, K, tw, tn, x, bf, status)          \
@@ -513,7 +520,7 @@ static bool launch_small(const ea_jobs& jobs, const ea_rot_jobs* rj, hipStream_t
             (rj ? launch_small_k2<CB_, K2_, true, true>(tj, r, tb, s, M, K, 2 * wk, nkt, x, bf, status)            \
                 : launch_small_k2<CB_, K2_, false, true>(tj, r, tb, s, M, K, 2 * wk, nkt, x, bf, status)))         \
             return true;                                                                                           \
-        if (M >= LS_PASS) return false;                                                                            \
+        if (M > flag_rows) return false;                                                                           \
         return rj ? launch_small_k2<CB_, K2_, true, false>(sj, r, nb, s, M, K, wk, nkt, x, bf, status)             \
                   : launch_small_k2<CB_, K2_, false, false>(sj, r, nb, s, M, K, wk, nkt, x, bf, status);           \
     }

@@ -132,6 +132,8 @@ def test_linear_three_jobs_one_launch(ea):
     (17, 640, (8192,), 8, 2),       # one split, the finish in the block, a ragged chunk (five Hadamard blocks)
     (31, 256, (6144,), 12, 2), (33, 2048, (1024, 128), 8, 1), (64, 6144, (256, 256), 10, 2), (65, 1536, (640,), 12, 2),
     (97, 6144, (2048,), 6, 1), (127, 2048, (6144,), 8, 1),
+    # rotated rows (the last call below) on the one-row kernel: flags at twelve rows, and tagged passes side by side
+    (12, 1792, (768,), 10, 2), (24, 6144, (256, 256), 8, 1), (120, 6144, (128,), 8, 1),
 ])
 @pytest.mark.parametrize("x_dtype", [1, 2])
 def test_linear_many_rows(ea, M, K, Ns, k2, cb, x_dtype):
